@@ -1849,37 +1849,179 @@ __device__ void diff_meta(const DiffArgs& a, const Where& w) {
     out[oS + 2 * i] = (uint32_t)v;
     out[oS + 2 * i + 1] = (uint32_t)(v >> 32);
   }
-  if (tid == 0) {
-    const uint64_t chunks = *a.total_chunks;
-    const uint64_t data_off = 32 + 4ull * F + 8ull * P + 8ull * S;
-    mtc_header h;
-    h.ref_id = a.ref_id;
-    h.chkpt_id = a.chkpt_id;
-    h.datalen = a.len;
-    h.chunk_size = a.C;
-    h.num_first_ocur = F;
-    h.num_prior_chkpts = P;
-    h.num_shift_dupl = S;
-    const uint32_t* hw = reinterpret_cast<const uint32_t*>(&h);
-    for (int k = 0; k < 8; k++) out[k] = hw[k];
-    a.ctl->data_chunks = chunks;
-    a.ctl->diff_size = data_off + chunks * a.C;
+}
+
+__device__ void diff_header(const DiffArgs& a) {
+  const uint32_t F = a.ctl->F, P = a.ctl->P, S = a.ctl->S;
+  const uint64_t chunks = *a.total_chunks;
+  const uint64_t data_off = 32 + 4ull * F + 8ull * P + 8ull * S;
+  mtc_header h;
+  h.ref_id = a.ref_id;
+  h.chkpt_id = a.chkpt_id;
+  h.datalen = a.len;
+  h.chunk_size = a.C;
+  h.num_first_ocur = F;
+  h.num_prior_chkpts = P;
+  h.num_shift_dupl = S;
+  uint32_t* out = reinterpret_cast<uint32_t*>(a.diff);
+  const uint32_t* hw = reinterpret_cast<const uint32_t*>(&h);
+  for (int k = 0; k < 8; k++) out[k] = hw[k];
+  a.ctl->data_chunks = chunks;
+  a.ctl->diff_size = data_off + chunks * a.C;
+}
+
+// The gather of stored chunks (tree and basic diffs) works on tiles of the data
+// section of at most kAsmTile bytes: K chunks (a power of two, at most 256), or one
+// of `pieces` slices of a chunk larger than that.  One block copies one tile: every
+// thread issues its (up to four) 16-byte loads before its stores, because on
+// gfx950 a wait for a load also waits for the stores issued before it, so a loop of
+// loads and stores pays a store's latency per turn.  HBM bounds it: the baseline of
+// 4 GiB in 128-byte chunks (3.9 GB stored) takes 1410 us, 1590 us as a loop over
+// 256-chunk tiles with one 16-byte copy a turn; tiles of 32 KiB spill at eight
+// waves per SIMD (1670 us), tiles of 8 KiB have too little in flight (1620 us).  A
+// tile is counted in bytes, not chunks, so that a diff of few large chunks still
+// spreads over many blocks (0.1% of 2 GiB in 4096-byte chunks: 260 us with
+// 256-chunk tiles, 9 us so).
+constexpr uint32_t kAsmTile = 16384;
+constexpr uint32_t kAsmLoads = kAsmTile / 16 / kThreads;
+struct AsmShape {
+  uint32_t K, pieces;
+  __host__ __device__ explicit AsmShape(uint32_t C) : K(256), pieces(1) {
+    while (K > 1 && (uint64_t)K * C > kAsmTile) K >>= 1;
+    if (C > kAsmTile) pieces = (C + kAsmTile - 1) / kAsmTile;
+  }
+  __host__ __device__ uint64_t tiles(uint64_t chunks) const { return pieces > 1 ? chunks * pieces : (chunks + K - 1) / K; }
+};
+
+// Copies one tile to dst: chunk s_src[k] (k < cnt), bytes from..from + size - 1 of
+// each (a whole chunk unless the chunk is sliced), zeros beyond the buffer's len.
+// pow2: C is a power of two of at least 16 and the data 16-byte aligned.  short_last:
+// one of the chunks is the buffer's short last chunk.
+__device__ __forceinline__ void gather_tile(const uint8_t* data, uint64_t len, uint32_t C, bool pow2, bool short_last,
+                                            const uint32_t* s_src, uint32_t cnt, uint32_t from, uint32_t size,
+                                            uint8_t* dst) {
+  const uint32_t bytes = cnt * size;
+  if (pow2 && !short_last) {
+    const uint32_t ulog = __ffs((int)C) - 5, units = bytes / 16;
+    uint4 v[kAsmLoads];
+#pragma unroll
+    for (uint32_t i = 0; i < kAsmLoads; i++) {
+      const uint32_t u = i * kThreads + threadIdx.x;
+      if (u >= units) continue;
+      const uint32_t k = u >> ulog, w = u & ((1u << ulog) - 1);  // a slice (cnt = 1): k = 0
+      v[i] = ld_stream16(data + (uint64_t)s_src[k] * C + from + 16 * w);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kAsmLoads; i++) {
+      const uint32_t u = i * kThreads + threadIdx.x;
+      if (u < units) *reinterpret_cast<u32x4_nt_a4*>(dst + 16 * u) = u32x4_nt_a4{v[i].x, v[i].y, v[i].z, v[i].w};
+    }
+    return;
+  }
+  // Any chunk size and alignment: 16 bytes of the tile at a time.  Where they come
+  // from one chunk, or from two that are neighbours in the buffer too (as inside a
+  // region), they are cut out of the five aligned words that hold them (bytes
+  // straddle words at any shift); elsewhere they go byte by byte.  (A baseline and
+  // four checkpoints of 200 MB in 1000-byte chunks at 5%: 5680 us of gathering byte
+  // by byte, 195 us so.)
+  const bool dst4 = ((uintptr_t)dst & 3) == 0;
+#pragma unroll 1
+  for (uint32_t o = 16 * threadIdx.x; o < bytes; o += 16 * kThreads) {
+    const uint32_t k = o / size, w = o - k * size;
+    const uint64_t so = (uint64_t)s_src[k] * C + from + w;
+    const uint8_t* p = data + so;
+    const uint32_t sh = (uint32_t)(uintptr_t)p & 3;
+    if (dst4 && o + 16 <= bytes && so >= sh && so + 20 <= len &&
+        (w + 16 <= size || (w + 16 <= 2 * size && s_src[k + 1] == s_src[k] + 1))) {
+      const uint32_t* q = reinterpret_cast<const uint32_t*>(p - sh);
+      const u32x4_nt_a4 v = *reinterpret_cast<const u32x4_nt_a4*>(q);
+      const uint32_t x = q[4];
+      *reinterpret_cast<u32x4_nt_a4*>(dst + o) = u32x4_nt_a4{
+          __builtin_amdgcn_alignbyte(v.y, v.x, sh), __builtin_amdgcn_alignbyte(v.z, v.y, sh),
+          __builtin_amdgcn_alignbyte(v.w, v.z, sh), __builtin_amdgcn_alignbyte(x, v.w, sh)};
+      continue;
+    }
+#pragma unroll 1
+    for (uint32_t b = o; b < min(o + 16, bytes); b++) {
+      const uint32_t kb = b / size;
+      const uint64_t sb = (uint64_t)s_src[kb] * C + from + (b - kb * size);
+      dst[b] = sb < len ? data[sb] : 0;
+    }
   }
 }
 
-constexpr uint32_t kAsmWindow = 512;  // region offsets staged per tile of 256 diff chunks
+constexpr uint32_t kAsmWindow = 512;  // region offsets staged per tile
 
-// The diff in one launch: metadata (every block, grid-stride), then block 0 folds
-// the counters and copies the control block out (its diff size is final once
-// block 0's own metadata thread has written it), then the chunks of every
-// first-occurrence region are gathered, regions in root order and leaves in
-// ascending chunk order; the short last chunk is zero padded (:636-650).
+// The diff in one launch.  The last block writes the header, folds the counters and
+// copies the control block out; the others gather the chunks of every first-
+// occurrence region, regions in root order and leaves in ascending chunk order, the
+// short last chunk zero padded (:636-650).  All of them write the metadata.
 __device__ __forceinline__ void ph_assemble(const Launch<DiffArgs>& L, const Where& wh, uint8_t* lds) {
   uint32_t* s_src = reinterpret_cast<uint32_t*>(lds);
   unsigned long long* s_fold = reinterpret_cast<unsigned long long*>(lds + sizeof(uint32_t) * kThreads);
   uint32_t* s_off = reinterpret_cast<uint32_t*>(lds + sizeof(uint32_t) * kThreads + sizeof(unsigned long long) * CTR_KINDS);
+  uint32_t* s_short = s_off + kAsmWindow;
   static_assert(kThreads == kStripes, "one block folds the striped counters");
   const DiffArgs a = L.args[wh.m].global();
+  const uint32_t F = a.ctl->F;
+  if (wh.blk + 1 == wh.nblk) {
+    if (threadIdx.x == 0) diff_header(a);
+    __syncthreads();  // the header thread's control fields
+    finish_member(a.ctr, a.changed, a.ctl, a.out, s_fold);
+  } else if (F) {
+    const uint64_t total = *a.total_chunks;
+    uint8_t* dst0 = a.diff + 32 + 4ull * F + 8ull * a.ctl->P + 8ull * a.ctl->S;
+    const uint32_t C = a.C;
+    const AsmShape shape(C);
+    const uint64_t ntiles = shape.tiles(total);
+    const bool ragged = (uint64_t)a.n * C > a.len;
+    for (uint64_t tile = wh.blk; tile < ntiles; tile += wh.nblk - 1) {
+      const uint64_t j0 = shape.pieces > 1 ? tile / shape.pieces : tile * shape.K;
+      const uint32_t from = shape.pieces > 1 ? (uint32_t)(tile % shape.pieces) * kAsmTile : 0u;
+      const uint32_t cnt = (uint32_t)min<uint64_t>(shape.K, total - j0);
+      // The regions of the tile's 256-chunk group start at tile_lo and end at the
+      // next group's: their offsets are staged in LDS (a search over every region's
+      // offset in global memory waited for about 18 dependent loads per chunk).
+      const uint64_t grp = j0 / 256;
+      const uint32_t lo0 = a.tile_lo[grp];
+      const uint32_t end = (grp + 1) * 256 < total ? a.tile_lo[grp + 1] + 1 : F;
+      const uint32_t win = min(end - lo0, kAsmWindow);
+      for (uint32_t t = threadIdx.x; t < win; t += kThreads) s_off[t] = a.region_off[lo0 + t];
+      if (threadIdx.x == 0) *s_short = 0;
+      __syncthreads();
+      if (threadIdx.x < cnt) {
+        const uint64_t j = j0 + threadIdx.x;
+        uint32_t lo, hi;  // last region whose offset <= j
+        if (win == kAsmWindow && j >= s_off[kAsmWindow - 1]) {  // many empty regions: the rest in global memory
+          lo = lo0 + kAsmWindow - 1;
+          hi = F;
+          while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (a.region_off[mid] <= j) lo = mid;
+            else hi = mid;
+          }
+        } else {
+          uint32_t l = 0, h = win;
+          while (h - l > 1) {
+            const uint32_t mid = (l + h) >> 1;
+            if (s_off[mid] <= j) l = mid;
+            else h = mid;
+          }
+          lo = lo0 + l;
+        }
+        uint32_t st[2], ct[2];
+        const int r = region_runs(a.g, a.first_roots[lo], a.compat, st, ct);
+        const uint32_t off = lo - lo0 < win ? s_off[lo - lo0] : a.region_off[lo];
+        const uint32_t src = run_at(r, st, ct, (uint32_t)(j - off));
+        s_src[threadIdx.x] = src;
+        if (ragged && (uint64_t)src + 1 >= a.n) *s_short = 1;
+      }
+      __syncthreads();
+      const uint32_t size = shape.pieces > 1 ? min(kAsmTile, C - from) : C;
+      gather_tile(a.data, a.len, C, a.aligned != 0, *s_short != 0, s_src, cnt, from, size, dst0 + j0 * C + from);
+      __syncthreads();
+    }
+  }
   diff_meta(a, wh);
   // Nothing reads the leaf labels after sweep B: the listed chunks go back to
   // L_FIXED, so the next step's leaf kernel labels only the chunks it lists.
@@ -1888,95 +2030,28 @@ __device__ __forceinline__ void ph_assemble(const Launch<DiffArgs>& L, const Whe
     for (uint64_t i = (uint64_t)wh.blk * kThreads + threadIdx.x; i < listed; i += (uint64_t)wh.nblk * kThreads)
       a.reset_labels[a.dense[i]] = L_FIXED;
   }
-  if (wh.blk == 0) {
-    __syncthreads();  // the header thread's control fields
-    finish_member(a.ctr, a.changed, a.ctl, a.out, s_fold);
-  }
-  const uint32_t F = a.ctl->F;
-  if (F == 0) return;
-  const uint64_t total = *a.total_chunks;
-  const uint64_t data_off = 32 + 4ull * F + 8ull * a.ctl->P + 8ull * a.ctl->S;
-  uint8_t* dst0 = a.diff + data_off;
-  const uint32_t C = a.C;
-  const uint32_t U = a.aligned ? C / 16 : C;  // copy units per chunk
-  for (uint64_t tile = wh.blk; tile * kThreads < total; tile += wh.nblk) {
-    const uint64_t j0 = tile * kThreads;
-    const uint64_t j = j0 + threadIdx.x;
-    // The tile's regions start at tile_lo[tile]: their offsets are staged in LDS
-    // (a search over every region's offset in global memory waited for about 18
-    // dependent loads per chunk).
-    const uint32_t lo0 = a.tile_lo[tile];
-    const uint32_t win = min(F - lo0, kAsmWindow);
-    for (uint32_t t = threadIdx.x; t < win; t += kThreads) s_off[t] = a.region_off[lo0 + t];
-    __syncthreads();
-    if (j < total) {
-      uint32_t lo, hi;  // last region whose offset <= j
-      if (win == kAsmWindow && j >= s_off[kAsmWindow - 1]) {  // many empty regions: the rest in global memory
-        lo = lo0 + kAsmWindow - 1;
-        hi = F;
-        while (hi - lo > 1) {
-          const uint32_t mid = (lo + hi) >> 1;
-          if (a.region_off[mid] <= j) lo = mid;
-          else hi = mid;
-        }
-      } else {
-        uint32_t l = 0, h = win;
-        while (h - l > 1) {
-          const uint32_t mid = (l + h) >> 1;
-          if (s_off[mid] <= j) l = mid;
-          else h = mid;
-        }
-        lo = lo0 + l;
-      }
-      uint32_t st[2], ct[2];
-      const int r = region_runs(a.g, a.first_roots[lo], a.compat, st, ct);
-      const uint32_t off = lo - lo0 < win ? s_off[lo - lo0] : a.region_off[lo];
-      s_src[threadIdx.x] = run_at(r, st, ct, (uint32_t)(j - off));
-    }
-    __syncthreads();
-    const uint64_t cnt = (total - j0 < kThreads) ? total - j0 : kThreads;
-    const uint64_t units = cnt * U;
-    for (uint64_t u = threadIdx.x; u < units; u += kThreads) {
-      const uint32_t jj = (uint32_t)(u / U), w = (uint32_t)(u % U);
-      const uint64_t chunk = s_src[jj];
-      const uint64_t so = chunk * C;
-      uint8_t* dst = dst0 + (j0 + jj) * C;
-      if (a.aligned) {
-        const uint64_t b0 = so + 16ull * w;
-        if (b0 + 16 <= a.len) {
-          const uint4 v = *reinterpret_cast<const uint4*>(a.data + b0);
-          *reinterpret_cast<u32x4_nt_a4*>(dst + 16ull * w) = u32x4_nt_a4{v.x, v.y, v.z, v.w};
-        } else {
-          for (int b = 0; b < 16; b++) dst[16ull * w + b] = (b0 + b < a.len) ? a.data[b0 + b] : 0;
-        }
-      } else {
-        dst[w] = (so + w < a.len) ? a.data[so + w] : 0;
-      }
-    }
-    __syncthreads();
-  }
 }
 
-__global__ __launch_bounds__(kThreads) void k_assemble(Launch<DiffArgs> L) {
+__global__ __launch_bounds__(kThreads, 8) void k_assemble(Launch<DiffArgs> L) {
   __shared__ __align__(16) uint8_t lds[sizeof(uint32_t) * kThreads + sizeof(unsigned long long) * CTR_KINDS +
-                                       sizeof(uint32_t) * kAsmWindow];
+                                       sizeof(uint32_t) * (kAsmWindow + 1)];
   ph_assemble(L, where(L), lds);
 }
 
 // Diff of the basic approach (src/basic_approach.cpp:54-142): the header (F = the
 // changed chunks, P = S = 0), their chunk indices, then their bytes, C each, the
 // short last chunk zero padded.  The reference orders the indices as its atomics
-// land; here they are ascending.  Block 0 also folds the counters and copies the
-// control block out, as k_assemble does for tree diffs.
+// land; here they are ascending.  The last block also folds the counters and copies
+// the control block out, as k_assemble does for tree diffs.
 
 __device__ __forceinline__ void ph_basic_diff(const Launch<BasicDiffArgs>& L, const Where& wh, uint8_t* lds) {
-  unsigned long long* s_fold = reinterpret_cast<unsigned long long*>(lds);
+  uint32_t* s_src = reinterpret_cast<uint32_t*>(lds);
+  unsigned long long* s_fold = reinterpret_cast<unsigned long long*>(lds + sizeof(uint32_t) * kThreads);
+  uint32_t* s_short = reinterpret_cast<uint32_t*>(lds + sizeof(uint32_t) * kThreads + sizeof(unsigned long long) * CTR_KINDS);
   const BasicDiffArgs a = L.args[wh.m].global();
   const uint32_t F = *a.total;
   uint32_t* out = reinterpret_cast<uint32_t*>(a.diff);
-  const uint64_t tid = (uint64_t)wh.blk * kThreads + threadIdx.x, stride = (uint64_t)wh.nblk * kThreads;
-  for (uint64_t i = tid; i < F; i += stride) out[8 + i] = a.dense[i];
-  if (wh.blk == 0) {
+  if (wh.blk + 1 == wh.nblk) {
     if (threadIdx.x == 0) {
       mtc_header h;
       h.ref_id = a.ref_id;
@@ -1996,30 +2071,34 @@ __device__ __forceinline__ void ph_basic_diff(const Launch<BasicDiffArgs>& L, co
     }
     __syncthreads();
     finish_member(a.ctr, a.total, a.ctl, a.out, s_fold);
-  }
-  uint8_t* dst0 = a.diff + 32 + 4ull * F;
-  const uint32_t C = a.C;
-  const uint32_t U = a.aligned ? C / 16 : C;  // copy units per chunk
-  for (uint64_t u = tid; u < (uint64_t)F * U; u += stride) {
-    const uint64_t j = u / U, w = u % U;
-    const uint64_t so = (uint64_t)a.dense[j] * C;
-    uint8_t* dst = dst0 + j * C;
-    if (a.aligned) {
-      const uint64_t b0 = so + 16 * w;
-      if (b0 + 16 <= a.len) {
-        const uint4 v = *reinterpret_cast<const uint4*>(a.data + b0);
-        *reinterpret_cast<u32x4_nt_a4*>(dst + 16 * w) = u32x4_nt_a4{v.x, v.y, v.z, v.w};
-      } else {
-        for (int b = 0; b < 16; b++) dst[16 * w + b] = (b0 + b < a.len) ? a.data[b0 + b] : 0;
+  } else {
+    uint8_t* dst0 = a.diff + 32 + 4ull * F;
+    const uint32_t C = a.C;
+    const AsmShape shape(C);
+    const uint64_t ntiles = shape.tiles(F);
+    const bool ragged = (uint64_t)a.n * C > a.len;
+    for (uint64_t tile = wh.blk; tile < ntiles; tile += wh.nblk - 1) {
+      const uint64_t j0 = shape.pieces > 1 ? tile / shape.pieces : tile * shape.K;
+      const uint32_t from = shape.pieces > 1 ? (uint32_t)(tile % shape.pieces) * kAsmTile : 0u;
+      const uint32_t cnt = (uint32_t)min<uint64_t>(shape.K, F - j0);
+      if (threadIdx.x == 0) *s_short = 0;
+      __syncthreads();
+      if (threadIdx.x < cnt) {
+        const uint32_t src = a.dense[j0 + threadIdx.x];
+        s_src[threadIdx.x] = src;
+        if (ragged && (uint64_t)src + 1 >= a.n) *s_short = 1;
       }
-    } else {
-      dst[w] = (so + w < a.len) ? a.data[so + w] : 0;
+      __syncthreads();
+      const uint32_t size = shape.pieces > 1 ? min(kAsmTile, C - from) : C;
+      gather_tile(a.data, a.len, C, a.aligned != 0, *s_short != 0, s_src, cnt, from, size, dst0 + j0 * C + from);
+      __syncthreads();
     }
   }
+  for (uint64_t i = (uint64_t)wh.blk * kThreads + threadIdx.x; i < F; i += (uint64_t)wh.nblk * kThreads) out[8 + i] = a.dense[i];
 }
 
-__global__ __launch_bounds__(kThreads) void k_basic_diff(Launch<BasicDiffArgs> L) {
-  __shared__ __align__(16) uint8_t lds[sizeof(unsigned long long) * CTR_KINDS];
+__global__ __launch_bounds__(kThreads, 8) void k_basic_diff(Launch<BasicDiffArgs> L) {
+  __shared__ __align__(16) uint8_t lds[sizeof(uint32_t) * kThreads + sizeof(unsigned long long) * CTR_KINDS + sizeof(uint32_t)];
   ph_basic_diff(L, where(L), lds);
 }
 
@@ -2658,6 +2737,23 @@ static void add_leaf_scan(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
   add_scan(ops, img, ss);
 }
 
+// Blocks of a diff kernel: one for the header, and one per tile the diff is likely to
+// hold.  A baseline's diff holds nearly the whole buffer; a later one rarely more
+// than an eighth, and blocks without a tile cost too (256 MiB at 2% store 330
+// of 16384 tiles: k_basic_diff 6.2 us with 2048 blocks, 6.7 us as 1024 looping ones
+// before), so it gets a block for every eighth tile, from 1024 to 8192, and they
+// loop if they have to.
+static uint32_t gather_blocks(const Member& M) {
+  const uint64_t tiles = AsmShape(M.h->chunk_size).tiles(M.n);
+  const uint64_t most = M.baseline ? 1u << 20 : std::min<uint64_t>(std::max<uint64_t>(tiles / 8, 1024), 8192);
+  return 1 + (uint32_t)std::min<uint64_t>(tiles, most);
+}
+
+static int gather_pow2(const Member& M) {
+  const uint32_t C = M.h->chunk_size;
+  return C >= 16 && (C & (C - 1)) == 0 && (uintptr_t)M.data % 16 == 0;
+}
+
 // After the leaf kernel, for tree members: table passes, both forests, roots and
 // the diff.
 static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
@@ -2916,7 +3012,7 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
       d.chkpt_id = M.cur;
       d.g = M.g;
       d.ctl = h->ctl_d;
-      d.aligned = ((h->chunk_size % 16) == 0 && (uintptr_t)M.data % 16 == 0) ? 1 : 0;
+      d.aligned = gather_pow2(M);
       d.compat = h->compat;
       d.ctr = h->ctr.p;
       d.changed = h->blk_off.p + M.nblk_leaf;
@@ -2924,7 +3020,7 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
       d.dense = h->dense.p;
       d.reset_labels = h->debug ? nullptr : h->labels.p;  // the debug view copies them after the step
       da.push_back(d);
-      gb.push_back(grid_for(M.n, 8 * kThreads, 8192));
+      gb.push_back(gather_blocks(M));
     }
     ops.add<DiffArgs>(72, img.add(da, gb), [](Launch<DiffArgs> L, uint32_t g, hipStream_t st) { k_assemble<<<g, kThreads, 0, st>>>(L); });
   }
@@ -2960,11 +3056,11 @@ static void build_basic_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) 
     d.ref_id = h->baseline_id;
     d.chkpt_id = M.cur;
     d.ctl = h->ctl_d;
-    d.aligned = ((h->chunk_size % 16) == 0 && (uintptr_t)M.data % 16 == 0) ? 1 : 0;
+    d.aligned = gather_pow2(M);
     d.ctr = h->ctr.p;
     d.out = M.ctl_out;
     da.push_back(d);
-    gb.push_back(grid_for(M.n, 8 * kThreads, 8192));
+    gb.push_back(gather_blocks(M));
   }
   ops.add<BasicDiffArgs>(80, img.add(da, gb), [](Launch<BasicDiffArgs> L, uint32_t g, hipStream_t st) { k_basic_diff<<<g, kThreads, 0, st>>>(L); });
 }

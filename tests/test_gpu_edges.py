@@ -41,3 +41,36 @@ def test_digests_shared_by_many_chunks(patterns, n):
     v2 = v1.copy()
     v2[rng.random(n) < 0.3] = bank[0]
     same_as_oracle([v0, v1.reshape(-1), v2.reshape(-1)], C)
+
+
+@pytest.mark.parametrize("approach", [M.TREE, M.BASIC])
+@pytest.mark.parametrize("C,n,tail", [
+    (1, 3000, 0), (3, 5000, 0), (16, 4097, 5), (17, 3000, 16), (48, 2500, 47), (100, 1300, 3), (1000, 333, 999),
+    (1024, 130, 1), (4096, 70, 4000), (4100, 40, 17), (16384, 9, 0), (16400, 11, 5), (32768, 5, 32767),
+    (65536, 4, 100), (65536, 3, 0), (100_003, 5, 77)])
+def test_gathered_chunks(approach, C, n, tail):
+    """The diff's data section around the sizes at which its tiles change: chunks of
+    one byte to several tiles, powers of two or not, with and without a short last
+    chunk, runs and single chunks, and a buffer that is not 16-byte aligned."""
+    rng = np.random.default_rng(C + n)
+    size = n * C + tail
+    v = [rng.integers(0, 256, size, dtype=np.uint8)]
+    for k in range(3):
+        w = v[-1].copy()
+        for first in rng.integers(0, n, 1 + n // 40):
+            e = min(size, (int(first) + int(rng.integers(1, 6))) * C)
+            w[first * C:e] = rng.integers(0, 256, max(0, e - first * C), dtype=np.uint8)
+        if k == 1:
+            w[-1:] ^= 1
+        v.append(w)
+    for off in (0, 5):
+        d = M.TreeDeduplicator(C, approach)
+        orc = O.OracleDedup(C, M.MURMUR3) if approach == M.TREE else O.OracleBasic(C, M.MURMUR3)
+        for k, host in enumerate(v):
+            print(f"gather C={C} n={n} tail={tail} approach={approach} off={off} k={k}", flush=True)
+            buf = torch.zeros(size + 16, dtype=torch.uint8, device="cuda:0")
+            buf[off:off + size] = torch.from_numpy(host)
+            g = d.checkpoint(buf[off:off + size], make_baseline=(k == 0))
+            e = orc.checkpoint(host, make_baseline=(k == 0))
+            assert g == e, (k, len(g), len(e))
+        d.close()
