@@ -200,6 +200,7 @@ struct RootArgs {
   uint32_t ndepth, nseg;
   uint32_t* first_roots;
   uint64_t* shift_tmp;
+  uint32_t segs;  // segments per wavefront (<= 64)
   __device__ RootArgs global() const {
     RootArgs c = *this;
     MTC_GLOBAL(staging); MTC_GLOBAL(cnt_f); MTC_GLOBAL(cnt_s); MTC_GLOBAL(off_f); MTC_GLOBAL(off_s); MTC_GLOBAL(seg_base); MTC_GLOBAL(first_roots); MTC_GLOBAL(shift_tmp);

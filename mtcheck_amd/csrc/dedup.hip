@@ -1571,10 +1571,18 @@ __device__ __forceinline__ void ph_single_leaf(const Launch<SweepArgs>& L, const
 __global__ void k_single_leaf(Launch<SweepArgs> L) { ph_single_leaf(L, where(L)); }
 
 // ---------------------------------------------------------------------------
-// Root compaction, in segment order (depth, then group).  A wavefront takes 64
+// Root compaction, in segment order (depth, then group).  A wavefront takes a few
 // segments, one per lane, and copies their roots 64 at a time: lane e of a round
 // finds its segment by bisection over the exclusive prefix of the root counts, and
 // its rank among the segment's first-occurrence (or shifted) roots from a ballot.
+//
+// The rounds of a wavefront run one after the other and segments differ widely in
+// their roots, so few wavefronts with many segments leave the chip waiting for the
+// fullest.  Microseconds by segments per wavefront (a baseline / a later checkpoint):
+//                                     64         16        8         4         2
+//   64 MiB, 128 B, 3% (2.3K segments) 171 / 22   47 / 9    28 / 7    18 / 6    12 / 5
+//   1 GiB, 64 B, 20% (67K)            187 / 156  58 / 46   40 / 31   31 / 25   35 / 27
+//   4 GiB, 128 B, 2% (135K)           207 / 22   69 / 13   51 / 15   47 / 20   58 / 31
 // ---------------------------------------------------------------------------
 
 // Lanes lo..hi-1 (0 <= lo, hi <= 64).
@@ -1593,9 +1601,9 @@ __device__ __forceinline__ void ph_scatter_roots(const Launch<RootArgs>& L, cons
   if (threadIdx.x <= 2 * a.ndepth) s_base[threadIdx.x] = a.seg_base[threadIdx.x];
   __syncthreads();
   const uint32_t lane = lane_id();
-  const uint32_t seg = w.blk * kThreads + threadIdx.x;
+  const uint32_t seg = (w.blk * (kThreads / 64) + threadIdx.x / 64) * a.segs + lane;
   uint32_t nf = 0, ns = 0;
-  if (seg < a.nseg) {
+  if (lane < a.segs && seg < a.nseg) {
     nf = a.cnt_f[seg];
     ns = a.cnt_s[seg];
   }
@@ -2333,6 +2341,10 @@ static uint32_t digits0(uint32_t nbins) {
   return 1u << std::min<uint32_t>(8, bits);
 }
 
+// Segments per wavefront of k_scatter_roots: 2 until there are enough wavefronts to
+// fill the chip (8192) with more each, up to 8.
+static uint32_t scatter_segs(uint32_t nseg) { return std::min<uint32_t>(8, std::max<uint32_t>(2, nseg / 16384)); }
+
 static uint32_t sort_blocks(uint32_t n) { return std::max<uint32_t>(1, std::min<uint32_t>(kSortBlocks, (n + 16 * kThreads - 1) / (16 * kThreads))); }
 
 static uint64_t scan_sums(uint64_t count) { return (count + kScanTile - 1) / kScanTile + 1; }
@@ -2928,8 +2940,8 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
     for (auto& M : ms) {
       mtc_dedup* h = M.h;
       ra.push_back(RootArgs{h->staging.p, h->seg_cnt_f.p, h->seg_cnt_s.p, h->seg_off_f.p, h->seg_off_s.p, h->seg_base.p,
-                            M.g.D + 1, M.nseg, h->first_roots.p, h->shift_tmp.p});
-      rb.push_back(grid_for(M.nseg));
+                            M.g.D + 1, M.nseg, h->first_roots.p, h->shift_tmp.p, scatter_segs(M.nseg)});
+      rb.push_back(grid_for(M.nseg, kThreads / 64 * scatter_segs(M.nseg)));
     }
     ops.add<RootArgs>(50, img.add(ra, rb), [](Launch<RootArgs> L, uint32_t g, hipStream_t st) { k_scatter_roots<<<g, kThreads, 0, st>>>(L); });
   }

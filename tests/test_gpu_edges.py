@@ -74,3 +74,26 @@ def test_gathered_chunks(approach, C, n, tail):
             e = orc.checkpoint(host, make_baseline=(k == 0))
             assert g == e, (k, len(g), len(e))
         d.close()
+
+
+@pytest.mark.parametrize("n", [(1 << 20) - 3, 1 << 21, 1 << 22])
+def test_root_segments_per_wavefront(n):
+    """Root segments of one tile each: 37 thousand (two segments per wavefront of the
+    root compaction), 74 thousand (four) and 147 thousand (eight)."""
+    C = 16
+    rng = np.random.default_rng(n)
+    v0 = rng.integers(0, 256, n * C, dtype=np.uint8)
+    v1 = v0.copy().reshape(n, C)
+    at = rng.random(n) < 0.02
+    v1[at] = rng.integers(0, 256, (int(at.sum()), C), dtype=np.uint8)
+    at = np.nonzero(rng.random(n) < 0.01)[0]
+    v1[at] = v1[rng.integers(0, n, at.size)]
+    v1 = v1.reshape(-1)
+    d, orc = M.TreeDeduplicator(C), O.OracleDedup(C)
+    d.set_sweep_tiles(1, 1)
+    for k, host in enumerate((v0, v1)):
+        print(f"segments n={n} k={k}", flush=True)
+        g = d.checkpoint(torch.from_numpy(host).to("cuda:0"), make_baseline=(k == 0))
+        e = orc.checkpoint(host, make_baseline=(k == 0), threads=8)
+        assert g == e, (k, first_mismatch(g, e))
+    d.close()
