@@ -202,7 +202,7 @@ int mtc_set_tuning(mtc_dedup* h, uint32_t leaf_tiles_per_block, float load_facto
 
 /* First-stage tiles of 256 positions each wavefront of sweep A (first occurrences)
  * and sweep B (shifted duplicates and roots) walks, 1..64, or 0 for the library's
- * default (8 and 8); no counterpart in the reference.  Applies from the next
+ * choice by the number of tiles (1 to 8); no counterpart in the reference.  Applies from the next
  * checkpoint.  Results do not depend on it. */
 int mtc_set_sweep_tiles(mtc_dedup* h, uint32_t tiles_a, uint32_t tiles_b);
 

@@ -3,9 +3,7 @@ synthetic sample buffer on the device under each schedule of a search space and
 keeps the fastest, unless the library's default is within MARGIN of it.  For a
 batched caller the sample is checkpointed by several deduplicators in one batched
 step (`members`), so that the schedule is timed with the device as full as the
-caller's batch keeps it: alone, a 256 MiB buffer favoured four stage-0 tiles per
-sweep wavefront, which made the 256-buffer batch 5% slower than the default eight.  A
-schedule is (leaf tiles per block, table load factor, tree levels fused per sweep
+caller's batch keeps it (a lone 256 MiB buffer leaves half of it empty).  A schedule is (leaf tiles per block, table load factor, tree levels fused per sweep
 stage, sweep A tiles per wavefront, sweep B tiles per wavefront).  The choice
 never changes results (diffs are identical for every schedule), only speed and,
 through the load factor, the table's memory."""
@@ -17,10 +15,10 @@ import time
 from .tree import MURMUR3, Batch, TreeDeduplicator
 from .workload import CheckpointSeries
 
-DEFAULT = (1, 0.125, 8, 8, 8)
+DEFAULT = (1, 0.125, 8, 0, 0)  # sweep tiles 0: the library's choice by the number of tiles
 LOAD_FACTORS = (0.125, 0.25)   # a 0.25 table holds half the slots (half the memory)
 FUSE = (6, 7, 8)
-SWEEP_TILES = ((8, 8), (4, 8), (8, 16), (4, 4))
+SWEEP_TILES = ((0, 0), (8, 8), (4, 8), (4, 4))
 LEAF_TILES = (1, 2, 4, 8)
 MARGIN = 0.03  # a schedule replaces the default only when it is this much faster
 # Chunk sizes the leaf kernel stages through LDS.  For these, one tile per block

@@ -38,14 +38,6 @@ constexpr uint32_t kScanTile = 8 * kThreads;   // elements per block-tile of the
 constexpr uint32_t kScanOneItems = 16;          // elements per thread of a one-launch scan
 constexpr uint32_t kScanOneMax = kScanOneItems * kThreads;
 constexpr uint32_t kSortBlocks = 1024;         // most blocks per member of the stable sort
-#ifndef MTC_TPW_A
-#define MTC_TPW_A 8
-#endif
-constexpr uint32_t kTilesPerWaveA = MTC_TPW_A;  // stage-0 tiles per wavefront, sweep A (<= 64)
-#ifndef MTC_TPW_B
-#define MTC_TPW_B 8
-#endif
-constexpr uint32_t kTilesPerWaveB = MTC_TPW_B;  // stage-0 tiles per wavefront, sweep B (<= 64)
 // Wavefronts per block of the sweeps.  Wavefronts of one block draw very
 // different numbers of busy tiles, and a block holds its slot (and sweep A's LDS
 // records) until its slowest wavefront ends: with four wavefronts per block only
@@ -2327,11 +2319,39 @@ static void plan_tree(mtc_dedup* h, uint32_t fuse_req, uint32_t group) {
   h->plan_dirty = true;
 }
 
-// Tiles per wavefront of sweep B's first stage, which is also the segment group:
-// every tile, one per wavefront, when the debug labels are recorded.
-static uint32_t sweep_b_group(const mtc_dedup* h) {
+// First-stage tiles that one wavefront of each sweep walks, by the number of tiles of
+// the whole step.  A wavefront walks its tiles one after the other, so several a
+// wavefront pay only once there are wavefronts enough to fill the chip (sweep A
+// holds 6144, sweep B 5120) several times over; sweep B's group is also the unit of
+// root counting, so one tile each doubles the segments that the scans and the root
+// compaction read.  Microseconds of a series' sweep A / sweep B + root compaction by
+// tiles a wavefront:
+//                                             1           2           4           8
+//   64 MiB, 128 B, 3%, x 10 (2048 tiles)      174/267     -/310       -/379     493/472
+//   256 MiB, 128 B, 2%, x 4 (8192)            297/151     309/164     361/183   415/228
+//   1 GiB, 128 B, 2%, x 4 (32768)             810/275     827/273     894/277   906/294
+//   1 GiB, 64 B, 20%, MD5, x 5 (65536)        2196/848    2242/801    2302/797  2504/858
+//   4 GiB, 128 B, 2%, x 8 (131072)            3275/1445   3261/1287   3303/1137 3392/1104
+// and 256 buffers of 23 GiB in one step (970 thousand tiles) take 8.9 ms with one to
+// two, 8.0 ms with eight.
+static uint64_t first_stage_tiles(uint64_t n, uint32_t fuse) {
+  const Geo g = make_geo((uint32_t)n);
+  return 1ull << (g.D > fuse ? g.D - fuse : 0);
+}
+
+static uint32_t sweep_a_tiles(const mtc_dedup* h, uint64_t step_tiles) {
+  if (h->tune.sweep_tiles_a) return h->tune.sweep_tiles_a;
+  return step_tiles <= 65536 ? 1u : step_tiles <= 262144 ? 2u : 8u;
+}
+
+// Sweep B's, which is also the segment group: every tile, one per wavefront, when
+// the debug labels are recorded.  A handle that steps now alone, now in a batch keeps
+// a plan whose group is near what the step would choose: a new plan is uploaded.
+static uint32_t sweep_b_group(const mtc_dedup* h, uint64_t step_tiles, bool planned) {
   if (h->debug) return 1;
-  return h->tune.sweep_tiles_b ? h->tune.sweep_tiles_b : kTilesPerWaveB;
+  if (h->tune.sweep_tiles_b) return h->tune.sweep_tiles_b;
+  const uint32_t want = (uint32_t)std::min<uint64_t>(8, std::max<uint64_t>(1, step_tiles / 16384));
+  return planned && h->plan_group <= 8 && h->plan_group < 4 * want && want < 4 * h->plan_group ? h->plan_group : want;
 }
 
 // Digit values of the sort's first pass for nbins source checkpoints.
@@ -2341,9 +2361,10 @@ static uint32_t digits0(uint32_t nbins) {
   return 1u << std::min<uint32_t>(8, bits);
 }
 
-// Segments per wavefront of k_scatter_roots: 2 until there are enough wavefronts to
-// fill the chip (8192) with more each, up to 8.
-static uint32_t scatter_segs(uint32_t nseg) { return std::min<uint32_t>(8, std::max<uint32_t>(2, nseg / 16384)); }
+// Segments per wavefront of k_scatter_roots: 2 until the step has enough wavefronts
+// to fill the chip (8192) twice with more each.  (256 buffers of 23 GiB, a million
+// segments: 250 us at 2 to 8, 59 us at 64.)
+static uint32_t scatter_segs(uint64_t nseg) { return (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>(2, nseg / 16384)); }
 
 static uint32_t sort_blocks(uint32_t n) { return std::max<uint32_t>(1, std::min<uint32_t>(kSortBlocks, (n + 16 * kThreads - 1) / (16 * kThreads))); }
 
@@ -2590,6 +2611,7 @@ struct Member {
   bool baseline;
   Ctl* ctl_out = nullptr;  // this member's entry of the step's result array
   int arena = 0;           // diff arena this step writes
+  uint64_t step_tiles = 0; // first-stage sweep tiles of all members of the step
   // derived
   uint32_t n = 0, cur = 0, nblk_leaf = 0, nseg = 0, nbins = 0, passes = 0, Gs = 0, R0 = 0;
   uint64_t tpb = 1, ntile0 = 1;
@@ -2668,9 +2690,9 @@ static void prepare_member(Member& M, hipStream_t st) {
     h->has_state = false;
     h->n = (uint32_t)n64;
     h->data_len = M.len;
-    plan_tree(h, h->tune.fuse, sweep_b_group(h));
-  } else if (h->plan_group != sweep_b_group(h)) {
-    plan_tree(h, h->plan_fuse, sweep_b_group(h));  // same stages, new root segments
+    plan_tree(h, h->tune.fuse, sweep_b_group(h, M.step_tiles, false));
+  } else if (h->plan_group != sweep_b_group(h, M.step_tiles, true)) {
+    plan_tree(h, h->plan_fuse, sweep_b_group(h, M.step_tiles, true));  // same stages, new root segments
   }
   ensure_buffers(h, st);
   // Until this step completes, the labels are not known to be reset.  A baseline
@@ -2753,11 +2775,11 @@ static void add_leaf_scan(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
 // hold.  A baseline's diff holds nearly the whole buffer; a later one rarely more
 // than an eighth, and blocks without a tile cost too (256 MiB at 2% store 330
 // of 16384 tiles: k_basic_diff 6.2 us with 2048 blocks, 6.7 us as 1024 looping ones
-// before), so it gets a block for every eighth tile, from 1024 to 8192, and they
-// loop if they have to.
-static uint32_t gather_blocks(const Member& M) {
+// before), so it gets a block for every sixteenth tile, at least its share of 1024
+// and at most 8192, and they loop if they have to.
+static uint32_t gather_blocks(const Member& M, size_t members) {
   const uint64_t tiles = AsmShape(M.h->chunk_size).tiles(M.n);
-  const uint64_t most = M.baseline ? 1u << 20 : std::min<uint64_t>(std::max<uint64_t>(tiles / 8, 1024), 8192);
+  const uint64_t most = M.baseline ? 1u << 20 : std::min<uint64_t>(std::max<uint64_t>({tiles / 16, 1024 / members, 1}), 8192);
   return 1 + (uint32_t)std::min<uint64_t>(tiles, most);
 }
 
@@ -2849,8 +2871,7 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
       a.out_slot = h->fr_slot.p + out_off;
       // stage 0: several tiles per wavefront, their flags read at once; sweep B's
       // tiles per wavefront are the root segment group the plan was made for
-      const uint32_t ta = h->tune.sweep_tiles_a ? h->tune.sweep_tiles_a : kTilesPerWaveA;
-      a.tiles_per_wave = !a.stage0 ? 1u : (pass == 0 ? ta : h->plan_group);
+      a.tiles_per_wave = !a.stage0 ? 1u : (pass == 0 ? sweep_a_tiles(h, ms[i].step_tiles) : h->plan_group);
       return a;
     };
     auto stage_waves = [](const SweepArgs& a) {
@@ -2937,11 +2958,14 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
     add_scan(ops, img, ss);
     std::vector<RootArgs> ra;
     std::vector<uint32_t> rb;
+    uint64_t all_segs = 0;
+    for (const auto& M : ms) all_segs += M.nseg;
+    const uint32_t segs = scatter_segs(all_segs);
     for (auto& M : ms) {
       mtc_dedup* h = M.h;
       ra.push_back(RootArgs{h->staging.p, h->seg_cnt_f.p, h->seg_cnt_s.p, h->seg_off_f.p, h->seg_off_s.p, h->seg_base.p,
-                            M.g.D + 1, M.nseg, h->first_roots.p, h->shift_tmp.p, scatter_segs(M.nseg)});
-      rb.push_back(grid_for(M.nseg, kThreads / 64 * scatter_segs(M.nseg)));
+                            M.g.D + 1, M.nseg, h->first_roots.p, h->shift_tmp.p, segs});
+      rb.push_back(grid_for(M.nseg, kThreads / 64 * segs));
     }
     ops.add<RootArgs>(50, img.add(ra, rb), [](Launch<RootArgs> L, uint32_t g, hipStream_t st) { k_scatter_roots<<<g, kThreads, 0, st>>>(L); });
   }
@@ -3032,7 +3056,7 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
       d.dense = h->dense.p;
       d.reset_labels = h->debug ? nullptr : h->labels.p;  // the debug view copies them after the step
       da.push_back(d);
-      gb.push_back(gather_blocks(M));
+      gb.push_back(gather_blocks(M, ms.size()));
     }
     ops.add<DiffArgs>(72, img.add(da, gb), [](Launch<DiffArgs> L, uint32_t g, hipStream_t st) { k_assemble<<<g, kThreads, 0, st>>>(L); });
   }
@@ -3072,7 +3096,7 @@ static void build_basic_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) 
     d.ctr = h->ctr.p;
     d.out = M.ctl_out;
     da.push_back(d);
-    gb.push_back(gather_blocks(M));
+    gb.push_back(gather_blocks(M, ms.size()));
   }
   ops.add<BasicDiffArgs>(80, img.add(da, gb), [](Launch<BasicDiffArgs> L, uint32_t g, hipStream_t st) { k_basic_diff<<<g, kThreads, 0, st>>>(L); });
 }
@@ -3230,7 +3254,13 @@ static void run_step_body(StepCtx& ctx, std::vector<Member>& ms, hipStream_t st,
   if (!ctx.ev[0])
     for (auto& e : ctx.ev) MTC_HIP(hipEventCreate(&e));
   MTC_HIP(hipEventRecord(ctx.ev[0], st));
-  for (auto& M : ms) prepare_member(M, st);
+  uint64_t step_tiles = 0;
+  for (const auto& M : ms)
+    step_tiles += first_stage_tiles((M.len + M.h->chunk_size - 1) / M.h->chunk_size, M.baseline ? M.h->tune.fuse : M.h->plan_fuse);
+  for (auto& M : ms) {
+    M.step_tiles = step_tiles;
+    prepare_member(M, st);
+  }
   // Reset tables of baseline members (basic members keep no table).
   for (auto& M : ms) {
     if (!M.baseline || M.h->approach == MTC_APPROACH_BASIC) continue;

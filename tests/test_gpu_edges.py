@@ -97,3 +97,32 @@ def test_root_segments_per_wavefront(n):
         e = orc.checkpoint(host, make_baseline=(k == 0), threads=8)
         assert g == e, (k, first_mismatch(g, e))
     d.close()
+
+
+def test_handle_alternates_between_alone_and_a_large_batch():
+    """A handle whose root segments are planned for steps alone joins a step of many
+    tiles (a new plan with four tiles a segment) and returns: the oracle's diffs."""
+    C, n, members = 8, 1 << 21, 8
+    rng = np.random.default_rng(8)
+    host = [rng.integers(0, 256, n * C, dtype=np.uint8)]
+    for _ in range(4):
+        w = host[-1].copy().reshape(n, C)
+        at = rng.random(n) < 0.01
+        w[at] = rng.integers(0, 256, (int(at.sum()), C), dtype=np.uint8)
+        at = np.nonzero(rng.random(n) < 0.005)[0]
+        w[at] = w[rng.integers(0, n, at.size)]
+        host.append(w.reshape(-1))
+    bufs = [torch.from_numpy(v).to("cuda:0") for v in host]
+    ds, batch, orc = [M.TreeDeduplicator(C) for _ in range(members)], M.Batch(), O.OracleDedup(C)
+    for k, b in enumerate(bufs):
+        print(f"alternating step {k}", flush=True)
+        if k % 2 == 0:
+            got = [d.checkpoint(b, make_baseline=(k == 0)) for d in ds]
+        else:
+            got = batch.checkpoint(ds, [b] * members, copy=True)
+        e = orc.checkpoint(host[k], make_baseline=(k == 0), threads=8)
+        for g in got:
+            assert g == e, (k, first_mismatch(g, e))
+    for d in ds:
+        d.close()
+    batch.close()
