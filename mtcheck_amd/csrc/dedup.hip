@@ -2341,6 +2341,12 @@ static uint64_t first_stage_tiles(uint64_t n, uint32_t fuse) {
 
 static uint32_t sweep_a_tiles(const mtc_dedup* h, uint64_t step_tiles) {
   if (h->tune.sweep_tiles_a) return h->tune.sweep_tiles_a;
+  // A small tree of two stages with tiles of few positions (fewer levels fused) runs
+  // as one block (a tail), each wavefront with as many positions as a full tile has.
+  // (Full tiles, several a wavefront, are better off in a launch of their own: 1 MiB
+  // of 128-byte chunks, four checkpoints, 116 us as a tail of 16 wavefronts, 74 us.)
+  const uint32_t per_wave = 256u >> h->plan_fuse;
+  if (h->stages.size() == 2 && per_wave > 1 && first_stage_tiles(h->n, h->plan_fuse) <= per_wave * kTailWaves) return per_wave;
   return step_tiles <= 65536 ? 1u : step_tiles <= 262144 ? 2u : 8u;
 }
 
