@@ -16,18 +16,13 @@
 namespace mtc {
 
 constexpr uint32_t kRThreads = 256;
-constexpr uint64_t kSlotBits = 40;
-constexpr uint64_t kSlotMask = (1ull << kSlotBits) - 1;
-constexpr uint64_t kNoCover = ~0ull;
-
-struct ChainDiff {
-  const uint8_t* base;     // device
-  uint64_t size;
-  mtc_header h;
-  uint64_t off_first, off_table, off_shift, off_data;
-  uint64_t data_chunks;    // whole chunks the data section can hold
-  uint64_t region_base;    // first entry of this diff in the flat region-offset array
-};
+constexpr uint64_t kNoKey = ~0ull;
+// Cover entries: the covering diff's chain position + 1 above the byte address of the
+// chunk's bytes; zero: not covered.  Diffs are covered in any order, the newest wins
+// by atomic max.  Chains of more than kCoverPos diffs take several passes.
+constexpr uint32_t kAddrBits = 47;
+constexpr uint64_t kAddrMask = (1ull << kAddrBits) - 1;
+constexpr uint32_t kCoverPos = (1u << (64 - kAddrBits)) - 1;
 
 static uint32_t rgrid(uint64_t items, uint32_t cap = 1u << 20) {
   uint64_t g = (items + kRThreads - 1) / kRThreads;
@@ -46,216 +41,412 @@ __device__ __forceinline__ uint64_t rs_home(uint64_t key, uint64_t mask) {
   return key & mask;
 }
 
-// One diff's first-occurrence roots: the region size of each, and its entry in
-// the (diff position, root node) set that resolves shifted entries' sources.
-// idb: added to every stored id (0 for tree diffs, whose ids are node ids; n - 1
-// for basic diffs, whose ids are chunk indices: leaf n - 1 + c holds chunk c).
-__global__ void k_r_roots(const uint8_t* first, uint32_t F, Geo g, uint32_t* sizes, uint32_t pos, uint64_t* keys,
-                          uint32_t* vals, uint64_t mask, uint32_t* err, uint32_t idb) {
-  const uint32_t i = blockIdx.x * kRThreads + threadIdx.x;
-  if (i >= F) return;
-  const uint64_t node = (uint64_t)ld32(first + 4ull * i) + idb;
-  if (node >= 2ull * g.n - 1) {
-    atomicOr(err, ERR_CORRUPT);
-    sizes[i] = 0;
-    return;
-  }
-  sizes[i] = leaf_count(g, (uint32_t)node);
-  const uint64_t key = ((uint64_t)pos << 32) | node;
-  uint64_t s = rs_home(key, mask);
-  for (uint64_t probes = 0; probes <= mask; probes++) {
-    const uint64_t old = atomicCAS((unsigned long long*)&keys[s], (unsigned long long)kNoCover, (unsigned long long)key);
-    if (old == kNoCover) {
-      vals[s] = i;
-      return;
-    }
-    if (old == key) {  // the same root twice in one diff
-      atomicOr(err, ERR_CORRUPT);
-      return;
-    }
-    s = (s + 1) & mask;
-  }
-  atomicOr(err, ERR_TABLE_FULL);
-}
-
 __device__ __forceinline__ uint32_t rs_find(const uint64_t* keys, const uint32_t* vals, uint64_t mask, uint64_t key) {
   uint64_t s = rs_home(key, mask);
   for (uint64_t probes = 0; probes <= mask; probes++) {
     const uint64_t k = keys[s];
     if (k == key) return vals[s];
-    if (k == kNoCover) return ~0u;
+    if (k == kNoKey) return ~0u;
     s = (s + 1) & mask;
   }
   return ~0u;
 }
 
-__global__ void k_r_fill64(uint64_t* p, uint64_t count, uint64_t v) {
-  for (uint64_t i = (uint64_t)blockIdx.x * kRThreads + threadIdx.x; i < count; i += (uint64_t)gridDim.x * kRThreads)
-    p[i] = v;
-}
+// The tables of a chain of L diffs, by chain position p (one array of 64-bit words;
+// prefix arrays have L + 1 entries).
+enum : uint32_t { M_FIRST, M_DATA, M_CHUNKS, M_SHIFT, M_TABLE, M_PS, M_CUM, M_REGION, M_CBASE, M_SBASE, M_ARRAYS };
+__host__ __device__ constexpr uint64_t meta_words(uint64_t L) { return M_ARRAYS * L + 3; }
 
-__global__ void k_r_fill32(uint32_t* p, uint64_t count, uint32_t v) {
-  for (uint64_t i = (uint64_t)blockIdx.x * kRThreads + threadIdx.x; i < count; i += (uint64_t)gridDim.x * kRThreads)
-    p[i] = v;
-}
-
-// Chunks of one diff's first-occurrence regions: cover[chunk] = (pos, data slot).
-__global__ void k_r_cover_first(const uint8_t* first, uint32_t F, const uint32_t* region_off, uint64_t total, Geo g,
-                                uint32_t pos, uint64_t* cover, uint32_t idb) {
-  for (uint64_t j = (uint64_t)blockIdx.x * kRThreads + threadIdx.x; j < total; j += (uint64_t)gridDim.x * kRThreads) {
-    uint32_t lo = 0, hi = F;
-    while (hi - lo > 1) {
-      const uint32_t mid = (lo + hi) >> 1;
-      if (region_off[mid] <= j) lo = mid;
-      else hi = mid;
-    }
-    uint32_t st[2], ct[2];
-    const int r = leaf_runs(g, ld32(first + 4ull * lo) + idb, st, ct);
-    const uint32_t chunk = run_at(r, st, ct, (uint32_t)(j - region_off[lo]));
-    cover[chunk] = ((uint64_t)pos << kSlotBits) | j;
-  }
-}
-
-struct RShiftArgs {
-  const uint8_t* shift;   // S (node, prev) pairs of this diff
-  uint32_t S;
-  const uint32_t* cum;    // inclusive running count by checkpoint id, ref..chkpt
-  uint32_t ncum;
+struct Chain {
+  uint32_t L;
+  uint32_t n, C;
   uint32_t ref;
-  uint32_t pos;
+  uint32_t idb;      // added to every stored id (0 for tree diffs, whose ids are node ids; n - 1
+                     // for basic diffs, whose ids are chunk indices: leaf n - 1 + c holds chunk c)
   Geo g;
-  const uint64_t* set_keys;
-  const uint32_t* set_vals;
-  uint64_t set_mask;
-  const uint64_t* first_ptr;   // per chain position: device address of its F roots
-  const uint64_t* region_base; // per chain position: first entry in region_off_all
-  const uint32_t* region_off_all;
+  const uint64_t* meta;
+  uint32_t* region;  // per root of every diff, then one end marker: sizes, then their running totals
+  uint32_t* cum;     // per diff: inclusive running count of its shifted entries by checkpoint id
+  uint64_t* keys;    // the (position, root) set
+  uint32_t* vals;
+  uint64_t mask;
   uint64_t* cover;
   uint32_t* err;
+  volatile uint32_t* err_host;  // pinned copy (may be null): an error's bits, one word each
+
+  __device__ const uint64_t* first() const { return meta; }                        // address of the F roots
+  __device__ const uint64_t* data() const { return meta + (uint64_t)M_DATA * L; }  // address of the data section
+  __device__ const uint64_t* chunks() const { return meta + (uint64_t)M_CHUNKS * L; }  // whole chunks it can hold
+  __device__ const uint64_t* shift() const { return meta + (uint64_t)M_SHIFT * L; }    // address of the S pairs
+  __device__ const uint64_t* table() const { return meta + (uint64_t)M_TABLE * L; }    // address of the P table
+  __device__ const uint64_t* ps() const { return meta + (uint64_t)M_PS * L; }          // P << 32 | S
+  __device__ const uint64_t* cum_off() const { return meta + (uint64_t)M_CUM * L; }
+  __device__ const uint64_t* region_base() const { return meta + (uint64_t)M_REGION * L; }     // L + 1
+  __device__ const uint64_t* chunk_base() const { return meta + (uint64_t)M_CBASE * L + 1; }   // L + 1: running chunks()
+  __device__ const uint64_t* shift_base() const { return meta + (uint64_t)M_SBASE * L + 2; }   // L + 1: running S
+
+  __device__ void fail(uint32_t bit) const {
+    atomicOr(err, bit);
+    if (err_host) err_host[bit == ERR_TABLE_FULL ? 1 : 0] = bit;
+  }
+  __device__ uint32_t roots(uint32_t p) const { return (uint32_t)(region_base()[p + 1] - region_base()[p] - 1); }
 };
 
-// Shifted-duplicate entries of one diff: each leaf of `node` takes the data slot
-// of the matching leaf of `prev` inside the source diff's region
-// (src/tree_approach.cpp:887-925, 1058-1118).
-__global__ void k_r_cover_shift(RShiftArgs a) {
-  const uint32_t i = blockIdx.x * kRThreads + threadIdx.x;
-  if (i >= a.S) return;
-  const uint32_t node = ld32(a.shift + 8ull * i), prev = ld32(a.shift + 8ull * i + 4);
-  const uint64_t nodes = 2ull * a.g.n - 1;
-  if (node >= nodes || prev >= nodes) {
-    atomicOr(a.err, ERR_CORRUPT);
-    return;
-  }
-  uint32_t lo = 0, hi = a.ncum;  // smallest checkpoint whose running count exceeds i
-  while (lo < hi) {
+// The position whose share of a prefix array (L + 1 entries) holds i.
+__device__ __forceinline__ uint32_t owner(const uint64_t* base, uint32_t lo, uint32_t hi, uint64_t i) {
+  while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
-    if (i < a.cum[mid]) hi = mid;
-    else lo = mid + 1;
+    if (base[mid] <= i) lo = mid;
+    else hi = mid;
   }
-  if (lo >= a.ncum || lo > a.pos) {
-    atomicOr(a.err, ERR_CORRUPT);
+  return lo;
+}
+
+// Everything a restart reads before it is written starts here: the chain's tables
+// (from `src`, host-visible memory), the set, the cover array and the counts.
+__global__ __launch_bounds__(kRThreads) void k_r_init(const uint64_t* src, uint64_t* meta, uint64_t meta_n, uint64_t* keys,
+                                                      uint64_t keys_n, uint64_t* cover, uint64_t cover_n, uint32_t* cum,
+                                                      uint64_t cum_n, uint32_t* err) {
+  const uint64_t t = (uint64_t)blockIdx.x * kRThreads + threadIdx.x, s = (uint64_t)gridDim.x * kRThreads;
+  if (t == 0) *err = 0;
+  if (src)
+    for (uint64_t i = t; i < meta_n; i += s) meta[i] = src[i];
+  for (uint64_t i = t; i < keys_n; i += s) keys[i] = kNoKey;
+  for (uint64_t i = t; i < cum_n; i += s) cum[i] = 0;
+  ulonglong2* c2 = reinterpret_cast<ulonglong2*>(cover);
+  for (uint64_t i = t; i < cover_n / 2; i += s) c2[i] = ulonglong2{0, 0};
+  if (t == 0 && (cover_n & 1)) cover[cover_n - 1] = 0;
+}
+
+// One block: the inclusive running count, by checkpoint id ref..ref+p, of the shifted
+// entries of diff p (its prior-checkpoint table, src/tree_approach.cpp:872-883),
+// checked against the diff's S.
+__device__ void cum_block(const Chain& c, uint32_t p) {
+  __shared__ uint32_t ws[kRThreads / 64];
+  const uint32_t P = (uint32_t)(c.ps()[p] >> 32), S = (uint32_t)c.ps()[p];
+  const uint8_t* tab = reinterpret_cast<const uint8_t*>(c.table()[p]);
+  uint32_t* cnt = c.cum + c.cum_off()[p];
+  for (uint32_t i = threadIdx.x; i < P; i += kRThreads) {
+    const uint32_t id = ld32(tab + 8ull * i), m = ld32(tab + 8ull * i + 4);
+    if (id < c.ref || id - c.ref > p) c.fail(ERR_CORRUPT);
+    else atomicAdd(&cnt[id - c.ref], m);
+  }
+  __syncthreads();
+  const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  uint32_t carry = 0;
+  for (uint64_t b = 0; b <= p; b += kRThreads) {
+    const uint64_t i = b + threadIdx.x;
+    uint32_t x = i <= p ? __hip_atomic_load(&cnt[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(x, o);
+      if (lane >= (uint32_t)o) x += y;
+    }
+    if (lane == 63) ws[w] = x;
+    __syncthreads();
+    uint32_t pre = carry;
+    for (uint32_t k = 0; k < kRThreads / 64; k++) {
+      if (k < w) pre += ws[k];
+      carry += ws[k];
+    }
+    if (i <= p) cnt[i] = pre + x;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0 && carry != S) c.fail(ERR_CORRUPT);
+}
+
+// Every diff's first-occurrence roots in one launch: the region size of each, and its
+// entry in the (diff position, root node) set that resolves shifted entries' sources.
+// The last L blocks build the running counts of shifted entries.
+__global__ __launch_bounds__(kRThreads) void k_r_roots(Chain c, uint32_t nblk) {
+  if (blockIdx.x >= nblk) {
+    cum_block(c, blockIdx.x - nblk);
     return;
   }
-  const uint32_t spos = lo;  // chain position of the source checkpoint
-  uint32_t anc = prev, region = ~0u;
-  while (true) {
-    region = rs_find(a.set_keys, a.set_vals, a.set_mask, ((uint64_t)spos << 32) | anc);
-    if (region != ~0u || anc == 0) break;
-    anc = (anc - 1) >> 1;
-  }
-  if (region == ~0u) {
-    atomicOr(a.err, ERR_CORRUPT);
-    return;
-  }
-  const uint8_t* sfirst = reinterpret_cast<const uint8_t*>(a.first_ptr[spos]);
-  const uint32_t root = ld32(sfirst + 4ull * region);
-  const uint32_t rbase = a.region_off_all[a.region_base[spos] + region];
-  uint32_t rs[2], rc[2], ns[2], nc[2], ps[2], pc[2];
-  const int rr = leaf_runs(a.g, root, rs, rc);
-  const int nr = leaf_runs(a.g, node, ns, nc);
-  const int pr = leaf_runs(a.g, prev, ps, pc);
-  const uint32_t cnt = nc[0] + (nr == 2 ? nc[1] : 0);
-  if (cnt != pc[0] + (pr == 2 ? pc[1] : 0)) {
-    atomicOr(a.err, ERR_CORRUPT);
-    return;
-  }
-  for (uint32_t j = 0; j < cnt; j++) {
-    const uint32_t dst_chunk = run_at(nr, ns, nc, j);
-    const uint32_t src_chunk = run_at(pr, ps, pc, j);
-    const uint64_t slot = rbase + run_rank(rr, rs, rc, src_chunk);
-    a.cover[dst_chunk] = ((uint64_t)spos << kSlotBits) | slot;
+  const uint64_t* base = c.region_base();
+  const uint64_t words = base[c.L];
+  for (uint64_t i = (uint64_t)blockIdx.x * kRThreads + threadIdx.x; i < words; i += (uint64_t)nblk * kRThreads) {
+    const uint32_t p = owner(base, 0, c.L, i);
+    if (i + 1 == base[p + 1]) {  // the diff's end marker
+      c.region[i] = 0;
+      continue;
+    }
+    const uint32_t r = (uint32_t)(i - base[p]);
+    const uint64_t node = (uint64_t)ld32(reinterpret_cast<const uint8_t*>(c.first()[p]) + 4ull * r) + c.idb;
+    if (node >= 2ull * c.g.n - 1) {
+      c.fail(ERR_CORRUPT);
+      c.region[i] = 0;
+      continue;
+    }
+    c.region[i] = leaf_count(c.g, (uint32_t)node);
+    const uint64_t key = ((uint64_t)p << 32) | node;
+    uint64_t s = rs_home(key, c.mask);
+    bool placed = false;
+    for (uint64_t probes = 0; probes <= c.mask; probes++) {
+      const uint64_t old = atomicCAS((unsigned long long*)&c.keys[s], (unsigned long long)kNoKey, (unsigned long long)key);
+      if (old == kNoKey) {
+        c.vals[s] = r;
+        placed = true;
+        break;
+      }
+      if (old == key) {  // the same root twice in one diff
+        c.fail(ERR_CORRUPT);
+        placed = true;
+        break;
+      }
+      s = (s + 1) & c.mask;
+    }
+    if (!placed) c.fail(ERR_TABLE_FULL);
   }
 }
 
+// One diff's regions: slots of its data section -> chunks, the last region found being
+// kept for the next slot (a baseline often has one region for the whole buffer).
+struct Regions {
+  const uint32_t* reg;
+  const uint8_t* roots;
+  uint32_t F, g0, total;
+  uint32_t from = 1, to = 0;  // slots of the region found last
+  uint32_t run0 = 0, run1 = 0, cnt0 = 0;  // its chunks: cnt0 from run0 on, then from run1 on
 
-// One scatter copy: out[chunk] = data section of diff pos, slot.
-__global__ __launch_bounds__(kRThreads) void k_r_copy(const uint64_t* cover, uint32_t n, uint32_t C, uint64_t datalen,
-                                                       const uint64_t* data_ptr, const uint64_t* data_chunks,
-                                                       uint8_t* out, int vec, uint32_t* err) {
-  __shared__ uint64_t s_src[kRThreads];
-  const uint32_t U = vec ? C / 16 : C;
-  for (uint64_t tile = blockIdx.x; tile * kRThreads < n; tile += gridDim.x) {
-    const uint64_t c0 = tile * kRThreads;
-    const uint64_t c = c0 + threadIdx.x;
-    if (c < n) {
-      const uint64_t e = cover[c];
-      uint64_t src = 0;
-      if (e == kNoCover) {
-        atomicOr(err, ERR_CORRUPT);
-      } else {
-        const uint32_t pos = (uint32_t)(e >> kSlotBits);
-        const uint64_t slot = e & kSlotMask;
-        if (slot >= data_chunks[pos]) atomicOr(err, ERR_CORRUPT);
-        else src = data_ptr[pos] + slot * C;
-      }
-      s_src[threadIdx.x] = src;
+  __device__ Regions(const Chain& c, uint32_t p)
+      : reg(c.region + c.region_base()[p]), roots(reinterpret_cast<const uint8_t*>(c.first()[p])), F(c.roots(p)),
+        g0(reg[0]), total(reg[F] - g0) {
+    if (total > c.chunks()[p]) {  // the data section is shorter than its regions
+      c.fail(ERR_CORRUPT);
+      total = 0;
     }
-    __syncthreads();
-    const uint64_t cnt = ((uint64_t)n - c0 < kRThreads) ? (uint64_t)n - c0 : kRThreads;
-    for (uint64_t u = threadIdx.x; u < cnt * U; u += kRThreads) {
-      const uint32_t jj = (uint32_t)(u / U), w = (uint32_t)(u % U);
-      const uint64_t src = s_src[jj];
-      if (!src) continue;
-      const uint64_t doff = (c0 + jj) * C;
-      const uint8_t* sp = reinterpret_cast<const uint8_t*>(src);
-      if (vec) {
-        const uint64_t b0 = doff + 16ull * w;
-        if (b0 + 16 <= datalen) {
-          st_stream16(out + b0, ld_stream16_a4(sp + 16ull * w));
-        } else {
-          for (uint32_t b = 0; b < 16 && b0 + b < datalen; b++) out[b0 + b] = sp[16ull * w + b];
+  }
+  __device__ uint32_t chunk(const Chain& c, uint32_t j) {  // j < total
+    if (j < from || j >= to) {
+      uint32_t lo = 0, hi = F;
+      while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (reg[mid] - g0 <= j) lo = mid;
+        else hi = mid;
+      }
+      from = reg[lo] - g0;
+      to = reg[lo + 1] - g0;
+      uint32_t st[2], ct[2];
+      const int r = leaf_runs(c.g, ld32(roots + 4ull * lo) + c.idb, st, ct);
+      run0 = st[0];
+      run1 = r == 2 ? st[1] : 0u;
+      cnt0 = ct[0];
+    }
+    const uint32_t k = j - from;
+    return k < cnt0 ? run0 + k : run1 + (k - cnt0);
+  }
+};
+
+// Chunks of the first-occurrence regions of the pass's oldest diff, which hold nearly
+// the whole buffer when it is the baseline: plain stores, nothing else writes the
+// cover meanwhile (atomic max runs at a third of their rate).
+__global__ __launch_bounds__(kRThreads) void k_r_cover_base(Chain c, uint32_t p) {
+  if (*c.err) return;
+  Regions d(c, p);
+  const uint64_t data = c.data()[p];
+  for (uint64_t j = (uint64_t)blockIdx.x * kRThreads + threadIdx.x; j < d.total; j += (uint64_t)gridDim.x * kRThreads)
+    c.cover[d.chunk(c, (uint32_t)j)] = (1ull << kAddrBits) | (data + j * c.C);
+}
+
+// The other diffs of a pass (positions lo .. hi - 1; lo's regions are covered
+// already), in one launch: nblk blocks for the first-occurrence chunks, the rest for
+// the shifted entries.  Each leaf of a shifted entry's `node` takes the data slot of
+// the matching leaf of `prev` inside the source diff's region
+// (src/tree_approach.cpp:887-925, 1058-1118); a wavefront shares the leaves of its
+// larger entries.
+constexpr uint32_t kShiftOwn = 4;  // most leaves a lane covers by itself
+__global__ __launch_bounds__(kRThreads) void k_r_cover_rest(Chain c, uint32_t lo, uint32_t hi, uint32_t nblk) {
+  if (*c.err) return;
+  if (blockIdx.x < nblk) {
+    const uint64_t* base = c.chunk_base();
+    const uint64_t end = base[hi];
+    for (uint64_t j = base[lo + 1] + (uint64_t)blockIdx.x * kRThreads + threadIdx.x; j < end; j += (uint64_t)nblk * kRThreads) {
+      const uint32_t p = owner(base, lo + 1, hi, j);
+      const uint64_t slot = j - base[p];
+      Regions d(c, p);
+      if (slot >= d.total) continue;
+      atomicMax((unsigned long long*)&c.cover[d.chunk(c, (uint32_t)slot)],
+                (unsigned long long)(((uint64_t)(p - lo + 1) << kAddrBits) | (c.data()[p] + slot * c.C)));
+    }
+    return;
+  }
+  const uint64_t* base = c.shift_base();
+  const uint64_t end = base[hi];
+  const uint64_t nodes = 2ull * c.g.n - 1;
+  const uint32_t lane = lane_id();
+  const uint64_t stride = (uint64_t)(gridDim.x - nblk) * kRThreads;
+  for (uint64_t w0 = base[lo] + (uint64_t)(blockIdx.x - nblk) * kRThreads + (threadIdx.x & ~63u); w0 < end; w0 += stride) {
+    const uint64_t i = w0 + lane;
+    uint32_t node = 0, prev = 0, root = 0, rbase = 0, spos = 0, cnt = 0, p = 0;
+    bool ok = i < end;
+    if (ok) {
+      p = owner(base, lo, hi, i);
+      const uint32_t e = (uint32_t)(i - base[p]);
+      const uint8_t* sh = reinterpret_cast<const uint8_t*>(c.shift()[p]) + 8ull * e;
+      node = ld32(sh);
+      prev = ld32(sh + 4);
+      ok = node < nodes && prev < nodes;
+      if (ok) {
+        const uint32_t* cum = c.cum + c.cum_off()[p];
+        uint32_t l = 0, h = p + 1;  // smallest checkpoint whose running count exceeds e
+        while (l < h) {
+          const uint32_t mid = (l + h) >> 1;
+          if (e < cum[mid]) h = mid;
+          else l = mid + 1;
         }
-      } else if (doff + w < datalen) {
-        out[doff + w] = sp[w];
+        spos = l;  // chain position of the source checkpoint
+        ok = l <= p;
+      }
+      uint32_t region = ~0u;
+      if (ok) {
+        for (uint32_t anc = prev;; anc = (anc - 1) >> 1) {
+          region = rs_find(c.keys, c.vals, c.mask, ((uint64_t)spos << 32) | anc);
+          if (region != ~0u || anc == 0) break;
+        }
+        ok = region != ~0u;
+      }
+      if (ok) {
+        root = ld32(reinterpret_cast<const uint8_t*>(c.first()[spos]) + 4ull * region) + c.idb;
+        const uint32_t* reg = c.region + c.region_base()[spos];
+        rbase = reg[region] - reg[0];
+        cnt = leaf_count(c.g, node);
+        ok = cnt == leaf_count(c.g, prev);
+      }
+      if (!ok) {
+        c.fail(ERR_CORRUPT);
+        cnt = 0;
       }
     }
-    __syncthreads();
+    auto cover_leaves = [&](uint32_t nd, uint32_t pv, uint32_t rt, uint32_t rb, uint32_t sp, uint32_t pos, uint32_t from,
+                            uint32_t step, uint32_t count) {
+      uint32_t rs[2], rc[2], ns[2], nc[2], ps[2], pc[2];
+      const int rr = leaf_runs(c.g, rt, rs, rc);
+      const int nr = leaf_runs(c.g, nd, ns, nc);
+      const int pr = leaf_runs(c.g, pv, ps, pc);
+      const uint64_t top = (uint64_t)(pos - lo + 1) << kAddrBits, data = c.data()[sp], cap = c.chunks()[sp];
+      for (uint32_t j = from; j < count; j += step) {
+        const uint64_t slot = (uint64_t)rb + run_rank(rr, rs, rc, run_at(pr, ps, pc, j));
+        if (slot >= cap) {
+          c.fail(ERR_CORRUPT);
+          break;
+        }
+        atomicMax((unsigned long long*)&c.cover[run_at(nr, ns, nc, j)], (unsigned long long)(top | (data + slot * c.C)));
+      }
+    };
+    if (cnt && cnt <= kShiftOwn) cover_leaves(node, prev, root, rbase, spos, p, 0, 1, cnt);
+    uint64_t big = __ballot(cnt > kShiftOwn);
+    while (big) {
+      const int l = __ffsll((long long)big) - 1;
+      big &= big - 1;
+      cover_leaves(__shfl(node, l), __shfl(prev, l), __shfl(root, l), __shfl(rbase, l), __shfl(spos, l), __shfl(p, l), lane,
+                   64, __shfl(cnt, l));
+    }
+  }
+}
+
+// Between two passes over a long chain: the cover keeps its addresses below every
+// position of the next pass.
+__global__ void k_r_cover_age(uint64_t* cover, uint64_t n) {
+  for (uint64_t i = (uint64_t)blockIdx.x * kRThreads + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kRThreads)
+    if (cover[i]) cover[i] &= kAddrMask;
+}
+
+// One scatter copy: out[chunk] = the bytes its cover names.  No loop: a block copies
+// 16 KiB with four 16-byte loads a thread before its stores (a wait for a load also
+// waits for the stores before it).  The card's copy rate bounds it: 8 GiB in 3.04 ms
+// (5.65 TB/s read and written), 3.53 ms as 8192 looping blocks.  C a power of
+// two of at least 16, 16-byte aligned out, 4-byte aligned data sections.
+constexpr uint32_t kCopyUnits = 4;
+__global__ __launch_bounds__(kRThreads) void k_r_copy(Chain c, uint64_t datalen, uint32_t ulog, uint8_t* out) {
+  if (*c.err) return;
+  const uint64_t units = datalen / 16, u0 = (uint64_t)blockIdx.x * (kCopyUnits * kRThreads) + threadIdx.x;
+  uint64_t e[kCopyUnits];
+#pragma unroll
+  for (uint32_t i = 0; i < kCopyUnits; i++) {
+    const uint64_t u = u0 + i * kRThreads;
+    e[i] = u < units ? c.cover[u >> ulog] : 1;
+    if (!e[i]) c.fail(ERR_CORRUPT);
+  }
+  uint4 v[kCopyUnits];
+#pragma unroll
+  for (uint32_t i = 0; i < kCopyUnits; i++) {
+    const uint64_t u = u0 + i * kRThreads;
+    if (u < units && e[i])
+      v[i] = ld_stream16_a4(reinterpret_cast<const uint8_t*>(e[i] & kAddrMask) + 16 * (u & ((1u << ulog) - 1)));
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < kCopyUnits; i++) {
+    const uint64_t u = u0 + i * kRThreads;
+    if (u < units && e[i]) st_stream16(out + 16 * u, v[i]);
+  }
+  if (blockIdx.x == 0 && threadIdx.x < (datalen & 15)) {  // the short last chunk's last bytes
+    const uint64_t o = 16 * units + threadIdx.x, ce = c.cover[o / c.C];
+    if (ce) out[o] = reinterpret_cast<const uint8_t*>(ce & kAddrMask)[o % c.C];
+    else c.fail(ERR_CORRUPT);
+  }
+}
+
+// The same for any chunk size and alignment: 16 bytes of the output per thread, cut
+// out of the aligned words that hold them where they lie in one chunk or in two that
+// are neighbours in the diff too, byte by byte elsewhere.
+__global__ __launch_bounds__(kRThreads) void k_r_copy_any(Chain c, uint64_t datalen, uint8_t* out) {
+  if (*c.err) return;
+  const uint64_t o = 16 * ((uint64_t)blockIdx.x * kRThreads + threadIdx.x);
+  if (o >= datalen) return;
+  const uint64_t k = o / c.C;
+  const uint32_t w = (uint32_t)(o - k * c.C);
+  const uint64_t e = c.cover[k];
+  if (((uintptr_t)out & 3) == 0 && o + 16 <= datalen && e &&
+      ((uint64_t)w + 16 <= c.C || ((uint64_t)w + 16 <= 2ull * c.C && (c.cover[k + 1] & kAddrMask) == (e & kAddrMask) + c.C))) {
+    const uint64_t src = (e & kAddrMask) + w;
+    const uint32_t sh = (uint32_t)src & 3;
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(src - sh);
+    const uint4 v = ld_stream16_a4(q);
+    const uint32_t x = sh ? q[4] : 0u;
+    st_stream16_a4(out + o, uint4{__builtin_amdgcn_alignbyte(v.y, v.x, sh), __builtin_amdgcn_alignbyte(v.z, v.y, sh),
+                                  __builtin_amdgcn_alignbyte(v.w, v.z, sh), __builtin_amdgcn_alignbyte(x, v.w, sh)});
+    return;
+  }
+#pragma unroll 1
+  for (uint64_t b = o; b < o + 16 && b < datalen; b++) {
+    const uint64_t kb = b / c.C, ce = c.cover[kb];
+    if (ce) out[b] = reinterpret_cast<const uint8_t*>(ce & kAddrMask)[b - kb * c.C];
+    else c.fail(ERR_CORRUPT);
+  }
+}
+
+// The headers of the chain that ends in diff k (a device chain's), read where they lie:
+// hdr[0] is k's, hdr[1 + i] that of its i-th diff (ref_id + i).  ptrs and sizes (from
+// diff `first` on; entries below the chain are not looked at) and hdr are pinned host
+// memory: one launch and one synchronisation for the whole chain.  A missing or short
+// diff leaves its header as it is.
+__global__ __launch_bounds__(kRThreads) void k_r_headers(const uint64_t* ptrs, const uint64_t* sizes, uint32_t first,
+                                                         uint32_t k, uint32_t* hdr) {
+  const uint32_t ref = ld32(reinterpret_cast<const uint8_t*>(ptrs[k - first]));
+  const uint32_t L = ref >= first && ref <= k ? k - ref + 1 : 0u;
+  for (uint64_t i = (uint64_t)blockIdx.x * kRThreads + threadIdx.x; i < 8ull * (L + 1ull); i += (uint64_t)gridDim.x * kRThreads) {
+    const uint64_t h = i / 8, w = i % 8;
+    const uint64_t idx = (h == 0 ? k : ref + (h - 1)) - first;
+    if (ptrs[idx] && sizes[idx] >= sizeof(mtc_header)) hdr[i] = ld32(reinterpret_cast<const uint8_t*>(ptrs[idx]) + 4 * w);
   }
 }
 
 struct RestartScratch {
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};  // start, chain uploaded, done
   Workspace ws;
-  DevBuf<uint32_t> err, region_off, set_vals;
+  DevBuf<uint32_t> err, region, set_vals, cum;
   DevBuf<uint64_t> set_keys, cover, meta;
-  uint8_t* stage = nullptr;  // pinned: per-position tables for the kernels
+  uint8_t* stage = nullptr;  // pinned: diff addresses and sizes, headers, per-position tables, error words
   uint64_t stage_cap = 0;
-  uint8_t* hstage = nullptr;  // pinned: headers and prior-checkpoint tables of device chains
-  uint64_t hstage_cap = 0;
-  uint8_t* totals = nullptr;  // pinned: every position's region total
-  uint64_t totals_cap = 0;
-  std::vector<uint32_t> totals_h;
+  bool busy = false;  // a restart that did not reach its end may still use the scratch
 };
 
-// Pinned staging that grows by at least half; the device is idle before the old
-// block is freed, since an earlier restart's copy may have used it.
+// Pinned staging that grows by at least half (no restart is using it).
 static void pinned_reserve(uint8_t*& p, uint64_t& cap, uint64_t want) {
   if (want <= cap) return;
   const uint64_t c = std::max<uint64_t>({want, cap + cap / 2, 4096});
-  if (p) {
-    MTC_HIP(hipDeviceSynchronize());
-    (void)hipHostFree(p);
-  }
+  if (p) (void)hipHostFree(p);
   p = nullptr;
   cap = 0;
   MTC_HIP(hipHostMalloc((void**)&p, c));
@@ -284,13 +475,119 @@ void last_restart_times(float* upload_ms, float* total_ms) {
   if (total_ms) *total_ms = g_restart_ms[1];
 }
 
+static void throw_err(uint32_t e) {
+  if (e & ERR_TABLE_FULL) throw Status{MTC_ERR_OUT_OF_MEMORY, "restart root set overflow"};
+  if (e) throw Status{MTC_ERR_CORRUPT_DIFF, "diff chain is inconsistent (err bits " + std::to_string(e) + ")"};
+}
+
 static void check_err(uint32_t* err_d, hipStream_t st) {
   uint32_t e = 0;
   MTC_HIP(hipMemcpyAsync(&e, err_d, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
   MTC_HIP(hipStreamSynchronize(st));
-  if (e & ERR_TABLE_FULL) throw Status{MTC_ERR_OUT_OF_MEMORY, "restart root set overflow"};
-  if (e) throw Status{MTC_ERR_CORRUPT_DIFF, "diff chain is inconsistent (err bits " + std::to_string(e) + ")"};
+  throw_err(e);
 }
+
+// The header of the requested checkpoint.
+static void check_last(const mtc_header& hk, uint32_t k, uint64_t out_len) {
+  if (hk.chkpt_id != k || hk.ref_id > k || hk.chunk_size == 0 || hk.datalen == 0)
+    throw Status{MTC_ERR_CORRUPT_DIFF, "bad header of the requested diff"};
+  if (out_len < hk.datalen) throw Status{MTC_ERR_BUFFER_TOO_SMALL, "output shorter than datalen"};
+  if ((hk.datalen + hk.chunk_size - 1) / hk.chunk_size > (1ull << 31)) throw Status{MTC_ERR_CORRUPT_DIFF, "too many chunks"};
+}
+
+// Totals of a chain, known from its headers and sizes.
+struct ChainSums {
+  uint64_t F = 0, S = 0, chunks = 0, cum = 0;
+  bool words = true;  // every data section is 4-byte aligned
+};
+
+// Fills the tables of a chain (meta_words(L) words) from its headers, device
+// addresses and sizes; every diff is checked against the last one's header.
+static ChainSums fill_meta(uint64_t* m, const mtc_header* hs, const uint64_t* addr, const uint64_t* sizes, uint32_t L,
+                           const mtc_header& hk, bool basic) {
+  ChainSums t;
+  uint64_t* region = m + (uint64_t)M_REGION * L;
+  uint64_t* cbase = m + (uint64_t)M_CBASE * L + 1;
+  uint64_t* sbase = m + (uint64_t)M_SBASE * L + 2;
+  for (uint32_t p = 0; p < L; p++) {
+    const uint32_t idx = hk.ref_id + p;
+    const mtc_header& h = hs[p];
+    if (h.chkpt_id != idx || h.ref_id != hk.ref_id || h.datalen != hk.datalen || h.chunk_size != hk.chunk_size)
+      throw Status{MTC_ERR_CORRUPT_DIFF, "diff " + std::to_string(idx) + " does not belong to the chain"};
+    if (basic && (h.num_prior_chkpts || h.num_shift_dupl))
+      throw Status{MTC_ERR_CORRUPT_DIFF, "diff " + std::to_string(idx) + " is not a basic diff"};
+    const uint64_t off_table = 32 + 4ull * h.num_first_ocur, off_shift = off_table + 8ull * h.num_prior_chkpts;
+    const uint64_t off_data = off_shift + 8ull * h.num_shift_dupl;
+    if (off_data > sizes[p]) throw Status{MTC_ERR_CORRUPT_DIFF, "diff shorter than its metadata"};
+    const uint64_t chunks = (sizes[p] - off_data) / hk.chunk_size;
+    if (h.num_first_ocur && !chunks) throw Status{MTC_ERR_CORRUPT_DIFF, "data section shorter than its regions"};
+    if ((addr[p] + sizes[p]) >> kAddrBits) throw Status{MTC_ERR_INVALID_ARG, "diff address above 2^47"};
+    m[(uint64_t)M_FIRST * L + p] = addr[p] + 32;
+    m[(uint64_t)M_DATA * L + p] = addr[p] + off_data;
+    m[(uint64_t)M_CHUNKS * L + p] = chunks;
+    m[(uint64_t)M_SHIFT * L + p] = addr[p] + off_shift;
+    m[(uint64_t)M_TABLE * L + p] = addr[p] + off_table;
+    m[(uint64_t)M_PS * L + p] = ((uint64_t)h.num_prior_chkpts << 32) | h.num_shift_dupl;
+    m[(uint64_t)M_CUM * L + p] = t.cum;
+    region[p] = t.F + p;
+    cbase[p] = t.chunks;
+    sbase[p] = t.S;
+    t.F += h.num_first_ocur;
+    t.S += h.num_shift_dupl;
+    t.chunks += chunks;
+    t.cum += p + 1;
+    t.words = t.words && (addr[p] + off_data) % 4 == 0;
+  }
+  region[L] = t.F + L;
+  cbase[L] = t.chunks;
+  sbase[L] = t.S;
+  return t;
+}
+
+static uint64_t set_slots(uint64_t roots) {
+  uint64_t cap = 16;
+  while (cap < 2 * roots) cap <<= 1;
+  return cap;
+}
+
+// The restart's launches, the chain's tables being in c.meta's source: the set and
+// counts, the region offsets (scan), the cover and the copy.  They come in a fixed
+// number whatever the chain's length: with one set of them per diff, ten diffs took 45
+// launches, each waiting for its own chain of lookups (64 MiB of 128-byte chunks,
+// restart and 4 KiB digests: 683 us, 194 us so).  Every later kernel stops at an error of an earlier one.
+template <class Scan>
+static void launch_restart(const Chain& c, const uint64_t* meta_src, const uint64_t* m, const ChainSums& t, uint64_t datalen,
+                           uint8_t* out, hipStream_t st, Scan scan) {
+  const uint32_t L = c.L, n = c.n;
+  k_r_init<<<rgrid(std::max<uint64_t>({n / 2, t.cum, c.mask + 1, meta_words(L)})), kRThreads, 0, st>>>(
+      meta_src, const_cast<uint64_t*>(c.meta), meta_words(L), c.keys, c.mask + 1, c.cover, n, c.cum, t.cum, c.err);
+  const uint32_t rblk = rgrid(t.F + L);
+  k_r_roots<<<rblk + L, kRThreads, 0, st>>>(c, rblk);
+  MTC_HIP(hipGetLastError());
+  scan();
+  const uint64_t* cbase = m + (uint64_t)M_CBASE * L + 1;
+  const uint64_t* sbase = m + (uint64_t)M_SBASE * L + 2;
+  for (uint64_t lo = 0; lo < L; lo += kCoverPos) {
+    const uint32_t hi = (uint32_t)std::min<uint64_t>(L, lo + kCoverPos);
+    if (lo) k_r_cover_age<<<rgrid(n), kRThreads, 0, st>>>(c.cover, n);
+    k_r_cover_base<<<rgrid(cbase[lo + 1] - cbase[lo], 4096), kRThreads, 0, st>>>(c, (uint32_t)lo);
+    const uint64_t first = cbase[hi] - cbase[lo + 1], shifted = sbase[hi] - sbase[lo];
+    const uint32_t fblk = first ? rgrid(first) : 0, sblk = shifted ? rgrid(shifted) : 0;
+    if (fblk + sblk) k_r_cover_rest<<<fblk + sblk, kRThreads, 0, st>>>(c, (uint32_t)lo, hi, fblk);
+    MTC_HIP(hipGetLastError());
+  }
+  const uint32_t C = c.C;
+  if (C >= 16 && (C & (C - 1)) == 0 && (uintptr_t)out % 16 == 0 && t.words)
+    k_r_copy<<<(uint32_t)std::max<uint64_t>(1, (datalen / 16 + kCopyUnits * kRThreads - 1) / (kCopyUnits * kRThreads)), kRThreads,
+               0, st>>>(c, datalen, (uint32_t)__builtin_ctz(C) - 4, out);
+  else
+    k_r_copy_any<<<(uint32_t)((datalen + 16 * kRThreads - 1) / (16 * kRThreads)), kRThreads, 0, st>>>(c, datalen, out);
+  MTC_HIP(hipGetLastError());
+}
+
+// Device chains of which this many diffs come before the restarted one or fewer have
+// their headers read in one launch (the addresses of all of them are staged).
+constexpr uint32_t kHeadersAtOnce = 4096;
 
 void restart_impl(const void* const* diffs, const uint64_t* sizes, uint32_t count, uint32_t k, bool on_device,
                   uint8_t* out, uint64_t out_len, hipStream_t st, bool basic) {
@@ -302,215 +599,104 @@ void restart_impl(const void* const* diffs, const uint64_t* sizes, uint32_t coun
   std::lock_guard<std::mutex> guard(scratch_mutex());
   RestartScratch& rs = scratch_for(dev);
   g_restart_ms[0] = g_restart_ms[1] = 0;
+  if (rs.busy) MTC_HIP(hipDeviceSynchronize());
+  rs.busy = false;
   if (!rs.ev[0])
     for (auto& e : rs.ev) MTC_HIP(hipEventCreate(&e));
   MTC_HIP(hipEventRecord(rs.ev[0], st));
-  auto present = [&](uint32_t idx) {
+  auto present = [&](uint64_t idx) {
     if (!diffs[idx] || sizes[idx] < sizeof(mtc_header)) throw Status{MTC_ERR_CORRUPT_DIFF, "missing or short diff"};
   };
-  // Headers of device chains come back through pinned staging, one
-  // synchronisation per batch of copies.
-  auto read_headers = [&](uint32_t first, uint32_t num, mtc_header* out) {
-    for (uint32_t i = 0; i < num; i++) present(first + i);
-    if (!on_device) {
-      for (uint32_t i = 0; i < num; i++) std::memcpy(out + i, diffs[first + i], sizeof(mtc_header));
-      return;
-    }
-    pinned_reserve(rs.hstage, rs.hstage_cap, (uint64_t)num * sizeof(mtc_header));
-    for (uint32_t i = 0; i < num; i++)
-      MTC_HIP(hipMemcpyAsync(rs.hstage + (uint64_t)i * sizeof(mtc_header), diffs[first + i], sizeof(mtc_header),
-                             hipMemcpyDeviceToHost, st));
+  present(k);
+  mtc_header hk{};
+  std::vector<mtc_header> hs;
+  if (!on_device) {
+    std::memcpy(&hk, diffs[k], sizeof(hk));
+  } else if (k < kHeadersAtOnce) {
+    pinned_reserve(rs.stage, rs.stage_cap, 16ull * (k + 1) + sizeof(mtc_header) * (k + 2ull));
+    uint64_t* ptrs = reinterpret_cast<uint64_t*>(rs.stage);
+    for (uint32_t i = 0; i <= k; i++) ptrs[i] = reinterpret_cast<uint64_t>(diffs[i]);
+    std::memcpy(ptrs + (k + 1), sizes, 8ull * (k + 1));
+    mtc_header* hdr = reinterpret_cast<mtc_header*>(ptrs + 2ull * (k + 1));
+    rs.busy = true;
+    k_r_headers<<<rgrid(8ull * (k + 2), 64), kRThreads, 0, st>>>(ptrs, ptrs + (k + 1), 0, k, reinterpret_cast<uint32_t*>(hdr));
+    MTC_HIP(hipGetLastError());
     MTC_HIP(hipStreamSynchronize(st));
-    std::memcpy(out, rs.hstage, (uint64_t)num * sizeof(mtc_header));
-  };
-  mtc_header hk;
-  read_headers(k, 1, &hk);
-  if (hk.chkpt_id != k || hk.ref_id > k || hk.chunk_size == 0 || hk.datalen == 0)
-    throw Status{MTC_ERR_CORRUPT_DIFF, "bad header of the requested diff"};
-  if (out_len < hk.datalen) throw Status{MTC_ERR_BUFFER_TOO_SMALL, "output shorter than datalen"};
-  const uint64_t C = hk.chunk_size;
-  const uint64_t n64 = (hk.datalen + C - 1) / C;
-  if (n64 > (1ull << 31)) throw Status{MTC_ERR_CORRUPT_DIFF, "too many chunks"};
-  const uint32_t n = (uint32_t)n64, ref = hk.ref_id, L = k - ref + 1;
-  const Geo g = make_geo(n);
-  const uint32_t idb = basic ? n - 1 : 0;
-
-  // Chain layout, with host diffs uploaded once.
-  std::vector<ChainDiff> ch(L);
-  {
-    std::vector<mtc_header> hs(L);
-    read_headers(ref, L, hs.data());
-    for (uint32_t p = 0; p < L; p++) ch[p].h = hs[p];
-  }
-  uint64_t up_total = 0;
-  if (!on_device)
-    for (uint32_t p = 0; p < L; p++) up_total += (sizes[ref + p] + 255) & ~255ull;
-  // host chains: an exact-size upload, freed when the restart returns (a chain
-  // can be as large as the buffer, so it is not kept)
-  DevBuf<uint8_t> upload;
-  if (!on_device) upload.ensure(up_total);
-  uint64_t up_off = 0, sumF = 0, pt_total = 0;
-  for (uint32_t p = 0; p < L; p++) {
-    const uint32_t idx = ref + p;
-    ChainDiff& d = ch[p];
-    if (d.h.chkpt_id != idx || d.h.ref_id != ref || d.h.datalen != hk.datalen || d.h.chunk_size != hk.chunk_size)
-      throw Status{MTC_ERR_CORRUPT_DIFF, "diff " + std::to_string(idx) + " does not belong to the chain"};
-    if (basic && (d.h.num_prior_chkpts || d.h.num_shift_dupl))
-      throw Status{MTC_ERR_CORRUPT_DIFF, "diff " + std::to_string(idx) + " is not a basic diff"};
-    d.size = sizes[idx];
-    d.off_first = 32;
-    d.off_table = d.off_first + 4ull * d.h.num_first_ocur;
-    d.off_shift = d.off_table + 8ull * d.h.num_prior_chkpts;
-    d.off_data = d.off_shift + 8ull * d.h.num_shift_dupl;
-    if (d.off_data > d.size) throw Status{MTC_ERR_CORRUPT_DIFF, "diff shorter than its metadata"};
-    d.data_chunks = (d.size - d.off_data) / C;
-    if (on_device) {
-      d.base = static_cast<const uint8_t*>(diffs[idx]);
-    } else {
-      MTC_HIP(hipMemcpyAsync(upload.p + up_off, diffs[idx], d.size, hipMemcpyHostToDevice, st));
-      d.base = upload.p + up_off;
-      up_off += (d.size + 255) & ~255ull;
-    }
-    d.region_base = sumF + p;
-    sumF += d.h.num_first_ocur;
-    pt_total += 8ull * d.h.num_prior_chkpts;
-  }
-  MTC_HIP(hipEventRecord(rs.ev[1], st));
-  // The prior-checkpoint tables (in bounds: off_data <= size was checked above).
-  std::vector<std::vector<uint32_t>> ptables(L);
-  if (on_device && pt_total) pinned_reserve(rs.hstage, rs.hstage_cap, pt_total);
-  uint64_t pt_off = 0;
-  for (uint32_t p = 0; p < L; p++) {
-    const ChainDiff& d = ch[p];
-    const uint64_t bytes = 8ull * d.h.num_prior_chkpts;
-    ptables[p].resize(2ull * d.h.num_prior_chkpts);
-    if (!bytes) continue;
-    if (on_device)
-      MTC_HIP(hipMemcpyAsync(rs.hstage + pt_off, d.base + d.off_table, bytes, hipMemcpyDeviceToHost, st));
-    else
-      std::memcpy(ptables[p].data(), static_cast<const uint8_t*>(diffs[ref + p]) + d.off_table, bytes);
-    pt_off += bytes;
-  }
-  if (on_device && pt_total) {
-    MTC_HIP(hipStreamSynchronize(st));
-    pt_off = 0;
-    for (uint32_t p = 0; p < L; p++) {
-      const uint64_t bytes = 8ull * ch[p].h.num_prior_chkpts;
-      if (bytes) std::memcpy(ptables[p].data(), rs.hstage + pt_off, bytes);
-      pt_off += bytes;
-    }
-  }
-
-  Workspace& ws = rs.ws;
-  rs.err.ensure(1);
-  k_r_fill32<<<1, kRThreads, 0, st>>>(rs.err.p, 1, 0);
-  rs.region_off.reserve(sumF + L);
-  uint64_t set_cap = 16;
-  while (set_cap < 2 * sumF) set_cap <<= 1;
-  rs.set_keys.ensure(set_cap);
-  rs.set_vals.ensure(set_cap);
-  k_r_fill64<<<rgrid(set_cap, 65536), kRThreads, 0, st>>>(rs.set_keys.p, set_cap, kNoCover);
-  rs.cover.ensure(n);
-  k_r_fill64<<<rgrid(n, 65536), kRThreads, 0, st>>>(rs.cover.p, n, kNoCover);
-  MTC_HIP(hipGetLastError());
-  uint32_t* err_p = rs.err.p;
-  uint32_t* region_p = rs.region_off.p;
-  uint64_t* cover_p = rs.cover.p;
-
-  // Per-position tables for the kernels: F-root address, region base, data address,
-  // data chunks; then every position's running count of shifted entries by source
-  // checkpoint (ascending id, :872-883).
-  std::vector<uint64_t> meta_h(4ull * L);
-  for (uint32_t p = 0; p < L; p++) {
-    meta_h[p] = reinterpret_cast<uint64_t>(ch[p].base + ch[p].off_first);
-    meta_h[L + p] = ch[p].region_base;
-    meta_h[2 * L + p] = reinterpret_cast<uint64_t>(ch[p].base + ch[p].off_data);
-    meta_h[3 * L + p] = ch[p].data_chunks;
-  }
-  std::vector<uint32_t> cum_h;
-  std::vector<uint64_t> cum_off(L, 0);
-  for (uint32_t p = 0; p < L; p++) {
-    const uint32_t idx = ref + p, S = ch[p].h.num_shift_dupl;
-    cum_off[p] = cum_h.size();
-    std::vector<uint32_t> cnt(idx - ref + 1, 0);
-    for (uint32_t t = 0; t < ch[p].h.num_prior_chkpts; t++) {
-      const uint32_t c = ptables[p][2 * t], m = ptables[p][2 * t + 1];
-      if (c < ref || c > idx) throw Status{MTC_ERR_CORRUPT_DIFF, "shifted entries name a checkpoint off the chain"};
-      cnt[c - ref] += m;
-    }
-    for (size_t t = 1; t < cnt.size(); t++) cnt[t] += cnt[t - 1];
-    if (cnt.back() != S) throw Status{MTC_ERR_CORRUPT_DIFF, "prior-checkpoint table does not sum to S"};
-    cum_h.insert(cum_h.end(), cnt.begin(), cnt.end());
-  }
-  // meta and cum share one upload from pinned staging
-  const uint64_t meta_bytes = 8 * meta_h.size(), cum_bytes = 4 * cum_h.size();
-  rs.meta.reserve(meta_h.size() + (cum_h.size() + 1) / 2);
-  pinned_reserve(rs.stage, rs.stage_cap, meta_bytes + cum_bytes);
-  MTC_HIP(hipStreamSynchronize(st));  // the staging may still feed the previous restart's copy
-  std::memcpy(rs.stage, meta_h.data(), meta_bytes);
-  std::memcpy(rs.stage + meta_bytes, cum_h.data(), cum_bytes);
-  MTC_HIP(hipMemcpyAsync(rs.meta.p, rs.stage, meta_bytes + cum_bytes, hipMemcpyHostToDevice, st));
-  const uint64_t* meta_p = rs.meta.p;
-  const uint32_t* cum_p = reinterpret_cast<const uint32_t*>(rs.meta.p + meta_h.size());
-
-  // Region offsets and the (position, root) set.
-  for (uint32_t p = 0; p < L; p++) {
-    const ChainDiff& d = ch[p];
-    const uint32_t F = d.h.num_first_ocur;
-    uint32_t* ro = region_p + d.region_base;
-    if (F) {
-      k_r_roots<<<rgrid(F), kRThreads, 0, st>>>(d.base + d.off_first, F, g, ro, p, rs.set_keys.p, rs.set_vals.p,
-                                                set_cap - 1, err_p, idb);
-      MTC_HIP(hipGetLastError());
-    }
-    exclusive_scan_u32(ro, ro, F, ro + F, ws, st);
-  }
-  rs.totals_h.resize(L);
-  // Each position's total sits at region_base + F.  A short region array comes
-  // back in one copy; a long one total by total.
-  const uint64_t region_words = sumF + L;
-  const bool whole = region_words <= (1u << 20);
-  pinned_reserve(rs.totals, rs.totals_cap, 4ull * (whole ? region_words : L));
-  uint32_t* totals = reinterpret_cast<uint32_t*>(rs.totals);
-  if (whole) {
-    MTC_HIP(hipMemcpyAsync(totals, region_p, 4ull * region_words, hipMemcpyDeviceToHost, st));
+    rs.busy = false;
+    hk = hdr[0];
+    if (hk.ref_id <= k) hs.assign(hdr + 1, hdr + 1 + (k - hk.ref_id + 1));
   } else {
+    MTC_HIP(hipMemcpyAsync(&hk, diffs[k], sizeof(hk), hipMemcpyDeviceToHost, st));
+    MTC_HIP(hipStreamSynchronize(st));
+  }
+  check_last(hk, k, out_len);
+  const uint64_t C = hk.chunk_size;
+  const uint32_t n = (uint32_t)((hk.datalen + C - 1) / C), ref = hk.ref_id, L = k - ref + 1;
+  for (uint32_t p = 0; p < L; p++) present(ref + (uint64_t)p);
+  if (hs.empty()) {
+    hs.resize(L);
+    if (!on_device) {
+      for (uint32_t p = 0; p < L; p++) std::memcpy(&hs[p], diffs[ref + (uint64_t)p], sizeof(mtc_header));
+    } else {
+      pinned_reserve(rs.stage, rs.stage_cap, 16ull * L + sizeof(mtc_header) * (L + 1ull));
+      uint64_t* ptrs = reinterpret_cast<uint64_t*>(rs.stage);
+      for (uint32_t p = 0; p < L; p++) ptrs[p] = reinterpret_cast<uint64_t>(diffs[ref + (uint64_t)p]);
+      std::memcpy(ptrs + L, sizes + ref, 8ull * L);
+      mtc_header* hdr = reinterpret_cast<mtc_header*>(ptrs + 2ull * L);
+      rs.busy = true;
+      k_r_headers<<<rgrid(8ull * (L + 1ull), 1024), kRThreads, 0, st>>>(ptrs, ptrs + L, ref, k, reinterpret_cast<uint32_t*>(hdr));
+      MTC_HIP(hipGetLastError());
+      MTC_HIP(hipStreamSynchronize(st));
+      rs.busy = false;
+      hs.assign(hdr + 1, hdr + 1 + L);
+    }
+  }
+  // Chain layout, with host diffs uploaded once: an exact-size upload, freed when the
+  // restart returns (a chain can be as large as the buffer, so it is not kept).
+  std::vector<uint64_t> addr(L);
+  DevBuf<uint8_t> upload;
+  if (on_device) {
+    for (uint32_t p = 0; p < L; p++) addr[p] = reinterpret_cast<uint64_t>(diffs[ref + (uint64_t)p]);
+  } else {
+    uint64_t total = 0;
+    for (uint32_t p = 0; p < L; p++) {
+      addr[p] = total;
+      total += (sizes[ref + (uint64_t)p] + 255) & ~255ull;
+    }
+    upload.ensure(total);
+    for (uint32_t p = 0; p < L; p++) addr[p] += reinterpret_cast<uint64_t>(upload.p);
+  }
+  const uint64_t words = meta_words(L);
+  pinned_reserve(rs.stage, rs.stage_cap, 8 * words + 8);
+  uint64_t* m = reinterpret_cast<uint64_t*>(rs.stage);
+  volatile uint32_t* err_h = reinterpret_cast<volatile uint32_t*>(m + words);
+  const ChainSums t = fill_meta(m, hs.data(), addr.data(), sizes + ref, L, hk, basic);
+  err_h[0] = err_h[1] = 0;
+  if (!on_device) {
     for (uint32_t p = 0; p < L; p++)
-      MTC_HIP(hipMemcpyAsync(totals + p, region_p + ch[p].region_base + ch[p].h.num_first_ocur, sizeof(uint32_t),
-                             hipMemcpyDeviceToHost, st));
+      MTC_HIP(hipMemcpyAsync(reinterpret_cast<void*>(addr[p]), diffs[ref + (uint64_t)p], sizes[ref + (uint64_t)p],
+                             hipMemcpyHostToDevice, st));
+    MTC_HIP(hipEventRecord(rs.ev[1], st));
   }
-  check_err(err_p, st);
-  for (uint32_t p = 0; p < L; p++) {
-    rs.totals_h[p] = whole ? totals[ch[p].region_base + ch[p].h.num_first_ocur] : totals[p];
-    if (rs.totals_h[p] > ch[p].data_chunks) throw Status{MTC_ERR_CORRUPT_DIFF, "data section shorter than its regions"};
-  }
-
-  // Cover chunks, oldest diff first so newer diffs overwrite.
-  for (uint32_t p = 0; p < L; p++) {
-    const ChainDiff& d = ch[p];
-    const uint32_t F = d.h.num_first_ocur, S = d.h.num_shift_dupl;
-    if (F) {
-      k_r_cover_first<<<rgrid(rs.totals_h[p], 65536), kRThreads, 0, st>>>(d.base + d.off_first, F,
-                                                                         region_p + d.region_base, rs.totals_h[p], g, p,
-                                                                         cover_p, idb);
-      MTC_HIP(hipGetLastError());
-    }
-    if (S) {
-      RShiftArgs sa{d.base + d.off_shift, S, cum_p + cum_off[p], p + 1, ref, p, g, rs.set_keys.p, rs.set_vals.p,
-                   set_cap - 1, meta_p, meta_p + L, region_p, cover_p, err_p};
-      k_r_cover_shift<<<rgrid(S), kRThreads, 0, st>>>(sa);
-      MTC_HIP(hipGetLastError());
-    }
-  }
-  const int vec = (C % 16 == 0) && ((uintptr_t)out % 16 == 0);
-  k_r_copy<<<rgrid(n, 8192), kRThreads, 0, st>>>(cover_p, n, (uint32_t)C, hk.datalen, meta_p + 2 * L, meta_p + 3 * L,
-                                                 out, vec, err_p);
-  MTC_HIP(hipGetLastError());
+  const uint64_t cap = set_slots(t.F);
+  rs.err.ensure(1);
+  rs.region.reserve(t.F + L);
+  rs.set_keys.ensure(cap);
+  rs.set_vals.ensure(cap);
+  rs.cover.ensure(n);
+  rs.cum.reserve(t.cum);
+  rs.meta.reserve(words);
+  Chain c{L, n, (uint32_t)C, ref, basic ? n - 1 : 0u, make_geo(n), rs.meta.p, rs.region.p, rs.cum.p, rs.set_keys.p,
+          rs.set_vals.p, cap - 1, rs.cover.p, rs.err.p, err_h};
+  rs.busy = true;
+  launch_restart(c, m, m, t, hk.datalen, out, st,
+                 [&] { exclusive_scan_u32(c.region, c.region, t.F + L, nullptr, rs.ws, st); });
   MTC_HIP(hipEventRecord(rs.ev[2], st));
-  check_err(err_p, st);
-  MTC_HIP(hipEventElapsedTime(&g_restart_ms[0], rs.ev[0], rs.ev[1]));
+  MTC_HIP(hipStreamSynchronize(st));
+  rs.busy = false;
+  throw_err(err_h[0] | err_h[1]);
+  if (!on_device) MTC_HIP(hipEventElapsedTime(&g_restart_ms[0], rs.ev[0], rs.ev[1]));  // else nothing was uploaded
   MTC_HIP(hipEventElapsedTime(&g_restart_ms[1], rs.ev[0], rs.ev[2]));
-  if (on_device) g_restart_ms[0] = 0;  // nothing was uploaded
 }
 
 // ---------------------------------------------------------------------------
@@ -543,57 +729,6 @@ __global__ void k_r_gather_headers(const uint64_t* ptrs, uint32_t L, uint32_t* o
   out[i] = ld32(reinterpret_cast<const uint8_t*>(ptrs[i / 8]) + 4 * (i % 8));
 }
 
-// One block per chain position p: the inclusive running count, by checkpoint id
-// ref..ref+p, of the shifted entries of diff p (its prior-checkpoint table,
-// src/tree_approach.cpp:872-883), checked against the diff's S.
-__global__ __launch_bounds__(kRThreads) void k_r_cum(const uint64_t* table_ptr, const uint64_t* ps,
-                                                     const uint64_t* cum_off, uint32_t ref, uint32_t* cum,
-                                                     uint32_t* err) {
-  __shared__ uint32_t cnt[kNoAllocMaxChain];
-  const uint32_t p = blockIdx.x, t = threadIdx.x;
-  const uint32_t P = (uint32_t)(ps[p] >> 32), S = (uint32_t)ps[p];
-  const uint8_t* tab = reinterpret_cast<const uint8_t*>(table_ptr[p]);
-  cnt[t] = 0;
-  __syncthreads();
-  for (uint32_t i = t; i < P; i += kRThreads) {
-    const uint32_t c = ld32(tab + 8ull * i), m = ld32(tab + 8ull * i + 4);
-    if (c < ref || c > ref + p) atomicOr(err, ERR_CORRUPT);
-    else atomicAdd(&cnt[c - ref], m);
-  }
-  __syncthreads();
-  for (uint32_t o = 1; o < kNoAllocMaxChain; o <<= 1) {  // inclusive scan
-    const uint32_t v = (t >= o) ? cnt[t - o] : 0u;
-    __syncthreads();
-    cnt[t] += v;
-    __syncthreads();
-  }
-  if (t <= p) cum[cum_off[p] + t] = cnt[t];
-  if (t == p && cnt[t] != S) atomicOr(err, ERR_CORRUPT);
-}
-
-// k_r_cover_first with the region total read on the device (region_off[F]) and
-// checked against the data section's capacity.
-__global__ void k_r_cover_first_dev(const uint8_t* first, uint32_t F, const uint32_t* region_off,
-                                    uint64_t data_chunks, Geo g, uint32_t pos, uint64_t* cover, uint32_t* err) {
-  const uint64_t total = region_off[F];
-  if (total > data_chunks) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, ERR_CORRUPT);
-    return;
-  }
-  for (uint64_t j = (uint64_t)blockIdx.x * kRThreads + threadIdx.x; j < total; j += (uint64_t)gridDim.x * kRThreads) {
-    uint32_t lo = 0, hi = F;
-    while (hi - lo > 1) {
-      const uint32_t mid = (lo + hi) >> 1;
-      if (region_off[mid] <= j) lo = mid;
-      else hi = mid;
-    }
-    uint32_t st[2], ct[2];
-    const int r = leaf_runs(g, ld32(first + 4ull * lo), st, ct);
-    const uint32_t chunk = run_at(r, st, ct, (uint32_t)(j - region_off[lo]));
-    cover[chunk] = ((uint64_t)pos << kSlotBits) | j;
-  }
-}
-
 // Bump carving of the scratch array (256-byte aligned pieces).
 struct Carve {
   uint64_t off = 0;
@@ -624,22 +759,19 @@ void restart_noalloc_impl(const void* const* diffs, const uint64_t* sizes, uint3
   mtc_header hk;
   MTC_HIP(hipMemcpyAsync(&hk, diffs[k], sizeof(hk), hipMemcpyDeviceToHost, st));
   MTC_HIP(hipStreamSynchronize(st));
-  if (hk.chkpt_id != k || hk.ref_id > k || hk.chunk_size == 0 || hk.datalen == 0)
-    throw Status{MTC_ERR_CORRUPT_DIFF, "bad header of the requested diff"};
-  if (out_len < hk.datalen) throw Status{MTC_ERR_BUFFER_TOO_SMALL, "output shorter than datalen"};
+  check_last(hk, k, out_len);
   const uint64_t C = hk.chunk_size;
-  const uint64_t n64 = (hk.datalen + C - 1) / C;
-  if (n64 > (1ull << 31)) throw Status{MTC_ERR_CORRUPT_DIFF, "too many chunks"};
-  const uint32_t n = (uint32_t)n64, ref = hk.ref_id, L = k - ref + 1;
+  const uint32_t n = (uint32_t)((hk.datalen + C - 1) / C), ref = hk.ref_id, L = k - ref + 1;
   if (L > kNoAllocMaxChain)
     throw Status{MTC_ERR_INVALID_ARG, "the no-allocation restart takes chains of at most 256 diffs"};
-  const Geo g = make_geo(n);
 
-  // Headers of the chain: one gather kernel, one copy.
+  // Headers of the chain: one gather kernel, one copy.  The tables come to lie where
+  // the addresses and headers were.
   Carve cv;
   uint32_t* err_p = reinterpret_cast<uint32_t*>(base + cv.take(4));
-  uint64_t* ptrs_d = reinterpret_cast<uint64_t*>(base + cv.take(8ull * L));
-  uint32_t* hdr_d = reinterpret_cast<uint32_t*>(base + cv.take(32ull * L));
+  uint8_t* const lead = base + cv.take(std::max<uint64_t>(8ull * L + 32ull * L, 8 * meta_words(L)));
+  uint64_t* ptrs_d = reinterpret_cast<uint64_t*>(lead);
+  uint32_t* hdr_d = reinterpret_cast<uint32_t*>(lead + 8ull * L);
   uint64_t ptrs_h[kNoAllocMaxChain];
   for (uint32_t p = 0; p < L; p++) {
     const uint32_t idx = ref + p;
@@ -654,90 +786,40 @@ void restart_noalloc_impl(const void* const* diffs, const uint64_t* sizes, uint3
   MTC_HIP(hipStreamSynchronize(st));
 
   // Chain layout (the same checks as the allocating restart).
-  uint64_t off_first[kNoAllocMaxChain], off_shift[kNoAllocMaxChain], off_table[kNoAllocMaxChain];
-  uint64_t meta_h[7 * kNoAllocMaxChain];  // F-root, region base, data, data chunks, table, (P, S), cum offset
-  uint64_t sumF = 0, cum_words = 0;
+  uint64_t meta_h[meta_words(kNoAllocMaxChain)];
+  const ChainSums t = fill_meta(meta_h, hs, ptrs_h, sizes + ref, L, hk, false);
   uint32_t maxF = 0;
   for (uint32_t p = 0; p < L; p++) {
-    const uint32_t idx = ref + p;
-    const mtc_header& h = hs[p];
-    if (h.chkpt_id != idx || h.ref_id != ref || h.datalen != hk.datalen || h.chunk_size != hk.chunk_size)
-      throw Status{MTC_ERR_CORRUPT_DIFF, "diff " + std::to_string(idx) + " does not belong to the chain"};
-    off_first[p] = 32;
-    off_table[p] = off_first[p] + 4ull * h.num_first_ocur;
-    off_shift[p] = off_table[p] + 8ull * h.num_prior_chkpts;
-    const uint64_t off_data = off_shift[p] + 8ull * h.num_shift_dupl;
-    if (off_data > sizes[idx]) throw Status{MTC_ERR_CORRUPT_DIFF, "diff shorter than its metadata"};
-    if (h.num_prior_chkpts > p + 1) throw Status{MTC_ERR_CORRUPT_DIFF, "prior-checkpoint table longer than the chain"};
-    const uint8_t* b = static_cast<const uint8_t*>(diffs[idx]);
-    meta_h[p] = reinterpret_cast<uint64_t>(b + off_first[p]);
-    meta_h[L + p] = sumF + p;
-    meta_h[2 * L + p] = reinterpret_cast<uint64_t>(b + off_data);
-    meta_h[3 * L + p] = (sizes[idx] - off_data) / C;
-    meta_h[4 * L + p] = reinterpret_cast<uint64_t>(b + off_table[p]);
-    meta_h[5 * L + p] = ((uint64_t)h.num_prior_chkpts << 32) | h.num_shift_dupl;
-    meta_h[6 * L + p] = cum_words;
-    cum_words += p + 1;
-    sumF += h.num_first_ocur;
-    maxF = std::max(maxF, h.num_first_ocur);
+    if (hs[p].num_prior_chkpts > p + 1) throw Status{MTC_ERR_CORRUPT_DIFF, "prior-checkpoint table longer than the chain"};
+    maxF = std::max(maxF, hs[p].num_first_ocur);
   }
-  uint64_t set_cap = 16;
-  while (set_cap < 2 * sumF) set_cap <<= 1;
+  const uint64_t cap = set_slots(t.F);
   uint64_t* cover_p = reinterpret_cast<uint64_t*>(base + cv.take(8ull * n));
-  uint64_t* keys_p = reinterpret_cast<uint64_t*>(base + cv.take(8 * set_cap));
-  uint32_t* vals_p = reinterpret_cast<uint32_t*>(base + cv.take(4 * set_cap));
-  const uint64_t off_region = cv.take(4 * (sumF + L));
-  const uint64_t off_meta = cv.take(8ull * 7 * L);
-  const uint64_t off_cum = cv.take(4 * cum_words);
+  uint64_t* keys_p = reinterpret_cast<uint64_t*>(base + cv.take(8 * cap));
+  uint32_t* vals_p = reinterpret_cast<uint32_t*>(base + cv.take(4 * cap));
+  const uint64_t off_region = cv.take(4 * (t.F + L));
+  const uint64_t off_cum = cv.take(4 * t.cum);
   uint64_t off_sums[3];
   for (int d = 0; d < 3; d++) off_sums[d] = cv.take(4 * scan_sums_words(maxF, d));
   if (cv.off > kNoAllocScratch)
     throw Status{MTC_ERR_INVALID_ARG, "this restart needs " + std::to_string(cv.off) +
                                           " bytes of scratch; the no-allocation restart has 64 MiB per GPU"};
   uint32_t* region_p = reinterpret_cast<uint32_t*>(base + off_region);
-  uint64_t* meta_p = reinterpret_cast<uint64_t*>(base + off_meta);
-  uint32_t* cum_p = reinterpret_cast<uint32_t*>(base + off_cum);
+  uint64_t* meta_p = reinterpret_cast<uint64_t*>(lead);
   uint32_t* const sums[3] = {reinterpret_cast<uint32_t*>(base + off_sums[0]),
                              reinterpret_cast<uint32_t*>(base + off_sums[1]),
                              reinterpret_cast<uint32_t*>(base + off_sums[2])};
-  MTC_HIP(hipMemcpyAsync(meta_p, meta_h, 8ull * 7 * L, hipMemcpyHostToDevice, st));
-  // The array keeps the previous call's contents: everything read before it is
-  // written starts from a fill.
-  k_r_fill32<<<1, kRThreads, 0, st>>>(err_p, 1, 0);
-  k_r_fill64<<<rgrid(set_cap, 65536), kRThreads, 0, st>>>(keys_p, set_cap, kNoCover);
-  k_r_fill64<<<rgrid(n, 65536), kRThreads, 0, st>>>(cover_p, n, kNoCover);
-  k_r_cum<<<L, kRThreads, 0, st>>>(meta_p + 4 * L, meta_p + 5 * L, meta_p + 6 * L, ref, cum_p, err_p);
-  MTC_HIP(hipGetLastError());
-  for (uint32_t p = 0; p < L; p++) {
-    const uint32_t F = hs[p].num_first_ocur;
-    const uint8_t* b = static_cast<const uint8_t*>(diffs[ref + p]);
-    uint32_t* ro = region_p + meta_h[L + p];
-    if (F) {
-      k_r_roots<<<rgrid(F), kRThreads, 0, st>>>(b + off_first[p], F, g, ro, p, keys_p, vals_p, set_cap - 1, err_p, 0);
-      MTC_HIP(hipGetLastError());
+  MTC_HIP(hipMemcpyAsync(meta_p, meta_h, 8 * meta_words(L), hipMemcpyHostToDevice, st));
+  Chain c{L, n, (uint32_t)C, ref, 0u, make_geo(n), meta_p, region_p, reinterpret_cast<uint32_t*>(base + off_cum), keys_p,
+          vals_p, cap - 1, cover_p, err_p, nullptr};
+  // Region offsets diff by diff: the scan's scratch is sized for the largest one.
+  launch_restart(c, nullptr, meta_h, t, hk.datalen, out, st, [&] {
+    const uint64_t* region = meta_h + (uint64_t)M_REGION * L;
+    for (uint32_t p = 0; p < L; p++) {
+      uint32_t* ro = region_p + region[p];
+      exclusive_scan_u32_fixed(ro, ro, hs[p].num_first_ocur, ro + hs[p].num_first_ocur, sums, st);
     }
-    exclusive_scan_u32_fixed(ro, ro, F, ro + F, sums, st);
-  }
-  check_err(err_p, st);  // every root lies inside the tree before any cover is written
-  for (uint32_t p = 0; p < L; p++) {
-    const uint32_t F = hs[p].num_first_ocur, S = hs[p].num_shift_dupl;
-    const uint8_t* b = static_cast<const uint8_t*>(diffs[ref + p]);
-    if (F) {
-      k_r_cover_first_dev<<<rgrid(std::max<uint64_t>(meta_h[3 * L + p], 1), 65536), kRThreads, 0, st>>>(
-          b + off_first[p], F, region_p + meta_h[L + p], meta_h[3 * L + p], g, p, cover_p, err_p);
-      MTC_HIP(hipGetLastError());
-    }
-    if (S) {
-      RShiftArgs sa{b + off_shift[p], S, cum_p + meta_h[6 * L + p], p + 1, ref, p, g, keys_p, vals_p, set_cap - 1,
-                   meta_p, meta_p + L, region_p, cover_p, err_p};
-      k_r_cover_shift<<<rgrid(S), kRThreads, 0, st>>>(sa);
-      MTC_HIP(hipGetLastError());
-    }
-  }
-  const int vec = (C % 16 == 0) && ((uintptr_t)out % 16 == 0);
-  k_r_copy<<<rgrid(n, 8192), kRThreads, 0, st>>>(cover_p, n, (uint32_t)C, hk.datalen, meta_p + 2 * L, meta_p + 3 * L,
-                                                 out, vec, err_p);
-  MTC_HIP(hipGetLastError());
+  });
   check_err(err_p, st);
 }
 

@@ -126,3 +126,80 @@ def test_handle_alternates_between_alone_and_a_large_batch():
     for d in ds:
         d.close()
     batch.close()
+
+
+@pytest.mark.parametrize("C,n,tail", [(1, 700, 0), (7, 1000, 3), (16, 513, 0), (48, 300, 47), (100, 2000, 1),
+                                      (128, 4096, 0), (128, 1000, 5), (1000, 129, 999), (4096, 33, 17)])
+def test_restart_copies(C, n, tail):
+    """Restarts of every checkpoint from device and host chains: chunk sizes that are
+    powers of two and not, short last chunks, outputs at any alignment, diffs that lie
+    at odd addresses, and shifted entries from one leaf to the whole buffer."""
+    size = n * C + tail
+    rng = np.random.default_rng(7 * C + n)
+    v0 = rng.integers(0, 256, size, dtype=np.uint8)
+    v1 = v0.copy()
+    half = n // 2 * C
+    v1[half:2 * half] = v0[:half]                      # large shifted entries
+    v2 = v1.copy()
+    for first in rng.integers(0, n, 6):
+        v2[first * C:(first + 2) * C] = rng.integers(0, 256, v2[first * C:(first + 2) * C].size, dtype=np.uint8)
+    versions = [v0, v1, v2, v0, v2[::-1].copy(), v1]   # v0 again: every leaf shifted
+    diffs = same_as_oracle(versions, C)
+    dev = [torch.frombuffer(bytearray(d), dtype=torch.uint8).to("cuda:0") for d in diffs]
+    odd = []
+    for i, d in enumerate(diffs):
+        t = torch.zeros(len(d) + 8, dtype=torch.uint8, device="cuda:0")
+        t[i % 5:i % 5 + len(d)] = dev[i]
+        odd.append(t[i % 5:i % 5 + len(d)])
+    for off in (0, 4, 1):
+        for chain in (dev, odd, diffs):
+            for k in range(len(versions)):
+                print(f"restart C={C} n={n} tail={tail} off={off} k={k}", flush=True)
+                buf = torch.full((size + 32,), 0xA5, dtype=torch.uint8, device="cuda:0")
+                M.restart_into(buf[off:off + size], chain, k)
+                got = buf.cpu().numpy()
+                assert np.array_equal(got[off:off + size], versions[k])
+                assert (got[:off] == 0xA5).all() and (got[off + size:] == 0xA5).all()
+
+
+def test_restart_of_a_late_chain():
+    """A device chain that starts after checkpoint 4096: its headers are read from the
+    chain's first diff on; what lies below it is not needed."""
+    d, size = M.TreeDeduplicator(16), 16 * 50 + 3
+    rng = np.random.default_rng(5)
+    host = rng.integers(0, 256, size, dtype=np.uint8)
+    buf = torch.from_numpy(host).to("cuda:0")
+    chain = []
+    for k in range(4099):
+        d.checkpoint_device(buf, make_baseline=(k == 4094))
+        chain.append(d.copy_last_diff_device() if k >= 4094 else None)
+        if k >= 4094:
+            buf[(k % 50) * 16:(k % 50) * 16 + 5] = k % 251
+    d.close()
+    want = torch.from_numpy(host).to("cuda:0")
+    for k in range(4094, 4099):
+        out = torch.zeros(size, dtype=torch.uint8, device="cuda:0")
+        M.restart_into(out, chain, k)
+        assert torch.equal(out, want), k
+        want[(k % 50) * 16:(k % 50) * 16 + 5] = k % 251
+
+
+def test_restart_refuses_short_data_and_leaves_the_output():
+    """A diff whose data section is cut to fewer chunks than its regions (to some, to
+    none) is refused before anything is written."""
+    C, n = 64, 40
+    rng = np.random.default_rng(9)
+    v0 = rng.integers(0, 256, n * C, dtype=np.uint8)
+    v1 = v0.copy()
+    v1[5 * C:9 * C] = rng.integers(0, 256, 4 * C, dtype=np.uint8)
+    diffs = same_as_oracle([v0, v1], C)
+    for cut0, cut1 in ((0, 1), (0, 4), (1, 0)):
+        chain = [torch.frombuffer(bytearray(d[:len(d) - cut * C]), dtype=torch.uint8).to("cuda:0")
+                 for d, cut in zip(diffs, (cut0, cut1))]
+        out = torch.full((n * C,), 7, dtype=torch.uint8, device="cuda:0")
+        with pytest.raises(M.MtcError) as e:
+            M.restart_into(out, chain, 1)
+        assert e.value.code == 5
+        assert bool((out == 7).all())
+    M.restart_into(out, [torch.frombuffer(bytearray(d), dtype=torch.uint8).to("cuda:0") for d in diffs], 1)
+    assert np.array_equal(out.cpu().numpy(), v1)
