@@ -203,3 +203,17 @@ def test_restart_refuses_short_data_and_leaves_the_output():
         assert bool((out == 7).all())
     M.restart_into(out, [torch.frombuffer(bytearray(d), dtype=torch.uint8).to("cuda:0") for d in diffs], 1)
     assert np.array_equal(out.cpu().numpy(), v1)
+
+
+@pytest.mark.parametrize("hk", [M.MURMUR3, M.MD5])
+@pytest.mark.parametrize("C", [16, 32, 64, 128, 256, 2048, 4096])
+def test_hash_chunks_blocks(C, hk):
+    """mtc_hash_chunks at one wavefront of chunks, one more, less, and short tails."""
+    rng = np.random.default_rng(C + hk)
+    for n, tail in ((1, 0), (63, 5), (64, 0), (64, 15), (65, C - 1), (300, 1)):
+        a = rng.integers(0, 256, n * C + tail, dtype=np.uint8)
+        print(f"hash_chunks C={C} hk={hk} n={n} tail={tail}", flush=True)
+        got = M.hash_chunks(torch.from_numpy(a).to("cuda:0"), C, hk).cpu().numpy().reshape(-1, 16)
+        assert len(got) == n + (tail > 0)
+        for c in range(len(got)):
+            assert got[c].tobytes() == O.hash_bytes(hk, a[c * C:(c + 1) * C]), c
