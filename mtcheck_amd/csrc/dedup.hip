@@ -367,27 +367,168 @@ __device__ __forceinline__ Digest staged_hash(const uint8_t* data, uint64_t firs
 // the serial loop of include/reference_impl.hpp:44-71).  One lane per chunk.
 // ---------------------------------------------------------------------------
 
+// Chunk sizes and alignments without a kernel of their own: a wavefront stages its 64
+// chunks in LDS, the next pass on its way meanwhile, and each lane cuts its chunk's
+// words out of the aligned 16-byte columns.  A pass takes 128 bytes of each chunk, as
+// the nine columns that hold them (rows of 144 bytes: sixteen rows' accesses fall on
+// distinct banks); chunks of fewer than kAnyPacked bytes are staged as one piece.
+// Hashing bounds it, with cutting a fourth of the instructions.  Microseconds of 4 GiB,
+// one thread a chunk byte by byte -> now:
+//   Murmur3  100 B 1851 -> 960    333 B 6991 -> 1037   1000 B 5463 -> 1055   5000 B 4690 -> 1171
+//   MD5      100 B 4474 -> 1324   333 B 2552 -> 1208   1000 B 3199 -> 1076   5000 B 1362 -> 1154
+// The leaf kernel of 200 MB in 1000-byte chunks: 144 -> 80.
+constexpr uint32_t kAnySeg = 128, kAnyCols = kAnySeg / 16 + 1, kAnyPacked = 112;
+
+// Bytes sh .. sh + 15 of the 32 bytes {a, b} (0 <= sh < 16).
+__device__ __forceinline__ uint4 cut16(const uint4& a, const uint4& b, uint32_t sh) {
+  // (a select between two fields of one vector would go through memory)
+  const uint32_t two = (sh & 8) ? ~0u : 0u;
+  const bool one = sh & 4;
+  auto pick = [two](uint32_t hi, uint32_t lo) { return (hi & two) | (lo & ~two); };
+  const uint32_t w0 = pick(a.z, a.x), w1 = pick(a.w, a.y), w2 = pick(b.x, a.z), w3 = pick(b.y, a.w), w4 = pick(b.z, b.x),
+                 w5 = pick(b.w, b.y);
+  const uint32_t v0 = one ? w1 : w0, v1 = one ? w2 : w1, v2 = one ? w3 : w2, v3 = one ? w4 : w3, v4 = one ? w5 : w4;
+  return uint4{__builtin_amdgcn_alignbyte(v1, v0, sh & 3), __builtin_amdgcn_alignbyte(v2, v1, sh & 3),
+               __builtin_amdgcn_alignbyte(v3, v2, sh & 3), __builtin_amdgcn_alignbyte(v4, v3, sh & 3)};
+}
+
+// The first `keep` bytes of v (all of them from 16 on), the rest zero.
+__device__ __forceinline__ uint4 keep_bytes(uint4 v, int keep) {
+  auto word = [](uint32_t w, int k) { return k >= 4 ? w : k <= 0 ? 0u : w & ((1u << (8 * k)) - 1); };
+  return uint4{word(v.x, keep), word(v.y, keep - 4), word(v.z, keep - 8), word(v.w, keep - 12)};
+}
+
+// Digest of chunk first + lane; lds: this wavefront's 64 * 16 * kAnyCols bytes.
+template <int HK>
+__device__ __forceinline__ Digest any_digest(const uint8_t* data, uint64_t len, uint32_t n, uint32_t C, uint64_t first,
+                                             uint8_t* lds) {
+  const uint32_t t = lane_id();
+  const uint64_t c = first + t;
+  const uintptr_t lo = (uintptr_t)data, base = lo + first * C;
+  // All 64 chunks whole, and the columns that hold them inside the buffer (every
+  // wavefront but the first, if the buffer is not aligned, and the last).
+  const bool inside = (base & ~(uintptr_t)15) >= lo && (first + 64) * C + 16 <= len;
+  if (!inside) return c < n ? hash_bytes<HK>(data + c * C, min<uint64_t>(C, len - c * C)) : Digest{0, 0};
+  const bool packed = C < kAnyPacked;
+  const uint32_t off = packed ? ((uint32_t)base & 15) + t * C : t * (16 * kAnyCols) + ((uint32_t)(base + (uint64_t)t * C) & 15);
+  const uint32_t sh = off & 15;  // the same in every pass
+  const bool cut = (C & 15) != 0 || (base & 15) != 0;  // some lane's words are not columns
+  const uint8_t* mine = lds + (off & ~15u);
+  uint64_t h1 = 0, h2 = 0;
+  uint32_t st[4], X[16];
+  md5_init(st);
+#pragma unroll
+  for (int k = 0; k < 16; k++) X[k] = 0;
+  uint4 v[kAnyCols];
+  const uint32_t units = packed ? (((uint32_t)base & 15) + 64 * C + 15) / 16 : 64 * kAnyCols;
+  auto load = [&](uint32_t at) {  // the columns of bytes at .. at + kAnySeg - 1 of each chunk
+#pragma unroll
+    for (uint32_t i = 0; i < kAnyCols; i++) {
+      const uint32_t u = i * 64 + t, r = u / kAnyCols, col = u % kAnyCols;
+      v[i] = uint4{0, 0, 0, 0};
+      if (packed) {
+        if (u < units) v[i] = *reinterpret_cast<const uint4*>((base & ~(uintptr_t)15) + 16 * u);
+      } else {
+        const uint32_t end = min(C - at, kAnySeg);
+        const uintptr_t a0 = base + at + (uint64_t)r * C;
+        if (16 * col < ((uint32_t)a0 & 15) + end) v[i] = *reinterpret_cast<const uint4*>((a0 & ~(uintptr_t)15) + 16 * col);
+      }
+    }
+  };
+  load(0);
+#pragma unroll 1
+  for (uint32_t at = 0; at < C; at += kAnySeg) {
+    // The LDS accesses of one wavefront execute in order.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (uint32_t i = 0; i < kAnyCols; i++)
+      if (64 * i < units) *reinterpret_cast<uint4*>(lds + 16 * (i * 64 + t)) = v[i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (C - at > kAnySeg) load(at + kAnySeg);
+    const uint32_t left = min(C - at, kAnySeg);
+    uint4 col = *reinterpret_cast<const uint4*>(mine);
+    auto next16 = [&](uint32_t q) {  // bytes 16 q .. 16 q + 15 of this pass
+      const uint4 was = col;
+      col = *reinterpret_cast<const uint4*>(mine + 16 * q + 16);
+      uint4 x = was;
+      if (cut) x = cut16(was, col, sh);
+      return x;
+    };
+    if constexpr (HK == HASH_MD5) {
+#pragma unroll 1
+      for (uint32_t b = 0; b < left; b += 64) {  // a partial block stays in X
+#pragma unroll
+        for (uint32_t q = 0; q < 4; q++) {
+          uint4 x = next16(b / 16 + q);
+          if (left - b < 64) x = keep_bytes(x, (int)(left - b) - 16 * (int)q);
+          X[4 * q] = x.x;
+          X[4 * q + 1] = x.y;
+          X[4 * q + 2] = x.z;
+          X[4 * q + 3] = x.w;
+        }
+        if (left - b >= 64) md5_compress(st, X);
+      }
+    } else {
+#pragma unroll
+      for (uint32_t q = 0; q < kAnySeg / 16; q++) {
+        if (16 * q >= left) continue;
+        const uint4 x = next16(q);
+        if (16 * q + 16 <= left) {
+          m3_block(h1, h2, (uint64_t)x.x | ((uint64_t)x.y << 32), (uint64_t)x.z | ((uint64_t)x.w << 32));
+        } else {
+          const uint32_t rem = left - 16 * q;
+          const uint4 y = keep_bytes(x, (int)rem);
+          m3_tail(h1, h2, (uint64_t)y.x | ((uint64_t)y.y << 32), (uint64_t)y.z | ((uint64_t)y.w << 32), rem);
+        }
+      }
+    }
+  }
+  if constexpr (HK == HASH_MD5) {
+    const uint32_t rem = C % 64;
+    if (rem == 0) {
+#pragma unroll
+      for (int k = 0; k < 16; k++) X[k] = 0;
+    }
+#pragma unroll
+    for (int k = 0; k < 16; k++)  // the end marker, by a static index
+      if (rem / 4 == (uint32_t)k) X[k] |= 0x80u << (8 * (rem & 3));
+    if (rem >= 56) {
+      md5_compress(st, X);
+#pragma unroll
+      for (int k = 0; k < 16; k++) X[k] = 0;
+    }
+    X[14] = C << 3;
+    X[15] = C >> 29;
+    md5_compress(st, X);
+    return md5_digest(st);
+  } else {
+    return m3_final(h1, h2, C);
+  }
+}
+
 // Digest of chunk tile*256 + threadIdx.x (zero beyond n).  CB > 0 selects the
-// LDS-staged path for 16-byte-aligned data and chunk sizes that are multiples of
-// 16; a short last chunk and CB == 0 use byte-granular hashing.
+// LDS-staged path for 16-byte-aligned data and power-of-two chunk sizes (a short last
+// chunk is hashed byte by byte); CB == 0 takes any size and alignment, CB == -1 too,
+// one thread a chunk and byte by byte (see leaf_cb).
 template <int HK, int CB>
 __device__ __forceinline__ Digest tile_digest(const uint8_t* data, uint64_t len, uint32_t n, uint32_t C,
                                               uint64_t tile) {
-  const uint64_t first = tile * kThreads;
-  const uint64_t c = first + threadIdx.x;
-  Digest d{0, 0};
   if constexpr (CB > 0) {
+    const uint64_t first = tile * kThreads;
+    const uint64_t c = first + threadIdx.x;
     __shared__ __align__(16) uint8_t lds[TileShape<CB>::LDS];
     const uint64_t full = len / CB;
-    d = staged_hash<HK, CB>(data, first, full, lds);
+    Digest d = staged_hash<HK, CB>(data, first, full, lds);
     if (c < n && c >= full) d = hash_bytes<HK>(data + c * CB, len - c * CB);
+    return d;
+  } else if constexpr (CB < 0) {
+    const uint64_t c = tile * kThreads + threadIdx.x;
+    return c < n ? hash_bytes<HK>(data + c * C, min<uint64_t>(C, len - c * C)) : Digest{0, 0};
   } else {
-    if (c < n) {
-      const uint64_t off = c * C;
-      d = hash_bytes<HK>(data + off, (off + C <= len) ? C : len - off);
-    }
+    __shared__ __align__(16) uint8_t lds[kThreads * 16 * kAnyCols];
+    const uint32_t w = threadIdx.x / 64;
+    return any_digest<HK>(data, len, n, C, tile * kThreads + 64 * w, lds + w * (64 * 16 * kAnyCols));
   }
-  return d;
 }
 
 // Fixed test, label and packing of one tile's chunks (chunk t*256 + threadIdx.x
@@ -436,7 +577,7 @@ __device__ __forceinline__ void leaf_epilogue(const LeafArgs& a, uint64_t t, con
 // current one is hashed out of LDS.  Chunks to insert are packed into the block's
 // region of the list; the table work runs densely afterwards.
 template <int HK, int CB>
-__global__ __launch_bounds__(kThreads) void k_leaf(Launch<LeafArgs> L) {
+__global__ __launch_bounds__(kThreads, CB ? 1 : 3) void k_leaf(Launch<LeafArgs> L) {
   __shared__ uint32_t s_wcnt[kThreads / 64];
   const Where wh = where(L);
   const LeafArgs a = L.args[wh.m].global();
@@ -446,10 +587,10 @@ __global__ __launch_bounds__(kThreads) void k_leaf(Launch<LeafArgs> L) {
   const uint64_t t1 = std::min<uint64_t>(t0 + a.tiles_per_block, ntiles);
   uint32_t* region = a.list + t0 * kThreads;
   uint32_t run = 0;
-  if constexpr (CB == 0) {
+  if constexpr (CB <= 0) {
     for (uint64_t t = t0; t < t1; t++) {
       const Digest pv = leaf_prev(a, t);
-      leaf_epilogue(a, t, tile_digest<HK, 0>(a.data, a.len, a.n, a.C, t), pv, region, run, s_wcnt);
+      leaf_epilogue(a, t, tile_digest<HK, CB>(a.data, a.len, a.n, a.C, t), pv, region, run, s_wcnt);
     }
   } else {
     using S = TileShape<CB>;
@@ -991,9 +1132,14 @@ __global__ __launch_bounds__(kThreads) void k_resolve(Launch<DenseArgs> L) {
 //   4 GiB        922 / 820   809 / 739   857 / 752   (HBM)
 //   64 MiB        27 / 24     25 / 23     56 / 42    (latency of a chunk's passes)
 template <int HK, int CB>
-__global__ __launch_bounds__(CB > 16 ? 64 : (int)kThreads, 5) void k_hash_chunks(const uint8_t* data, uint64_t len, uint32_t n,
+__global__ __launch_bounds__(CB < 0 || CB == 16 ? (int)kThreads : 64, CB < 0 ? 1 : CB ? 5 : 4) void k_hash_chunks(const uint8_t* data, uint64_t len, uint32_t n,
                                                                                 uint32_t C, Digest* out) {
-  if constexpr (CB <= 16) {
+  if constexpr (CB == 0) {
+    __shared__ __align__(16) uint8_t lds[64 * 16 * kAnyCols];
+    const uint64_t first = (uint64_t)blockIdx.x * 64, c = first + threadIdx.x;
+    const Digest d = any_digest<HK>(data, len, n, C, first, lds);
+    if (c < n) out[c] = d;
+  } else if constexpr (CB < 0 || CB == 16) {
     const uint64_t c = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
     const Digest d = tile_digest<HK, CB>(data, len, n, C, blockIdx.x);
     if (c < n) out[c] = d;
@@ -2241,16 +2387,31 @@ static uint64_t next_pow2(uint64_t x) {
   return p;
 }
 
+// The kernel that hashes chunks of C bytes: one for the size (16-byte aligned data), 0
+// for any other, or -1: byte by byte, which is still the better way for chunks under 20
+// bytes, for Murmur3 chunks under 50 with at most four beyond whole 16-byte blocks (their reads hit the
+// cache, and little is left of the wide columns' gain) and for MD5 of few chunks (each
+// thread's chain of steps decides).  Microseconds staged / byte by byte:
+//   Murmur3, 4 GiB:  20 B 2346 / 1855   33 B 1469 / 1296   48 B 1146 / 1037
+//                    28 B 1672 / 2477   40 B 1264 / 1792   50 B 1140 / 1395
+//   64 MiB, 7 B:     Murmur3 102 / 74   MD5 189 / 135
+//   MD5, 64 MiB:     1500 B (44.7 thousand chunks) 48 / 41   5000 B (13.4 thousand) 115 / 84
+//                    1000 B (67.1 thousand) 45 / 47          333 B 42 / 49
+static int leaf_cb(int hk, uint32_t C, uint64_t n, const void* data) {
+  if ((uintptr_t)data % 16 == 0 && C >= 16 && C <= 4096 && (C & (C - 1)) == 0) return (int)C;
+  return C < 20 || (hk == HASH_MD5 ? n < 65536 : C < 50 && C % 16 <= 4) ? -1 : 0;
+}
+
 template <int HK, int CB>
 static void launch_hash_cb(const uint8_t* data, uint64_t len, uint32_t n, uint32_t C, Digest* out, hipStream_t st) {
-  constexpr uint32_t per = CB > 16 ? 64 : kThreads;
+  constexpr uint32_t per = CB < 0 || CB == 16 ? kThreads : 64;
   k_hash_chunks<HK, CB><<<(uint32_t)(((uint64_t)n + per - 1) / per), per, 0, st>>>(data, len, n, C, out);
 }
 
 template <int HK>
-static void launch_hash_chunks(const uint8_t* data, uint64_t len, uint32_t n, uint32_t C, Digest* out, bool fast,
-                               hipStream_t st) {
-  switch (fast ? C : 0) {
+static void launch_hash_chunks(const uint8_t* data, uint64_t len, uint32_t n, uint32_t C, Digest* out, hipStream_t st) {
+  switch (leaf_cb(HK, C, n, data)) {
+    case -1: launch_hash_cb<HK, -1>(data, len, n, C, out, st); break;
     case 16: launch_hash_cb<HK, 16>(data, len, n, C, out, st); break;
     case 32: launch_hash_cb<HK, 32>(data, len, n, C, out, st); break;
     case 64: launch_hash_cb<HK, 64>(data, len, n, C, out, st); break;
@@ -2266,19 +2427,9 @@ static void launch_hash_chunks(const uint8_t* data, uint64_t len, uint32_t n, ui
 
 void hash_chunks(const uint8_t* data, uint64_t len, uint32_t C, int hk, Digest* out, hipStream_t st) {
   const uint32_t n = (uint32_t)((len + C - 1) / C);
-  const bool fast = (C % 16 == 0) && ((uintptr_t)data % 16 == 0);
-  if (hk == HASH_MD5) launch_hash_chunks<HASH_MD5>(data, len, n, C, out, fast, st);
-  else launch_hash_chunks<HASH_MURMUR3>(data, len, n, C, out, fast, st);
+  if (hk == HASH_MD5) launch_hash_chunks<HASH_MD5>(data, len, n, C, out, st);
+  else launch_hash_chunks<HASH_MURMUR3>(data, len, n, C, out, st);
   MTC_HIP(hipGetLastError());
-}
-
-// Chunk sizes with an LDS-staged leaf kernel; other sizes hash byte by byte.
-static int staged_cb(uint32_t C, bool aligned) {
-  if (!aligned) return 0;
-  switch (C) {
-    case 16: case 32: case 64: case 128: case 256: case 512: case 1024: case 2048: case 4096: return (int)C;
-    default: return 0;
-  }
 }
 
 template <int HK, int CB>
@@ -2298,6 +2449,7 @@ static void launch_leaf(int cb, Launch<LeafArgs> L, uint32_t grid, hipStream_t s
     case 1024: launch_leaf_cb<HK, 1024>(L, grid, st); break;
     case 2048: launch_leaf_cb<HK, 2048>(L, grid, st); break;
     case 4096: launch_leaf_cb<HK, 4096>(L, grid, st); break;
+    case -1: launch_leaf_cb<HK, -1>(L, grid, st); break;
     default: launch_leaf_cb<HK, 0>(L, grid, st); break;
   }
 }
@@ -2754,7 +2906,7 @@ static void prepare_member(Member& M, hipStream_t st) {
   M.n = h->n;
   M.cur = h->current_id;
   M.g = make_geo(M.n);
-  M.cb = staged_cb(h->chunk_size, (uintptr_t)M.data % 16 == 0);
+  M.cb = leaf_cb(h->hash_kind, h->chunk_size, M.n, M.data);
   // With asynchronous copies, checkpoints alternate diff arenas; this step waits
   // (on the device) for the copy still reading the arena it is about to write.
   // The pending flag is cleared once the step has completed.
@@ -3237,7 +3389,7 @@ static void build_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img, int ph
         direct->la = la[0];
         continue;
       }
-      const uint32_t tag = 100 + (uint32_t)hk * 32 + (lean ? 16u : 0u) + (uint32_t)(cb ? __builtin_ctz((unsigned)cb) : 0);
+      const uint32_t tag = 100 + (uint32_t)hk * 32 + (lean ? 16u : 0u) + (uint32_t)(cb > 0 ? __builtin_ctz((unsigned)cb) : -cb);
       ops.add<LeafArgs>(tag, img.add(la, lb), [hk, cb, lean](Launch<LeafArgs> L, uint32_t g, hipStream_t st) {
         if (lean) {
           if (hk == HASH_MD5) launch_leaf1<HASH_MD5>(cb, L, g, st);

@@ -217,3 +217,39 @@ def test_hash_chunks_blocks(C, hk):
         assert len(got) == n + (tail > 0)
         for c in range(len(got)):
             assert got[c].tobytes() == O.hash_bytes(hk, a[c * C:(c + 1) * C]), c
+
+
+@pytest.mark.parametrize("hk", [M.MURMUR3, M.MD5])
+@pytest.mark.parametrize("C", [1, 5, 15, 17, 20, 24, 40, 51, 63, 100, 111, 112, 113, 127, 129, 144, 200, 255, 257, 1000])
+def test_hash_chunks_any_size(C, hk):
+    """Digests of chunk sizes that are no power of two, at every data alignment modulo
+    16: chunks staged as one piece and by rows, tails of every class, wavefronts at the
+    buffer's edges (first unaligned, last partial), and MD5 of few and many chunks."""
+    rng = np.random.default_rng(3 * C + hk)
+    n = 66_000 if hk == M.MD5 and C in (17, 100, 113) else 333
+    a = rng.integers(0, 256, n * C + 16, dtype=np.uint8)
+    some = range(n) if n < 1000 else sorted({*range(130), *range(n - 130, n), *rng.integers(0, n, 200).tolist()})
+    for off, cut in ((0, 0), (1, 1), (4, 0), (7, 0), (8, C // 2), (13, 0), (15, 0)):
+        size = n * C - cut
+        buf = torch.zeros(size + 32, dtype=torch.uint8, device="cuda:0")
+        buf[off:off + size] = torch.from_numpy(a[:size])
+        print(f"hash any C={C} hk={hk} n={n} off={off} cut={cut}", flush=True)
+        got = M.hash_chunks(buf[off:off + size], C, hk).cpu().numpy().reshape(-1, 16)
+        assert len(got) == (size + C - 1) // C
+        for c in some:
+            if c * C < size:
+                assert got[c].tobytes() == O.hash_bytes(hk, a[c * C:min((c + 1) * C, size)]), c
+
+
+@pytest.mark.parametrize("C,hk,n", [(100, 0, 3000), (100, 1, 66_000), (20, 0, 3000), (333, 0, 1000), (1000, 1, 700)])
+def test_series_of_any_chunk_size(C, hk, n):
+    rng = np.random.default_rng(C * n)
+    v = [rng.integers(0, 256, n * C + 3, dtype=np.uint8)]
+    for _ in range(2):
+        w = v[-1].copy()
+        for first in rng.integers(0, n, 12):
+            w[first * C:(first + 3) * C] = rng.integers(0, 256, w[first * C:(first + 3) * C].size, dtype=np.uint8)
+        src, dst = rng.integers(0, n, 2)
+        w[dst * C:(dst + 1) * C] = w[src * C:(src + 1) * C]
+        v.append(w)
+    same_as_oracle(v, C, hk)
