@@ -11,6 +11,7 @@ void restart_impl(const void* const* diffs, const uint64_t* sizes, uint32_t coun
 void last_restart_times(float* upload_ms, float* total_ms);
 void restart_noalloc_impl(const void* const* diffs, const uint64_t* sizes, uint32_t count, uint32_t k, uint8_t* out,
                           uint64_t out_len, hipStream_t st);
+void copy_device(const uint8_t* src, uint8_t* dst, uint64_t size, hipStream_t st);
 void hash_chunks(const uint8_t* data, uint64_t len, uint32_t C, int hk, Digest* out, hipStream_t st);
 void checkpoint_batch_impl(mtc_dedup* const* hs, const uint8_t* const* datas, const uint64_t* lens,
                            const int* baselines, uint32_t count, StepCtx& ctx, hipStream_t st, bool use_graph);
@@ -115,6 +116,8 @@ int mtc_destroy(mtc_dedup* h) {
     for (hipEvent_t e : h->copy_done)
       if (e) (void)hipEventDestroy(e);
   }
+  for (hipEvent_t e : h->copy_ev)
+    if (e) (void)hipEventDestroy(e);
   if (h->ctl_d) (void)hipFree(h->ctl_d);
   if (h->ctl_h) (void)hipHostFree(h->ctl_h);
   delete h;  // device buffers are released by their destructors
@@ -150,17 +153,22 @@ int mtc_copy_diff(mtc_dedup* h, void* host_dst, uint64_t capacity, void* stream)
     if (capacity < h->last_diff_size) throw Status{MTC_ERR_BUFFER_TOO_SMALL, "host buffer smaller than the diff"};
     MTC_HIP(hipSetDevice(h->device));
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipEvent_t a, b;
-    MTC_HIP(hipEventCreate(&a));
-    MTC_HIP(hipEventCreate(&b));
-    MTC_HIP(hipEventRecord(a, st));
-    // host or device destination (unified addressing decides the direction)
-    MTC_HIP(hipMemcpyAsync(host_dst, h->diff_ptr(), h->last_diff_size, hipMemcpyDefault, st));
-    MTC_HIP(hipEventRecord(b, st));
-    MTC_HIP(hipEventSynchronize(b));
-    (void)hipEventElapsedTime(&h->last_ms[3], a, b);
-    (void)hipEventDestroy(a);
-    (void)hipEventDestroy(b);
+    for (hipEvent_t& e : h->copy_ev)
+      if (!e) MTC_HIP(hipEventCreate(&e));
+    MTC_HIP(hipEventRecord(h->copy_ev[0], st));
+    // Device memory of this GPU: the library's own copy kernel (word-aligned); other
+    // memory: the runtime's (unified addressing decides the direction).
+    hipPointerAttribute_t attr;
+    const bool here = hipPointerGetAttributes(&attr, host_dst) == hipSuccess && attr.type == hipMemoryTypeDevice &&
+                      attr.device == h->device && (uintptr_t)host_dst % 4 == 0;
+    (void)hipGetLastError();  // a plain host pointer is no error
+    if (here) mtc::copy_device(h->diff_ptr(), static_cast<uint8_t*>(host_dst), h->last_diff_size, st);
+    else MTC_HIP(hipMemcpyAsync(host_dst, h->diff_ptr(), h->last_diff_size, hipMemcpyDefault, st));
+    MTC_HIP(hipEventRecord(h->copy_ev[1], st));
+    // (the stream, not the event: another thread may record the event again)
+    MTC_HIP(hipStreamSynchronize(st));
+    (void)hipEventElapsedTime(&h->last_ms[3], h->copy_ev[0], h->copy_ev[1]);
+    (void)hipGetLastError();
   });
 }
 

@@ -2432,6 +2432,27 @@ void hash_chunks(const uint8_t* data, uint64_t len, uint32_t C, int hk, Digest* 
   MTC_HIP(hipGetLastError());
 }
 
+// A device-to-device copy, 16 bytes a thread and no loop (a wait for a load also waits
+// for the stores before it).  src is 16-byte aligned, dst 4-byte aligned: the stores
+// are aligned, the loads shifted.  4 GiB read and written: 6.5 TB/s, 4.6 TB/s by the
+// runtime's copy kernel (which loops), 4.7 to 5.5 TB/s with looping blocks.
+__global__ __launch_bounds__(kThreads) void k_copy(const uint8_t* src, uint8_t* dst, uint64_t size) {
+  const uint32_t head = (uint32_t)min<uint64_t>((16 - ((uint32_t)(uintptr_t)dst & 15)) & 15, size & ~3ull);
+  const uint64_t units = (size - head) / 16, u = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (u < units) st_stream16(dst + head + 16 * u, ld_stream16_a4(src + head + 16 * u));
+  if (blockIdx.x == 0) {  // before the first aligned unit, and after the last
+    if (threadIdx.x < head) dst[threadIdx.x] = src[threadIdx.x];
+    const uint64_t t = head + 16 * units + threadIdx.x;
+    if (t < size) dst[t] = src[t];
+  }
+}
+
+void copy_device(const uint8_t* src, uint8_t* dst, uint64_t size, hipStream_t st) {
+  if (!size) return;
+  k_copy<<<(uint32_t)(size / 16 / kThreads + 1), kThreads, 0, st>>>(src, dst, size);
+  MTC_HIP(hipGetLastError());
+}
+
 template <int HK, int CB>
 static void launch_leaf_cb(Launch<LeafArgs> L, uint32_t grid, hipStream_t st) {
   k_leaf<HK, CB><<<grid, kThreads, 0, st>>>(L);

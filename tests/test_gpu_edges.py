@@ -253,3 +253,20 @@ def test_series_of_any_chunk_size(C, hk, n):
         w[dst * C:(dst + 1) * C] = w[src * C:(src + 1) * C]
         v.append(w)
     same_as_oracle(v, C, hk)
+
+
+def test_diff_copies_to_device_memory():
+    """mtc_copy_diff to device memory at every word offset modulo 16, and at byte
+    offsets: the diff's bytes and nothing around them."""
+    rng = np.random.default_rng(2)
+    for C, n in ((4, 1), (4, 3), (16, 5), (64, 700), (100, 333)):
+        host = rng.integers(0, 256, n * C, dtype=np.uint8)
+        d = M.TreeDeduplicator(C)
+        want = d.checkpoint(torch.from_numpy(host).to("cuda:0"), make_baseline=True)
+        for off in (0, 4, 8, 12, 1, 6):
+            out = torch.full((len(want) + 48,), 0x5A, dtype=torch.uint8, device="cuda:0")
+            got = d.copy_last_diff_device(out[16 + off:16 + off + len(want)])
+            o = out.cpu().numpy()
+            assert got.cpu().numpy().tobytes() == want
+            assert (o[:16 + off] == 0x5A).all() and (o[16 + off + len(want):] == 0x5A).all()
+        d.close()
