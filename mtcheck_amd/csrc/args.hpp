@@ -67,7 +67,7 @@ struct LeafArgs {
   Digest* leaf_dg;
   uint8_t* labels;
   int baseline;       // 1: previous digests are zero (a reset); 2: every chunk counts as changed
-  uint32_t* list;     // chunks to insert, packed per block
+  uint32_t* list;     // chunks to insert, packed per block (a baseline: the dense list)
   uint32_t* blk_cnt;  // their count per block
   uint64_t tiles_per_block;
   // 1: label every chunk.  0: the labels already hold L_FIXED for every chunk (the
@@ -115,6 +115,7 @@ struct CompactArgs {
   uint64_t len;
   uint32_t C;
   int hash_chunks;
+  int listed;               // a baseline: dense and the leaf digests are in place already
   __device__ CompactArgs global() const {
     CompactArgs c = *this;
     MTC_GLOBAL(list); MTC_GLOBAL(blk_cnt); MTC_GLOBAL(blk_off); MTC_GLOBAL(dense); MTC_GLOBAL(list_dg); MTC_GLOBAL(dense_dg);
@@ -139,7 +140,7 @@ struct DenseArgs {
   uint32_t R0;          // levels of the first sweep stage
   uint8_t* tile_first;  // per stage-0 tile: holds a first-occurrence leaf
   uint8_t* tile_busy;   // per stage-0 tile: holds a leaf that is not a fixed duplicate
-  const Digest* dense_dg;  // the listed chunks' digests, in dense order
+  const Digest* dense_dg;  // the listed chunks' digests, in dense order (a baseline: leaf_dg)
   int leaf_labels;         // the leaf kernel labelled the chunks (otherwise they count as pending)
   uint32_t* pend;          // k_insert lists the chunks k_fixmin and k_resolve visit, each group of
                            // 64 dense entries at the front of its own 64 words ...

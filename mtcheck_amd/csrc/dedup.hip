@@ -811,7 +811,8 @@ __device__ __forceinline__ void leaf1_tile(const LeafArgs& a, uint32_t blk, uint
   if (lane == 0 && m) base = atomicAdd(a.blk_cnt + blk, (uint32_t)__popcll(m));
   base = __shfl(base, 0);
   if (ins) {
-    const uint64_t k = t * kThreads + base + __popcll(m & ((1ull << lane) - 1));
+    // A baseline lists every chunk: in its own place (list is the dense list).
+    const uint64_t k = a.baseline ? c : t * kThreads + base + __popcll(m & ((1ull << lane) - 1));
     a.list[k] = (uint32_t)c;
     if (a.list_dg && !a.hash_later) a.list_dg[k] = d;
   }
@@ -877,6 +878,11 @@ __device__ __forceinline__ Digest chunk_m3(const uint8_t* data, uint64_t len, ui
 
 constexpr uint32_t kCompactPer = 32;  // leaf blocks per compaction block
 
+// A baseline lists every chunk, so its leaf kernel writes the dense list (each chunk in
+// its own place, its digest in the leaf array) and nothing is moved here: 283 us of a
+// 4 GiB baseline in 128-byte chunks, and 16 bytes a chunk less to read and write in
+// k_insert.
+//
 // The regions of kCompactPer consecutive leaf blocks land contiguously in the dense
 // list (their offsets are a prefix sum), so each thread copies entries by their
 // position in the group and finds the source region by a search in LDS.
@@ -884,6 +890,10 @@ __device__ __forceinline__ void ph_compact(const Launch<CompactArgs>& L, const W
   uint32_t* s_pre = reinterpret_cast<uint32_t*>(lds);
   const CompactArgs a = L.args[w.m].global();
   const uint32_t b0 = w.blk * kCompactPer, nb = min(kCompactPer, a.nblk - b0);
+  if (a.listed) {  // the leaf kernel wrote the dense list itself
+    if (threadIdx.x < nb) a.blk_cnt[b0 + threadIdx.x] = 0;
+    return;
+  }
   // One wavefront loads the counts at once and scans them (a walk by one thread
   // waits for each load in turn).
   if (threadIdx.x < 64) {
@@ -974,7 +984,7 @@ __device__ __forceinline__ void ph_insert(const Launch<DenseArgs>& L, const Wher
     if (follower) slot = hslot;
     if (v) {
       a.leaf_slot[c] = slot;
-      if (a.dense_dg) a.leaf_dg[c] = d;
+      if (a.dense_dg && a.dense_dg != a.leaf_dg) a.leaf_dg[c] = d;
       // Every leaf that is not a fixed duplicate is on this list, so sweep B walks
       // only the stage-0 tiles flagged here.
       if (a.R0) a.tile_busy[chunk_tile(a.g, a.R0, c)] = 1;
@@ -3031,11 +3041,11 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
     for (auto& M : ms) {
       mtc_dedup* h = M.h;
       ca.push_back(CompactArgs{h->list.p, h->blk_cnt.p, h->blk_off.p, M.tpb, h->dense.p, M.nblk_leaf, h->list_dg.p,
-                               h->dense_dg.p, M.data, M.len, h->chunk_size, M.hash_later ? 1 : 0});
+                               h->dense_dg.p, M.data, M.len, h->chunk_size, M.hash_later ? 1 : 0, M.baseline ? 1 : 0});
       cb.push_back((M.nblk_leaf + kCompactPer - 1) / kCompactPer);
       da.push_back(DenseArgs{h->dense.p, h->blk_off.p + M.nblk_leaf, M.n, h->leaf_dg.p, h->leaf_slot.p, h->labels.p,
                              h->table.p, h->table_cap - 1, M.cur, h->ctl_d, h->ctr.p, M.g, M.R0, h->tile_flags.p,
-                             h->tile_flags.p + M.ntile0, h->dense_dg.p, M.all_labels ? 1 : 0, h->pend.p,
+                             h->tile_flags.p + M.ntile0, M.baseline ? h->leaf_dg.p : h->dense_dg.p, M.all_labels ? 1 : 0, h->pend.p,
                              h->pcnt.p});
       db.push_back(grid_for(M.n, 8 * kThreads, 16384));
       pb.push_back(grid_for(M.n, kPendPerBlock, 4096));
@@ -3302,7 +3312,8 @@ static void build_basic_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) 
     std::vector<uint32_t> cb;
     for (auto& M : ms) {
       mtc_dedup* h = M.h;
-      ca.push_back(CompactArgs{h->list.p, h->blk_cnt.p, h->blk_off.p, M.tpb, h->dense.p, M.nblk_leaf, nullptr, nullptr});
+      ca.push_back(CompactArgs{h->list.p, h->blk_cnt.p, h->blk_off.p, M.tpb, h->dense.p, M.nblk_leaf, nullptr, nullptr, nullptr, 0, 0, 0,
+                               M.baseline ? 1 : 0});
       cb.push_back((M.nblk_leaf + kCompactPer - 1) / kCompactPer);
     }
     ops.add<CompactArgs>(21, img.add(ca, cb), [](Launch<CompactArgs> L, uint32_t g, hipStream_t st) { k_compact<<<g, kThreads, 0, st>>>(L); });
@@ -3402,8 +3413,9 @@ static void build_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img, int ph
         // basic approach: every chunk of the first checkpoint is changed (src/basic_approach.cpp:36-45)
         const int reset = !M.baseline ? 0 : (h->approach == MTC_APPROACH_BASIC && M.cur == 0) ? 2 : 1;
         la.push_back(LeafArgs{M.data, M.len, M.n, h->chunk_size, h->leaf_dg.p, h->labels.p, reset,
-                              h->list.p, h->blk_cnt.p, M.tpb, M.all_labels ? 1 : 0,
-                              h->approach == MTC_APPROACH_BASIC ? nullptr : h->list_dg.p, &h->ctl_d->t_begin,
+                              M.baseline ? h->dense.p : h->list.p, h->blk_cnt.p, M.tpb, M.all_labels ? 1 : 0,
+                              h->approach == MTC_APPROACH_BASIC ? nullptr : M.baseline ? h->leaf_dg.p : h->list_dg.p,
+                              &h->ctl_d->t_begin,
                               M.hash_later ? 1 : 0});
         lb.push_back(M.nblk_leaf);
       }
