@@ -102,7 +102,7 @@ struct Prologue {
 
 struct CompactArgs {
   const uint32_t* list;
-  uint32_t* blk_cnt;  // read, then cleared for the next step's leaf kernel
+  uint32_t* blk_cnt;  // read, then cleared for the next step's leaf kernel (see total)
   const uint32_t* blk_off;
   uint64_t tiles_per_block;
   uint32_t* dense;
@@ -116,8 +116,15 @@ struct CompactArgs {
   uint32_t C;
   int hash_chunks;
   int listed;               // a baseline: dense and the leaf digests are in place already
+  uint32_t n;
+  // Set: no scan came before.  The blocks add up the counts before their own, the last
+  // one writes the total here, and the first one closes the leaf phase (stamp); the
+  // counts are cleared by the step's diff kernel.
+  uint32_t* total;
+  unsigned long long* stamp;
   __device__ CompactArgs global() const {
     CompactArgs c = *this;
+    MTC_GLOBAL(total); MTC_GLOBAL(stamp);
     MTC_GLOBAL(list); MTC_GLOBAL(blk_cnt); MTC_GLOBAL(blk_off); MTC_GLOBAL(dense); MTC_GLOBAL(list_dg); MTC_GLOBAL(dense_dg);
     MTC_GLOBAL(data);
     return c;
@@ -243,6 +250,7 @@ struct SortArgs {
   const uint32_t* S;
   uint32_t shift, nb;  // digit shift and number of digit values (a power of two <= 256)
   uint32_t* hist;      // nb * G counts, then their exclusive scan
+  uint32_t raw;        // 1: hist stays the counts; k_sort_move adds them up itself
   __device__ SortArgs global() const {
     SortArgs c = *this;
     MTC_GLOBAL(key_in); MTC_GLOBAL(val_in); MTC_GLOBAL(key_out); MTC_GLOBAL(val_out); MTC_GLOBAL(S); MTC_GLOBAL(hist);
@@ -269,8 +277,10 @@ struct RegionArgs {
   uint32_t* sizes;
   int compat;     // the reference's leaf ranges
   PtableArgs pt;  // the (chkpt, count) table, built by block 0
+  uint32_t* sums;  // per scan tile: the sum of its sizes
   __device__ RegionArgs global() const {
     RegionArgs c = *this;
+    MTC_GLOBAL(sums);
     MTC_GLOBAL(first_roots); MTC_GLOBAL(F); MTC_GLOBAL(sizes);
     c.pt = pt.global();
     return c;
@@ -298,8 +308,11 @@ struct DiffArgs {
   Ctl* out;                       // the member's entry of the step's result array
   const uint32_t* dense;          // the listed chunks (*changed of them)
   uint8_t* reset_labels;          // when set: their labels go back to L_FIXED
+  uint32_t* clear_cnt;            // leaf block counts to clear (clear_n of them)
+  uint32_t clear_n;
   __device__ DiffArgs global() const {
     DiffArgs c = *this;
+    MTC_GLOBAL(clear_cnt);
     MTC_GLOBAL(diff); MTC_GLOBAL(first_roots); MTC_GLOBAL(ptable); MTC_GLOBAL(shift_sorted); MTC_GLOBAL(region_off); MTC_GLOBAL(tile_lo); MTC_GLOBAL(total_chunks); MTC_GLOBAL(data); MTC_GLOBAL(ctl);
     MTC_GLOBAL(ctr); MTC_GLOBAL(changed); MTC_GLOBAL(out); MTC_GLOBAL(dense); MTC_GLOBAL(reset_labels);
     return c;
@@ -318,8 +331,11 @@ struct BasicDiffArgs {
   int aligned;
   const unsigned long long* ctr;
   Ctl* out;
+  uint32_t* clear_cnt;  // leaf block counts to clear (clear_n of them)
+  uint32_t clear_n;
   __device__ BasicDiffArgs global() const {
     BasicDiffArgs c = *this;
+    MTC_GLOBAL(clear_cnt);
     MTC_GLOBAL(diff); MTC_GLOBAL(dense); MTC_GLOBAL(total); MTC_GLOBAL(data); MTC_GLOBAL(ctl); MTC_GLOBAL(ctr); MTC_GLOBAL(out);
     return c;
   }

@@ -38,6 +38,10 @@ constexpr uint32_t kScanTile = 8 * kThreads;   // elements per block-tile of the
 constexpr uint32_t kScanOneItems = 16;          // elements per thread of a one-launch scan
 constexpr uint32_t kScanOneMax = kScanOneItems * kThreads;
 constexpr uint32_t kSortBlocks = 1024;         // most blocks per member of the stable sort
+// Most counts that each block of a sort pass adds up by itself, in place of a scan's
+// launch (64 MiB of 128-byte chunks, up to 2048 counts: 6.3 us, 3.9 and a scan of 4.2
+// before; with 8192 counts 28 us against 5.3 and 10).
+constexpr uint32_t kSortRaw = 2048;
 // Wavefronts per block of the sweeps.  Wavefronts of one block draw very
 // different numbers of busy tiles, and a block holds its slot (and sweep A's LDS
 // records) until its slowest wavefront ends: with four wavefronts per block only
@@ -877,6 +881,9 @@ __device__ __forceinline__ Digest chunk_m3(const uint8_t* data, uint64_t len, ui
 }
 
 constexpr uint32_t kCompactPer = 32;  // leaf blocks per compaction block
+// Most leaf blocks whose counts every compaction block adds up by itself, up to its
+// own, in place of a scan's launch (4 us, of about 190 us of a 64 MiB checkpoint).
+constexpr uint32_t kSelfScan = 4096;
 
 // A baseline lists every chunk, so its leaf kernel writes the dense list (each chunk in
 // its own place, its digest in the leaf array) and nothing is moved here: 283 us of a
@@ -890,16 +897,28 @@ __device__ __forceinline__ void ph_compact(const Launch<CompactArgs>& L, const W
   uint32_t* s_pre = reinterpret_cast<uint32_t*>(lds);
   const CompactArgs a = L.args[w.m].global();
   const uint32_t b0 = w.blk * kCompactPer, nb = min(kCompactPer, a.nblk - b0);
+  if (a.total && w.blk == 0 && threadIdx.x == 0) *a.stamp = wall_clock64();  // no scan's launch to close the leaf phase
   if (a.listed) {  // the leaf kernel wrote the dense list itself
-    if (threadIdx.x < nb) a.blk_cnt[b0 + threadIdx.x] = 0;
+    if (!a.total) {
+      if (threadIdx.x < nb) a.blk_cnt[b0 + threadIdx.x] = 0;
+    } else if (w.blk == 0 && threadIdx.x == 0) {
+      *a.total = a.n;
+    }
     return;
+  }
+  uint32_t before = 0;
+  if (a.total) {  // few leaf blocks: add up the counts before this block's
+    uint32_t v = 0;
+    for (uint32_t i = threadIdx.x; i < b0; i += kThreads) v += a.blk_cnt[i];
+    uint32_t* ws = s_pre + kCompactPer + 2;
+    block_scan_excl(v, &before, ws);
   }
   // One wavefront loads the counts at once and scans them (a walk by one thread
   // waits for each load in turn).
   if (threadIdx.x < 64) {
     const uint32_t lane = threadIdx.x;
     const uint32_t v = lane < nb ? a.blk_cnt[b0 + lane] : 0u;
-    if (lane == 0) s_pre[kCompactPer + 1] = a.blk_off[b0];
+    if (lane == 0) s_pre[kCompactPer + 1] = a.total ? before : a.blk_off[b0];
     uint32_t x = v;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -910,10 +929,12 @@ __device__ __forceinline__ void ph_compact(const Launch<CompactArgs>& L, const W
     if (lane + 1 == nb) s_pre[nb] = x;
   }
   __syncthreads();
-  // The last reader of the counts clears them (the leaf scan read them before).
-  if (threadIdx.x < nb) a.blk_cnt[b0 + threadIdx.x] = 0;
+  // The last reader of the counts clears them (the leaf scan read them before; without
+  // one the step's diff kernel does).
+  if (!a.total && threadIdx.x < nb) a.blk_cnt[b0 + threadIdx.x] = 0;
   const uint32_t total = s_pre[nb];
   const uint32_t off = s_pre[kCompactPer + 1];
+  if (a.total && b0 + nb == a.nblk && threadIdx.x == 0) *a.total = off + total;
   uint32_t* dst = a.dense + off;
   for (uint32_t e = threadIdx.x; e < total; e += kThreads) {
     uint32_t lo = 0, hi = nb;  // last region whose start <= e
@@ -930,7 +951,7 @@ __device__ __forceinline__ void ph_compact(const Launch<CompactArgs>& L, const W
 }
 
 __global__ __launch_bounds__(kThreads, 8) void k_compact(Launch<CompactArgs> L) {
-  __shared__ __align__(16) uint8_t lds[sizeof(uint32_t) * (kCompactPer + 2)];
+  __shared__ __align__(16) uint8_t lds[sizeof(uint32_t) * (kCompactPer + 2 + kThreads / 64)];
   ph_compact(L, where(L), lds);
 }
 
@@ -1956,6 +1977,26 @@ __device__ __forceinline__ void ph_sort_move(const Launch<SortArgs>& L, const Wh
   run[tid] = 0;
   uint32_t lo, hi;
   sort_range(*a.S, wh.blk, wh.nblk, lo, hi);
+  if (lo >= hi) return;  // the whole block
+  if (a.raw) {
+    // Few counts: each block adds up those before its own (all of the smaller digits',
+    // and the earlier blocks' of each digit) instead of waiting for a scan's launch.
+    uint32_t *all = &cnt[0][0], *before = &cnt[1][0], *ws = &cnt[2][0];
+    all[tid] = 0;
+    before[tid] = 0;
+    __syncthreads();
+    for (uint32_t i = tid; i < a.nb * wh.nblk; i += kThreads) {
+      const uint32_t v = a.hist[i];
+      if (!v) continue;
+      const uint32_t d = i / wh.nblk, g = i - d * wh.nblk;
+      atomicAdd(&all[d], v);
+      if (g < wh.blk) atomicAdd(&before[d], v);
+    }
+    __syncthreads();
+    uint32_t tot;
+    const uint32_t mine = tid < a.nb ? all[tid] : 0u, pre = tid < a.nb ? before[tid] : 0u;
+    run[tid] = block_scan_excl(mine, &tot, ws) + pre;  // (syncs before cnt is cleared)
+  }
   for (uint32_t r0 = lo; r0 < hi; r0 += kThreads) {
     for (uint32_t j = tid; j < (kThreads / 64) * 256; j += kThreads) (&cnt[0][0])[j] = 0;
     __syncthreads();
@@ -1981,7 +2022,7 @@ __device__ __forceinline__ void ph_sort_move(const Launch<SortArgs>& L, const Wh
     }
     __syncthreads();
     if (valid) {
-      uint32_t pos = a.hist[dg * wh.nblk + wh.blk] + run[dg] + rank;
+      uint32_t pos = (a.raw ? 0u : a.hist[dg * wh.nblk + wh.blk]) + run[dg] + rank;
       for (uint32_t ww = 0; ww < w; ww++) pos += cnt[ww][dg];
       a.key_out[pos] = k;
       a.val_out[pos] = a.val_in[i];
@@ -2025,11 +2066,24 @@ __device__ __forceinline__ void ph_region_sizes(const Launch<RegionArgs>& L, con
   uint32_t* s_ws = reinterpret_cast<uint32_t*>(lds);
   const RegionArgs a = L.args[w.m].global();
   if (w.blk == 0) build_ptable(a.pt, s_ws);
-  const uint32_t F = *a.F;
-  for (uint32_t i = w.blk * kThreads + threadIdx.x; i < F; i += w.nblk * kThreads) {
-    uint32_t st[2], ct[2];
-    const int r = region_runs(a.g, a.first_roots[i], a.compat, st, ct);
-    a.sizes[i] = r == 0 ? 0 : (r == 1 ? ct[0] : ct[0] + ct[1]);
+  // By the scan's tiles, whose sums are written too (the first launch of the region
+  // scan would only read the sizes again).
+  const uint32_t F = *a.F, ntiles = (F + kScanTile - 1) / kScanTile;
+  for (uint32_t tile = w.blk; tile < ntiles; tile += w.nblk) {
+    uint32_t sum = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kScanTile / kThreads; j++) {
+      const uint32_t i = tile * kScanTile + j * kThreads + threadIdx.x;
+      if (i >= F) continue;
+      uint32_t st[2], ct[2];
+      const int r = region_runs(a.g, a.first_roots[i], a.compat, st, ct);
+      const uint32_t size = r == 0 ? 0 : (r == 1 ? ct[0] : ct[0] + ct[1]);
+      a.sizes[i] = size;
+      sum += size;
+    }
+    uint32_t tot;
+    block_scan_excl(sum, &tot, s_ws);
+    if (threadIdx.x == 0) a.sums[tile] = tot;
   }
 }
 
@@ -2228,6 +2282,7 @@ __device__ __forceinline__ void ph_assemble(const Launch<DiffArgs>& L, const Whe
       __syncthreads();
     }
   }
+  for (uint32_t i = wh.blk * kThreads + threadIdx.x; i < a.clear_n; i += wh.nblk * kThreads) a.clear_cnt[i] = 0;
   diff_meta(a, wh);
   // Nothing reads the leaf labels after sweep B: the listed chunks go back to
   // L_FIXED, so the next step's leaf kernel labels only the chunks it lists.
@@ -2300,6 +2355,7 @@ __device__ __forceinline__ void ph_basic_diff(const Launch<BasicDiffArgs>& L, co
       __syncthreads();
     }
   }
+  for (uint32_t i = wh.blk * kThreads + threadIdx.x; i < a.clear_n; i += wh.nblk * kThreads) a.clear_cnt[i] = 0;
   for (uint64_t i = (uint64_t)wh.blk * kThreads + threadIdx.x; i < F; i += (uint64_t)wh.nblk * kThreads) out[8 + i] = a.dense[i];
 }
 
@@ -2860,6 +2916,7 @@ struct Member {
   bool all_labels = true;  // the leaf kernel labels every chunk, not only the listed ones
   bool hash_later = false;  // k_compact hashes the listed chunks; the leaf kernel stores no digest
   uint64_t blk_zero = 0;   // leading block counts known to be zero when the step starts
+  bool self_scan = false;  // few leaf blocks: the compaction adds up their counts itself
   Geo g{};
   uint32_t* ws_blk = nullptr;  // scan partial sums of this member
   uint32_t* ws_f = nullptr;
@@ -2960,6 +3017,7 @@ static void prepare_member(Member& M, hipStream_t st) {
   M.hash_later = !M.baseline && h->approach != MTC_APPROACH_BASIC && h->hash_kind == HASH_MURMUR3 && M.cb >= 16 &&
                  M.tpb == 1 && hash_later_fits(M.n, h->chunk_size) && h->ctl_h &&
                  h->ctl_h->changed * kHashLaterBelow <= M.n;
+  M.self_scan = M.nblk_leaf <= kSelfScan;
   // Block counts that k_compact cleared at the end of the last completed step (the
   // same buffer); unknown again until this step completes.
   M.blk_zero = h->blk_zero_p == h->blk_cnt.p ? h->blk_zero : 0;
@@ -2988,7 +3046,8 @@ static void prepare_member(Member& M, hipStream_t st) {
   }
 }
 
-static void add_scan(Ops& ops, ArenaImage& img, const std::vector<ScanSeg>& segs) {
+// have_sums: the tile sums are written already.
+static void add_scan(Ops& ops, ArenaImage& img, const std::vector<ScanSeg>& segs, bool have_sums = false) {
   if (segs.empty()) return;
   std::vector<uint32_t> tiles, ones(segs.size(), 1);
   if (std::all_of(segs.begin(), segs.end(), [](const ScanSeg& s) { return s.count_max <= kScanOneMax; })) {
@@ -2997,16 +3056,16 @@ static void add_scan(Ops& ops, ArenaImage& img, const std::vector<ScanSeg>& segs
   }
   for (const auto& s : segs) tiles.push_back(std::max<uint32_t>(1, std::min<uint32_t>(512, (s.count_max + kScanTile - 1) / kScanTile)));
   const LaunchRec rt = img.add(segs, tiles);
-  ops.add<ScanSeg>(10, rt, [](Launch<ScanSeg> L, uint32_t g, hipStream_t st) { k_scan_reduce<<<g, kThreads, 0, st>>>(L); });
+  if (!have_sums) ops.add<ScanSeg>(10, rt, [](Launch<ScanSeg> L, uint32_t g, hipStream_t st) { k_scan_reduce<<<g, kThreads, 0, st>>>(L); });
   ops.add<ScanSeg>(14, rt, [](Launch<ScanSeg> L, uint32_t g, hipStream_t st) { k_scan_down2<<<g, kThreads, 0, st>>>(L); });
 }
 
 // The scan of the leaf blocks' counts (the offsets of each block's list of
-// chunks to insert, and their total).
+// chunks to insert, and their total), unless the compaction adds them up itself.
 static void add_leaf_scan(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
   std::vector<ScanSeg> ss;
   for (auto& M : ms)  // its first block's start closes the leaf phase
-    ss.push_back(ScanSeg{M.h->blk_cnt.p, M.h->blk_off.p, nullptr, M.nblk_leaf, M.h->blk_off.p + M.nblk_leaf, M.ws_blk,
+    if (!M.self_scan) ss.push_back(ScanSeg{M.h->blk_cnt.p, M.h->blk_off.p, nullptr, M.nblk_leaf, M.h->blk_off.p + M.nblk_leaf, M.ws_blk,
                          &M.h->ctl_d->t_leaf});
   add_scan(ops, img, ss);
 }
@@ -3041,7 +3100,8 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
     for (auto& M : ms) {
       mtc_dedup* h = M.h;
       ca.push_back(CompactArgs{h->list.p, h->blk_cnt.p, h->blk_off.p, M.tpb, h->dense.p, M.nblk_leaf, h->list_dg.p,
-                               h->dense_dg.p, M.data, M.len, h->chunk_size, M.hash_later ? 1 : 0, M.baseline ? 1 : 0});
+                               h->dense_dg.p, M.data, M.len, h->chunk_size, M.hash_later ? 1 : 0, M.baseline ? 1 : 0, M.n,
+                               M.self_scan ? h->blk_off.p + M.nblk_leaf : nullptr, &h->ctl_d->t_leaf});
       cb.push_back((M.nblk_leaf + kCompactPer - 1) / kCompactPer);
       da.push_back(DenseArgs{h->dense.p, h->blk_off.p + M.nblk_leaf, M.n, h->leaf_dg.p, h->leaf_slot.p, h->labels.p,
                              h->table.p, h->table_cap - 1, M.cur, h->ctl_d, h->ctr.p, M.g, M.R0, h->tile_flags.p,
@@ -3240,11 +3300,12 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
         while ((1ull << bits) < M.nbins) bits++;
         const uint32_t shift = 8 * p;
         const uint32_t nb = (p < M.passes) ? (1u << std::min<uint32_t>(8, bits - shift)) : 1u;
+        const bool raw = nb * M.Gs <= kSortRaw;
         so.push_back(SortArgs{h->sort_key[p % 2].p, h->sort_val[p % 2].p, h->sort_key[1 - p % 2].p,
-                              h->sort_val[1 - p % 2].p, &h->ctl_d->S, shift, nb, h->sort_hist.p});
+                              h->sort_val[1 - p % 2].p, &h->ctl_d->S, shift, nb, h->sort_hist.p, raw ? 1u : 0u});
         sblk.push_back(p < M.passes ? M.Gs : 0u);
         cblk.push_back(p < M.passes && !(p == 0 && M.nbins <= kLdsBins) ? M.Gs : 0u);  // else counted by k_shift_src
-        if (p < M.passes) hs.push_back(ScanSeg{h->sort_hist.p, h->sort_hist.p, nullptr, nb * M.Gs, nullptr, M.ws_sort});
+        if (p < M.passes && !raw) hs.push_back(ScanSeg{h->sort_hist.p, h->sort_hist.p, nullptr, nb * M.Gs, nullptr, M.ws_sort});
       }
       const LaunchRec r = img.add(so, sblk), rc = img.add(so, cblk);
       ops.add<SortArgs>(61, rc, [](Launch<SortArgs> L, uint32_t g, hipStream_t st) { k_sort_count<<<g, kThreads, 0, st>>>(L); });
@@ -3260,13 +3321,13 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
     for (auto& M : ms) {
       mtc_dedup* h = M.h;
       ra.push_back(RegionArgs{h->first_roots.p, &h->ctl_d->F, M.g, h->region_off.p, h->compat,
-                              PtableArgs{h->src_hist.p, M.nbins, h->baseline_id, h->ptable.p, h->ctl_d}});
-      rb.push_back(grid_for(M.n, 16 * kThreads, 256));
+                              PtableArgs{h->src_hist.p, M.nbins, h->baseline_id, h->ptable.p, h->ctl_d}, M.ws_reg});
+      rb.push_back(grid_for(M.n, 16 * kThreads, 512));
       ss.push_back(ScanSeg{h->region_off.p, h->region_off.p, &h->ctl_d->F, M.n, h->region_off.p + M.n, M.ws_reg,
                            nullptr, h->tile_lo.p});
     }
     ops.add<RegionArgs>(70, img.add(ra, rb), [](Launch<RegionArgs> L, uint32_t g, hipStream_t st) { k_region_sizes<<<g, kThreads, 0, st>>>(L); });
-    add_scan(ops, img, ss);
+    add_scan(ops, img, ss, true);
     std::vector<DiffArgs> da;
     std::vector<uint32_t> gb;
     for (size_t i = 0; i < B; i++) {
@@ -3295,6 +3356,8 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
       d.out = M.ctl_out;
       d.dense = h->dense.p;
       d.reset_labels = h->debug ? nullptr : h->labels.p;  // the debug view copies them after the step
+      d.clear_cnt = h->blk_cnt.p;
+      d.clear_n = M.self_scan ? M.nblk_leaf : 0;
       da.push_back(d);
       gb.push_back(gather_blocks(M, ms.size()));
     }
@@ -3313,7 +3376,8 @@ static void build_basic_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) 
     for (auto& M : ms) {
       mtc_dedup* h = M.h;
       ca.push_back(CompactArgs{h->list.p, h->blk_cnt.p, h->blk_off.p, M.tpb, h->dense.p, M.nblk_leaf, nullptr, nullptr, nullptr, 0, 0, 0,
-                               M.baseline ? 1 : 0});
+                               M.baseline ? 1 : 0, M.n, M.self_scan ? h->blk_off.p + M.nblk_leaf : nullptr,
+                               &h->ctl_d->t_leaf});
       cb.push_back((M.nblk_leaf + kCompactPer - 1) / kCompactPer);
     }
     ops.add<CompactArgs>(21, img.add(ca, cb), [](Launch<CompactArgs> L, uint32_t g, hipStream_t st) { k_compact<<<g, kThreads, 0, st>>>(L); });
@@ -3336,6 +3400,8 @@ static void build_basic_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) 
     d.aligned = gather_pow2(M);
     d.ctr = h->ctr.p;
     d.out = M.ctl_out;
+    d.clear_cnt = h->blk_cnt.p;
+    d.clear_n = M.self_scan ? M.nblk_leaf : 0;
     da.push_back(d);
     gb.push_back(gather_blocks(M, ms.size()));
   }
@@ -3515,6 +3581,8 @@ static void run_step_body(StepCtx& ctx, std::vector<Member>& ms, hipStream_t st,
 
   const bool debug = std::any_of(ms.begin(), ms.end(), [](const Member& M) { return M.h->debug != 0; });
   const bool split = std::any_of(ms.begin(), ms.end(), [](const Member& M) { return M.split; });
+  if (split)  // the counts of chunks to insert are read before the second part
+    for (auto& M : ms) M.self_scan = false;
   const bool graph = use_graph && !debug;
   // Each member's last kernel writes its control block straight into pinned host
   // memory: no copy (and no idle time before one) ends the step.
