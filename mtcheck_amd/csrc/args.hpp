@@ -270,19 +270,24 @@ struct PtableArgs {
   }
 };
 
+// Two launches take this: k_root_info (the shifted entries' sources in the first
+// shift_blocks blocks, the regions' sizes in the others) and k_region_scan (the sort's
+// first pass in the first sort_blocks blocks, the scan of the sizes and the (chkpt,
+// count) table in the others).
 struct RegionArgs {
   const uint32_t* first_roots;
   const uint32_t* F;
   Geo g;
   uint32_t* sizes;
   int compat;     // the reference's leaf ranges
-  PtableArgs pt;  // the (chkpt, count) table, built by block 0
-  uint32_t* sums;  // per scan tile: the sum of its sizes
-  __device__ RegionArgs global() const {
+  PtableArgs pt;  // the (chkpt, count) table
+  ShiftArgs shift;
+  SortArgs sort;
+  ScanSeg scan;    // of the sizes; its sums come from k_root_info
+  uint32_t shift_blocks, sort_blocks;
+  __device__ RegionArgs global() const {  // k_root_info's own part
     RegionArgs c = *this;
-    MTC_GLOBAL(sums);
-    MTC_GLOBAL(first_roots); MTC_GLOBAL(F); MTC_GLOBAL(sizes);
-    c.pt = pt.global();
+    MTC_GLOBAL(first_roots); MTC_GLOBAL(F); MTC_GLOBAL(sizes); MTC_GLOBAL(scan.sums);
     return c;
   }
 };

@@ -218,9 +218,8 @@ __global__ __launch_bounds__(kThreads) void k_scan_reduce(Launch<ScanSeg> L) {
 // The second launch of the scan: each block sums the tile sums before its tiles
 // itself (reading each sum once, as its tiles advance), so the top-level scan
 // needs no launch of its own; the block of the last tile writes the total.
-__device__ __forceinline__ void ph_scan_down2(const Launch<ScanSeg>& L, const Where& w, uint8_t* lds) {
+__device__ __forceinline__ void ph_scan_down2(const ScanSeg& s, const Where& w, uint8_t* lds) {
   uint32_t* ws = reinterpret_cast<uint32_t*>(lds);
-  const ScanSeg s = L.args[w.m].global();
   const uint32_t cnt = scan_count(s), ntiles = (cnt + kScanTile - 1) / kScanTile;
   if (ntiles == 0 && w.blk == 0 && threadIdx.x == 0 && s.total) *s.total = 0;
   uint32_t pre = 0, done = 0;  // pre = sums[0] + ... + sums[done - 1]
@@ -255,7 +254,8 @@ __device__ __forceinline__ void ph_scan_down2(const Launch<ScanSeg>& L, const Wh
 
 __global__ __launch_bounds__(kThreads) void k_scan_down2(Launch<ScanSeg> L) {
   __shared__ __align__(16) uint8_t lds[sizeof(uint32_t) * (kThreads / 64)];
-  ph_scan_down2(L, where(L), lds);
+  const Where w = where(L);
+  ph_scan_down2(L.args[w.m].global(), w, lds);
 }
 
 // A scan whose every segment has at most kScanOneMax elements: one block per
@@ -278,10 +278,7 @@ __device__ __forceinline__ void ph_scan_one(const Launch<ScanSeg>& L, const Wher
   const uint32_t off = block_scan_excl(run, &tot, ws);
 #pragma unroll
   for (uint32_t j = 0; j < kScanOneItems; j++)
-    if (base + j < cnt) {
-      if (s.tile_lo) mark_tiles(s.tile_lo, off + v[j], (j + 1 < kScanOneItems ? v[j + 1] : run) - v[j], base + j);
-      s.out[base + j] = off + v[j];
-    }
+    if (base + j < cnt) s.out[base + j] = off + v[j];
   if (threadIdx.x == 0 && s.total) *s.total = tot;
 }
 
@@ -1891,9 +1888,8 @@ __device__ __forceinline__ void sort_range(uint32_t S, uint32_t g, uint32_t G, u
   hi = min(S, lo + per);
 }
 
-__device__ __forceinline__ void ph_shift_src(const Launch<ShiftArgs>& L, const Where& w, uint8_t* lds) {
+__device__ __forceinline__ void ph_shift_src(const ShiftArgs& a, const Where& w, uint8_t* lds) {
   uint32_t* h = reinterpret_cast<uint32_t*>(lds);
-  const ShiftArgs a = L.args[w.m].global();
   const bool in_lds = a.nbins <= kLdsBins;
   if (in_lds)
     for (uint32_t b = threadIdx.x; b < a.nbins; b += kThreads) h[b] = 0;
@@ -1940,11 +1936,6 @@ __device__ __forceinline__ void ph_shift_src(const Launch<ShiftArgs>& L, const W
     }
 }
 
-__global__ __launch_bounds__(kThreads) void k_shift_src(Launch<ShiftArgs> L) {
-  __shared__ __align__(16) uint8_t lds[sizeof(uint32_t) * kLdsBins];
-  ph_shift_src(L, where(L), lds);
-}
-
 // Stable counting sort by one 8-bit digit with a fixed grid: block g of G owns a
 // contiguous range of the S entries (S read on the device), counts its digits,
 // and after a scan of the digit-major (digit, block) counts moves its entries in
@@ -1968,10 +1959,10 @@ __global__ __launch_bounds__(kThreads) void k_sort_count(Launch<SortArgs> L) {
   ph_sort_count(L, where(L), lds);
 }
 
-__device__ __forceinline__ void ph_sort_move(const Launch<SortArgs>& L, const Where& wh, uint8_t* lds) {
+constexpr uint32_t kSortMoveLds = sizeof(uint32_t) * ((kThreads / 64) * 256 + 256);
+__device__ __forceinline__ void ph_sort_move(const SortArgs& a, const Where& wh, uint8_t* lds) {
   auto& cnt = *reinterpret_cast<uint32_t(*)[kThreads / 64][256]>(lds);
   uint32_t* run = reinterpret_cast<uint32_t*>(lds + sizeof(uint32_t) * (kThreads / 64) * 256);
-  const SortArgs a = L.args[wh.m].global();
   const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const uint64_t lt = (1ull << lane) - 1;
   run[tid] = 0;
@@ -2038,8 +2029,9 @@ __device__ __forceinline__ void ph_sort_move(const Launch<SortArgs>& L, const Wh
 }
 
 __global__ __launch_bounds__(kThreads) void k_sort_move(Launch<SortArgs> L) {
-  __shared__ __align__(16) uint8_t lds[sizeof(uint32_t) * ((kThreads / 64) * 256 + 256)];
-  ph_sort_move(L, where(L), lds);
+  __shared__ __align__(16) uint8_t lds[kSortMoveLds];
+  const Where w = where(L);
+  ph_sort_move(L.args[w.m].global(), w, lds);
 }
 
 // (chkpt, count) table in ascending checkpoint id (src/tree_approach.cpp:657-665).
@@ -2062,12 +2054,10 @@ __device__ void build_ptable(const PtableArgs& a, uint32_t* s_ws) {
   if (threadIdx.x == 0) a.ctl->P = base;
 }
 
-__device__ __forceinline__ void ph_region_sizes(const Launch<RegionArgs>& L, const Where& w, uint8_t* lds) {
+// Sizes of the regions under the first-occurrence roots, by the scan's tiles, whose
+// sums are written too (the first launch of a scan would only read the sizes again).
+__device__ __forceinline__ void ph_region_sizes(const RegionArgs& a, const Where& w, uint8_t* lds) {
   uint32_t* s_ws = reinterpret_cast<uint32_t*>(lds);
-  const RegionArgs a = L.args[w.m].global();
-  if (w.blk == 0) build_ptable(a.pt, s_ws);
-  // By the scan's tiles, whose sums are written too (the first launch of the region
-  // scan would only read the sizes again).
   const uint32_t F = *a.F, ntiles = (F + kScanTile - 1) / kScanTile;
   for (uint32_t tile = w.blk; tile < ntiles; tile += w.nblk) {
     uint32_t sum = 0;
@@ -2083,13 +2073,37 @@ __device__ __forceinline__ void ph_region_sizes(const Launch<RegionArgs>& L, con
     }
     uint32_t tot;
     block_scan_excl(sum, &tot, s_ws);
-    if (threadIdx.x == 0) a.sums[tile] = tot;
+    if (threadIdx.x == 0) a.scan.sums[tile] = tot;
   }
 }
 
-__global__ __launch_bounds__(kThreads) void k_region_sizes(Launch<RegionArgs> L) {
-  __shared__ __align__(16) uint8_t lds[sizeof(uint32_t) * (kThreads / 64)];
-  ph_region_sizes(L, where(L), lds);
+// What only the compacted roots are needed for: the shifted entries' sources and the
+// regions' sizes, side by side in one launch.  A small checkpoint is a chain of
+// launches of 4-7 us whose work takes one or two: this and k_region_scan are two
+// launches where there were four (a baseline and the 9 checkpoints after it of 64 MiB
+// in 128-byte chunks: 1819 us, 1886 before).
+__global__ __launch_bounds__(kThreads) void k_root_info(Launch<RegionArgs> L) {
+  __shared__ __align__(16) uint8_t lds[sizeof(uint32_t) * kLdsBins];
+  const Where w = where(L);
+  const RegionArgs& a = L.args[w.m];
+  if (w.blk < a.shift_blocks) ph_shift_src(a.shift.global(), Where{w.m, w.blk, a.shift_blocks}, lds);
+  else ph_region_sizes(a.global(), Where{w.m, w.blk - a.shift_blocks, w.nblk - a.shift_blocks}, lds);
+}
+
+// What the launch of k_root_info leaves: the first pass of the sort by source (if
+// there is more than one source), the scan of the region sizes, and the (chkpt, count)
+// table in the scan's last block (which has no tile unless there are as many regions
+// as the grid was sized for).
+__global__ __launch_bounds__(kThreads) void k_region_scan(Launch<RegionArgs> L) {
+  __shared__ __align__(16) uint8_t lds[kSortMoveLds];
+  const Where w = where(L);
+  const RegionArgs& a = L.args[w.m];
+  if (w.blk < a.sort_blocks) {
+    ph_sort_move(a.sort.global(), Where{w.m, w.blk, a.sort_blocks}, lds);
+    return;
+  }
+  if (w.blk + 1 == w.nblk) build_ptable(a.pt.global(), reinterpret_cast<uint32_t*>(lds));
+  ph_scan_down2(a.scan.global(), Where{w.m, w.blk - a.sort_blocks, w.nblk - a.sort_blocks}, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -3046,8 +3060,7 @@ static void prepare_member(Member& M, hipStream_t st) {
   }
 }
 
-// have_sums: the tile sums are written already.
-static void add_scan(Ops& ops, ArenaImage& img, const std::vector<ScanSeg>& segs, bool have_sums = false) {
+static void add_scan(Ops& ops, ArenaImage& img, const std::vector<ScanSeg>& segs) {
   if (segs.empty()) return;
   std::vector<uint32_t> tiles, ones(segs.size(), 1);
   if (std::all_of(segs.begin(), segs.end(), [](const ScanSeg& s) { return s.count_max <= kScanOneMax; })) {
@@ -3056,7 +3069,7 @@ static void add_scan(Ops& ops, ArenaImage& img, const std::vector<ScanSeg>& segs
   }
   for (const auto& s : segs) tiles.push_back(std::max<uint32_t>(1, std::min<uint32_t>(512, (s.count_max + kScanTile - 1) / kScanTile)));
   const LaunchRec rt = img.add(segs, tiles);
-  if (!have_sums) ops.add<ScanSeg>(10, rt, [](Launch<ScanSeg> L, uint32_t g, hipStream_t st) { k_scan_reduce<<<g, kThreads, 0, st>>>(L); });
+  ops.add<ScanSeg>(10, rt, [](Launch<ScanSeg> L, uint32_t g, hipStream_t st) { k_scan_reduce<<<g, kThreads, 0, st>>>(L); });
   ops.add<ScanSeg>(14, rt, [](Launch<ScanSeg> L, uint32_t g, hipStream_t st) { k_scan_down2<<<g, kThreads, 0, st>>>(L); });
 }
 
@@ -3269,28 +3282,35 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
     }
     ops.add<RootArgs>(50, img.add(ra, rb), [](Launch<RootArgs> L, uint32_t g, hipStream_t st) { k_scatter_roots<<<g, kThreads, 0, st>>>(L); });
   }
-  // 6. shifted entries: source checkpoint, stable sort by source, (chkpt, count) table
+  // 6. shifted entries: source checkpoint, stable sort by source, (chkpt, count) table;
+  // region sizes and offsets
   std::vector<const uint64_t*> sorted(B);
   {
-    std::vector<ShiftArgs> sa;
-    std::vector<uint32_t> sb;
+    std::vector<RegionArgs> ra;
+    std::vector<uint32_t> ib, sb;
     uint32_t max_passes = 0;
     for (size_t i = 0; i < B; i++) {
       Member& M = ms[i];
       mtc_dedup* h = M.h;
-      // k_shift_src counts the first pass's digits per sort block itself when its
+      // k_root_info counts the first pass's digits per sort block itself when its
       // histogram of sources is in LDS (fewer than kLdsBins checkpoints since the
       // baseline): one launch fewer.
       const bool fold = M.passes > 0 && M.nbins <= kLdsBins;
-      sa.push_back(ShiftArgs{h->shift_tmp.p, &h->ctl_d->S, h->leaf_slot.p, M.n, h->table.p, h->table_cap - 1, h->baseline_id, M.cur,
-                             h->sort_key[0].p, h->sort_val[0].p, h->src_hist.p, M.nbins, h->ctl_d,
-                             fold ? h->sort_hist.p : nullptr, fold ? digits0(M.nbins) : 0u});
-      sb.push_back(M.Gs);
+      const ShiftArgs sa{h->shift_tmp.p, &h->ctl_d->S, h->leaf_slot.p, M.n, h->table.p, h->table_cap - 1, h->baseline_id, M.cur,
+                         h->sort_key[0].p, h->sort_val[0].p, h->src_hist.p, M.nbins, h->ctl_d,
+                         fold ? h->sort_hist.p : nullptr, fold ? digits0(M.nbins) : 0u};
+      const ScanSeg sc{h->region_off.p, h->region_off.p, &h->ctl_d->F, M.n, h->region_off.p + M.n, M.ws_reg,
+                       nullptr, h->tile_lo.p};
+      ra.push_back(RegionArgs{h->first_roots.p, &h->ctl_d->F, M.g, h->region_off.p, h->compat,
+                              PtableArgs{h->src_hist.p, M.nbins, h->baseline_id, h->ptable.p, h->ctl_d}, sa, SortArgs{}, sc,
+                              M.Gs, M.passes ? M.Gs : 0u});
+      ib.push_back(M.Gs + grid_for(M.n, 2 * kScanTile, 512));
+      sb.push_back((M.passes ? M.Gs : 0u) + grid_for(M.n, kScanTile, 512));
       max_passes = std::max(max_passes, M.passes);
       sorted[i] = h->sort_val[M.passes % 2].p;
     }
-    ops.add<ShiftArgs>(60, img.add(sa, sb), [](Launch<ShiftArgs> L, uint32_t g, hipStream_t st) { k_shift_src<<<g, kThreads, 0, st>>>(L); });
-    for (uint32_t p = 0; p < max_passes; p++) {
+    ops.add<RegionArgs>(60, img.add(ra, ib), [](Launch<RegionArgs> L, uint32_t g, hipStream_t st) { k_root_info<<<g, kThreads, 0, st>>>(L); });
+    for (uint32_t p = 0; p < std::max(max_passes, 1u); p++) {
       std::vector<SortArgs> so;
       std::vector<uint32_t> sblk, cblk;
       std::vector<ScanSeg> hs;
@@ -3304,30 +3324,21 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
         so.push_back(SortArgs{h->sort_key[p % 2].p, h->sort_val[p % 2].p, h->sort_key[1 - p % 2].p,
                               h->sort_val[1 - p % 2].p, &h->ctl_d->S, shift, nb, h->sort_hist.p, raw ? 1u : 0u});
         sblk.push_back(p < M.passes ? M.Gs : 0u);
-        cblk.push_back(p < M.passes && !(p == 0 && M.nbins <= kLdsBins) ? M.Gs : 0u);  // else counted by k_shift_src
+        cblk.push_back(p < M.passes && !(p == 0 && M.nbins <= kLdsBins) ? M.Gs : 0u);  // else counted by k_root_info
         if (p < M.passes && !raw) hs.push_back(ScanSeg{h->sort_hist.p, h->sort_hist.p, nullptr, nb * M.Gs, nullptr, M.ws_sort});
       }
-      const LaunchRec r = img.add(so, sblk), rc = img.add(so, cblk);
-      ops.add<SortArgs>(61, rc, [](Launch<SortArgs> L, uint32_t g, hipStream_t st) { k_sort_count<<<g, kThreads, 0, st>>>(L); });
+      ops.add<SortArgs>(61, img.add(so, cblk), [](Launch<SortArgs> L, uint32_t g, hipStream_t st) { k_sort_count<<<g, kThreads, 0, st>>>(L); });
       add_scan(ops, img, hs);
-      ops.add<SortArgs>(62, r, [](Launch<SortArgs> L, uint32_t g, hipStream_t st) { k_sort_move<<<g, kThreads, 0, st>>>(L); });
+      if (p == 0) {
+        for (size_t i = 0; i < B; i++) ra[i].sort = so[i];
+        ops.add<RegionArgs>(70, img.add(ra, sb), [](Launch<RegionArgs> L, uint32_t g, hipStream_t st) { k_region_scan<<<g, kThreads, 0, st>>>(L); });
+      } else {
+        ops.add<SortArgs>(62, img.add(so, sblk), [](Launch<SortArgs> L, uint32_t g, hipStream_t st) { k_sort_move<<<g, kThreads, 0, st>>>(L); });
+      }
     }
   }
-  // 7. region sizes and offsets, metadata, gathered data, counters
+  // 7. metadata, gathered data, counters
   {
-    std::vector<RegionArgs> ra;
-    std::vector<uint32_t> rb;
-    std::vector<ScanSeg> ss;
-    for (auto& M : ms) {
-      mtc_dedup* h = M.h;
-      ra.push_back(RegionArgs{h->first_roots.p, &h->ctl_d->F, M.g, h->region_off.p, h->compat,
-                              PtableArgs{h->src_hist.p, M.nbins, h->baseline_id, h->ptable.p, h->ctl_d}, M.ws_reg});
-      rb.push_back(grid_for(M.n, 16 * kThreads, 512));
-      ss.push_back(ScanSeg{h->region_off.p, h->region_off.p, &h->ctl_d->F, M.n, h->region_off.p + M.n, M.ws_reg,
-                           nullptr, h->tile_lo.p});
-    }
-    ops.add<RegionArgs>(70, img.add(ra, rb), [](Launch<RegionArgs> L, uint32_t g, hipStream_t st) { k_region_sizes<<<g, kThreads, 0, st>>>(L); });
-    add_scan(ops, img, ss, true);
     std::vector<DiffArgs> da;
     std::vector<uint32_t> gb;
     for (size_t i = 0; i < B; i++) {

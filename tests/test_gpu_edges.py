@@ -270,3 +270,23 @@ def test_diff_copies_to_device_memory():
             assert got.cpu().numpy().tobytes() == want
             assert (o[:16 + off] == 0x5A).all() and (o[16 + off + len(want):] == 0x5A).all()
         d.close()
+
+
+@pytest.mark.parametrize("n", [3000, 36_000])
+def test_shifted_chunks_of_many_checkpoints(n):
+    """Shifted entries of one, a few and more than 256 sources (none, one and two sort
+    passes; their counts added up by the sort's blocks or scanned first), beside the
+    scan of the region sizes."""
+    C, rng = 16, np.random.default_rng(n)
+    cur = rng.integers(0, 256, (n, C), dtype=np.uint8)
+    fresh, versions = [cur[:50].copy()], [cur.reshape(-1).copy()]
+    for k in range(1, 290):
+        new = rng.integers(0, 256, (20, C), dtype=np.uint8)
+        cur[rng.choice(n, 20, replace=False)] = new
+        fresh.append(new)
+        if k in (2, 5, 40, 270, 289):  # chunks of every earlier checkpoint, at new places
+            bank = np.concatenate(fresh)
+            to = rng.choice(n, n // 3, replace=False)
+            cur[to] = bank[rng.integers(0, len(bank), len(to))]
+        versions.append(cur.reshape(-1).copy())
+    same_as_oracle(versions, C)
