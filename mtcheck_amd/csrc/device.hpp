@@ -137,7 +137,16 @@ __host__ __device__ __forceinline__ uint32_t rotl32(uint32_t x, int s) { return 
 
 #define MTC_MD5_F(x, y, z) (((x) & (y)) | (~(x) & (z)))
 #define MTC_MD5_G(x, y, z) (((x) & (z)) | ((y) & ~(z)))
-#define MTC_MD5_H(x, y, z) ((x) ^ (y) ^ (z))
+// One three-input operation on the device: left to itself the compiler shares an xor
+// between two steps and spends three operations on them.
+__host__ __device__ __forceinline__ uint32_t xor3(uint32_t x, uint32_t y, uint32_t z) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return (uint32_t)__builtin_amdgcn_bitop3_b32((int)x, (int)y, (int)z, 0x96);
+#else
+  return x ^ y ^ z;
+#endif
+}
+#define MTC_MD5_H(x, y, z) xor3(x, y, z)
 #define MTC_MD5_I(x, y, z) ((y) ^ ((x) | ~(z)))
 #define MTC_MD5_STEP(f, a, b, c, d, x, t, s) \
   a += f(b, c, d) + (x) + (t);               \
