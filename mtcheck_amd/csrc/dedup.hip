@@ -1048,20 +1048,30 @@ __global__ __launch_bounds__(kThreads) void k_insert(Launch<DenseArgs> L) {
   ph_insert(L, where(L), nullptr);
 }
 
-// The chunks k_insert left for k_fixmin and k_resolve.  A wavefront takes 64
-// groups of the dense list at a time (one count per lane), ranks their entries with
+// The chunks k_insert left for k_fixmin and k_resolve.  A wavefront takes G groups of
+// 64 entries of the dense list at a time (one count per lane), ranks their entries with
 // a wave scan and gives each lane one entry per round: lane e of a round finds its
 // group by bisection over the exclusive prefix, so every lane has work whether the
 // entries sit in few groups or many.  f(valid, chunk) is called by whole wavefronts.
-constexpr uint32_t kPendPerBlock = (kThreads / 64) * 64 * 64;  // dense entries per block and pass
+//
+// The grid is sized for 64 groups a wavefront of a baseline's full list.  A later list
+// is shorter, and each round is a chain of loads from anywhere, so G is the least that
+// lets the grid take the list at once: at 1 GiB in 64-byte chunks and 20% change
+// k_fixmin 17.6 us and k_resolve 9.7 us (30.0 and 14.4 with 64 groups always), at
+// 64 MiB in 128-byte chunks and 3% 5.2 and 3.5 (6.8 and 3.9).  Eight groups always and
+// eight times the blocks: 14.2 and 9.1 us there, but 48 and 23 us instead of 33 and 15
+// for a 4 GiB baseline, most of whose groups are empty.
+constexpr uint32_t kPendPerBlock = (kThreads / 64) * 64 * 64;  // dense entries per block
 template <class F>
 __device__ __forceinline__ void for_pending(const DenseArgs& a, const Where& w, F&& f) {
   const uint32_t lane = lane_id();
   const uint64_t groups = ((uint64_t)*a.total + 63) / 64;
   const uint64_t wave = ((uint64_t)w.blk * kThreads + threadIdx.x) >> 6;
   const uint64_t waves = ((uint64_t)w.nblk * kThreads) >> 6;
-  for (uint64_t g0 = wave * 64; g0 < groups; g0 += waves * 64) {
-    const uint32_t cnt = g0 + lane < groups ? a.pcnt[g0 + lane] : 0u;
+  uint32_t G = 4;  // at least: a round fills a wavefront's lanes
+  while (G < 64 && G * waves < groups) G *= 2;
+  for (uint64_t g0 = wave * G; g0 < groups; g0 += waves * G) {
+    const uint32_t cnt = lane < G && g0 + lane < groups ? a.pcnt[g0 + lane] : 0u;
     uint32_t x = cnt;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
