@@ -809,8 +809,25 @@ __device__ __forceinline__ void leaf1_tile(const LeafArgs& a, uint32_t blk, uint
   const uint32_t lane = lane_id();
   const uint64_t m = __ballot(ins);
   uint32_t base = 0;
-  if (lane == 0 && m) base = atomicAdd(a.blk_cnt + blk, (uint32_t)__popcll(m));
-  base = __shfl(base, 0);
+  if (a.list_dg) {
+    if (lane == 0 && m) base = atomicAdd(a.blk_cnt + blk, (uint32_t)__popcll(m));
+    base = __shfl(base, 0);
+  } else {
+    // The basic approach's diff is the list: ascending, so the wavefronts' runs follow
+    // each other.  (The staged bytes are done with; 16 bytes of LDS more would cost
+    // one block of five.)
+    uint32_t* cnt = reinterpret_cast<uint32_t*>(lds);
+    __syncthreads();
+    if (lane == 0) cnt[tid / 64] = __popcll(m);
+    __syncthreads();
+    uint32_t total = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kThreads / 64; w++) {
+      if (w < tid / 64) base += cnt[w];
+      total += cnt[w];
+    }
+    if (tid == 0) a.blk_cnt[blk] = total;
+  }
   if (ins) {
     // A baseline lists every chunk: in its own place (list is the dense list).
     const uint64_t k = a.baseline ? c : t * kThreads + base + __popcll(m & ((1ull << lane) - 1));
@@ -3443,7 +3460,7 @@ struct DirectLeaf {
   Prologue pro{};
 };
 
-static bool lean_leaf(const Member& M) { return M.cb >= 16 && M.tpb == 1 && M.h->approach != MTC_APPROACH_BASIC; }
+static bool lean_leaf(const Member& M) { return M.cb >= 16 && M.tpb == 1; }
 
 static void build_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img, int phase, bool leaf_scan,
                       DirectLeaf* direct = nullptr) {

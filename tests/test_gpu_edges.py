@@ -290,3 +290,26 @@ def test_shifted_chunks_of_many_checkpoints(n):
             cur[to] = bank[rng.integers(0, len(bank), len(to))]
         versions.append(cur.reshape(-1).copy())
     same_as_oracle(versions, C)
+
+
+@pytest.mark.parametrize("hk", [M.MURMUR3, M.MD5])
+@pytest.mark.parametrize("C,n", [(16, 1), (128, 255), (32, 256), (64, 257), (128, 70_001), (512, 3000), (4096, 300)])
+def test_basic_lists_are_ascending(C, n, hk):
+    """The basic approach's lists from leaf blocks of one tile: no, one, few and all
+    chunks of a block changed, in one and in several of its wavefronts."""
+    rng = np.random.default_rng(C * n)
+    v = [rng.integers(0, 256, n * C - 3, dtype=np.uint8)]
+    for frac in (0.0, 0.01, 0.5, 1.0):
+        w = v[-1].copy()
+        for c in np.nonzero(rng.random(n) < frac)[0]:
+            w[c * C] ^= 1
+        v.append(w)
+    w = v[-1].copy()
+    w[-1] ^= 1
+    v.append(w)
+    d, orc = M.TreeDeduplicator(C, M.BASIC, hash_kind=hk), O.OracleBasic(C, hk)
+    for k, host in enumerate(v):
+        g = d.checkpoint(torch.from_numpy(host).to("cuda:0"), make_baseline=(k == 0))
+        e = orc.checkpoint(host, make_baseline=(k == 0))
+        assert g == e, (k, first_mismatch(g, e))
+    d.close()
