@@ -545,8 +545,8 @@ __device__ __forceinline__ Digest tile_digest(const uint8_t* data, uint64_t len,
 // The previous checkpoint's digest of this lane's chunk in tile t (zero after a
 // reset).  Callers issue it with the tile's data loads so that its latency hides
 // behind theirs.
-__device__ __forceinline__ Digest leaf_prev(const LeafArgs& a, uint64_t t) {
-  const uint64_t c = t * kThreads + threadIdx.x;
+__device__ __forceinline__ Digest leaf_prev(const LeafArgs& a, uint64_t t, uint32_t tid) {
+  const uint64_t c = t * kThreads + tid;
   if (c >= a.n || a.baseline) return Digest{0, 0};
   const uint4 v = ld_stream16(a.leaf_dg + c);
   return Digest{(uint64_t)v.x | ((uint64_t)v.y << 32), (uint64_t)v.z | ((uint64_t)v.w << 32)};
@@ -598,7 +598,7 @@ __global__ __launch_bounds__(kThreads, CB ? 1 : 3) void k_leaf(Launch<LeafArgs> 
   uint32_t run = 0;
   if constexpr (CB <= 0) {
     for (uint64_t t = t0; t < t1; t++) {
-      const Digest pv = leaf_prev(a, t);
+      const Digest pv = leaf_prev(a, t, threadIdx.x);
       leaf_epilogue(a, t, tile_digest<HK, CB>(a.data, a.len, a.n, a.C, t), pv, region, run, s_wcnt);
     }
   } else {
@@ -623,7 +623,7 @@ __global__ __launch_bounds__(kThreads, CB ? 1 : 3) void k_leaf(Launch<LeafArgs> 
     Digest pv{0, 0};  // previous digest of this lane's chunk in the current tile
     if (steps) {
       load(0, v);
-      pv = leaf_prev(a, t0);
+      pv = leaf_prev(a, t0, tid);
     }
     uint64_t h1 = 0, h2 = 0;
     uint32_t st[4], X[16];
@@ -632,7 +632,7 @@ __global__ __launch_bounds__(kThreads, CB ? 1 : 3) void k_leaf(Launch<LeafArgs> 
       Digest npv = pv;
       if (step + 1 < steps) {
         load(step + 1, nv);
-        if ((step + 1) % S::PASSES == 0) npv = leaf_prev(a, t0 + (step + 1) / S::PASSES);
+        if ((step + 1) % S::PASSES == 0) npv = leaf_prev(a, t0 + (step + 1) / S::PASSES, tid);
       }
       __syncthreads();  // the previous segment's LDS reads are done
 #pragma unroll
@@ -785,15 +785,15 @@ __device__ __forceinline__ Digest lean_digest(const uint8_t* data, uint64_t firs
   return h.finish();
 }
 
-template <int HK, int CB>
-__device__ __forceinline__ void leaf1_tile(const LeafArgs& a, uint32_t blk, uint8_t* lds) {
+// Thread `tid` of tile blk's 256; WAVE: its wavefront is a block of its own.
+template <int HK, int CB, bool WAVE>
+__device__ __forceinline__ void leaf1_tile(const LeafArgs& a, uint32_t blk, uint32_t tid, uint8_t* lds) {
   static_assert(CB >= 16 && (CB & (CB - 1)) == 0, "power-of-two chunk size");
-  if (a.stamp && blk == 0 && threadIdx.x == 0) *a.stamp = wall_clock64();
+  if (a.stamp && blk == 0 && tid == 0) *a.stamp = wall_clock64();
   const uint64_t t = blk;
   const uint64_t full = a.len / CB;
-  const uint32_t tid = threadIdx.x;
-  const Digest pv = leaf_prev(a, t);
-  Digest d = lean_digest<HK, CB, false>(a.data, t * kThreads, full, lds);
+  const Digest pv = leaf_prev(a, t, tid);
+  Digest d = lean_digest<HK, CB, WAVE>(a.data, t * kThreads + (WAVE ? tid & ~63u : 0u), full, lds);
   const uint64_t c = t * kThreads + tid;
   if (c >= full) d = (c < a.n) ? hash_bytes<HK>(a.data + c * CB, a.len - c * CB) : Digest{0, 0};
   const bool valid = c < a.n;
@@ -809,7 +809,7 @@ __device__ __forceinline__ void leaf1_tile(const LeafArgs& a, uint32_t blk, uint
   const uint32_t lane = lane_id();
   const uint64_t m = __ballot(ins);
   uint32_t base = 0;
-  if (a.list_dg) {
+  if (WAVE || a.list_dg) {
     if (lane == 0 && m) base = atomicAdd(a.blk_cnt + blk, (uint32_t)__popcll(m));
     base = __shfl(base, 0);
   } else {
@@ -840,7 +840,7 @@ template <int HK, int CB>
 __global__ __launch_bounds__(kThreads, 5) void k_leaf1(Launch<LeafArgs> L) {
   __shared__ __align__(16) uint8_t lds[kThreads * (CB < 128 ? CB : 128)];
   const Where wh = where(L);
-  leaf1_tile<HK, CB>(L.args[wh.m].global(), wh.blk, lds);
+  leaf1_tile<HK, CB, false>(L.args[wh.m].global(), wh.blk, threadIdx.x, lds);
 }
 
 // The same kernel for a step of one member, started before anything else of the
@@ -852,19 +852,38 @@ __global__ __launch_bounds__(kThreads, 5) void k_leaf1(Launch<LeafArgs> L) {
 // (Spread over every block, the same work made the kernel 3% slower: each block
 // read the fill list before its loads.)
 constexpr uint32_t kPrologueBlocks = 64;
+// A thread's part of the prologue: thread gt of gs.
+__device__ __forceinline__ void leaf_prologue(const Prologue& p, uint64_t gt, uint64_t gs) {
+  for (uint64_t i = gt; i < p.n16; i += gs) p.dst[i] = p.src[i];
+  for (uint32_t f = 0; f < p.nfill; f++) {
+    const FillSeg s = p.fill[f].global();
+    for (uint64_t i = gt; i < s.count; i += gs) s.p[i] = s.v;
+  }
+}
+
 template <int HK, int CB>
 __global__ __launch_bounds__(kThreads, 5) void k_leaf1_direct(LeafArgs a, Prologue p) {
   __shared__ __align__(16) uint8_t lds[kThreads * (CB < 128 ? CB : 128)];
-  if (blockIdx.x < kPrologueBlocks) {
-    const uint64_t gt = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
-    const uint64_t gs = (uint64_t)min(gridDim.x, kPrologueBlocks) * kThreads;
-    for (uint64_t i = gt; i < p.n16; i += gs) p.dst[i] = p.src[i];
-    for (uint32_t f = 0; f < p.nfill; f++) {
-      const FillSeg s = p.fill[f].global();
-      for (uint64_t i = gt; i < s.count; i += gs) s.p[i] = s.v;
-    }
-  }
-  leaf1_tile<HK, CB>(a.global(), blockIdx.x, lds);
+  if (blockIdx.x < kPrologueBlocks)
+    leaf_prologue(p, (uint64_t)blockIdx.x * kThreads + threadIdx.x, (uint64_t)min(gridDim.x, kPrologueBlocks) * kThreads);
+  leaf1_tile<HK, CB, false>(a.global(), blockIdx.x, threadIdx.x, lds);
+}
+
+// The same by blocks of one wavefront, four to a tile (a grid of tiles x 4, taken in
+// dispatch order), for the largest staged chunks of a tree: 256 rows 4096 bytes apart
+// that march in step through their 128-byte pieces meet in the same memory channels,
+// and 64 rows less so.  4 GiB with few changes 805 -> 743 us, 2 GiB 410 -> 391 us; at
+// 2048 bytes and below the blocks of 256 threads are the faster ones (2 GiB: 2048 bytes
+// 332 against 349 us, 512 bytes 339 against 364).  A basic list's order needs the
+// tile's wavefronts together.
+constexpr uint32_t kTileWaves = kThreads / 64;
+template <int HK, int CB>
+__global__ __launch_bounds__(64, 4) void k_leaf1_direct_wave(LeafArgs a, Prologue p) {
+  __shared__ __align__(16) uint8_t lds[64 * 128];
+  const uint32_t b = blockIdx.y * gridDim.x + blockIdx.x;
+  constexpr uint32_t pb = kPrologueBlocks * kTileWaves;
+  if (b < pb) leaf_prologue(p, (uint64_t)b * 64 + threadIdx.x, (uint64_t)min(gridDim.x * kTileWaves, pb) * 64);
+  leaf1_tile<HK, CB, true>(a.global(), b / kTileWaves, b % kTileWaves * 64 + threadIdx.x, lds);
 }
 
 // Concatenate the per-block regions into the dense list of chunks to insert.
@@ -2616,7 +2635,10 @@ static void launch_leaf1_direct(int cb, const LeafArgs& a, const Prologue& p, ui
     case 512: k_leaf1_direct<HK, 512><<<grid, kThreads, 0, st>>>(a, p); break;
     case 1024: k_leaf1_direct<HK, 1024><<<grid, kThreads, 0, st>>>(a, p); break;
     case 2048: k_leaf1_direct<HK, 2048><<<grid, kThreads, 0, st>>>(a, p); break;
-    default: k_leaf1_direct<HK, 4096><<<grid, kThreads, 0, st>>>(a, p); break;
+    default:
+      if (a.list_dg) k_leaf1_direct_wave<HK, 4096><<<dim3(grid, kTileWaves), 64, 0, st>>>(a, p);
+      else k_leaf1_direct<HK, 4096><<<grid, kThreads, 0, st>>>(a, p);
+      break;
   }
 }
 

@@ -313,3 +313,19 @@ def test_basic_lists_are_ascending(C, n, hk):
         e = orc.checkpoint(host, make_baseline=(k == 0))
         assert g == e, (k, first_mismatch(g, e))
     d.close()
+
+
+@pytest.mark.parametrize("hk", [M.MURMUR3, M.MD5])
+@pytest.mark.parametrize("n,tail", [(1, 0), (64, 0), (65, 4095), (255, 1), (256, 0), (257, 77), (5000, 100)])
+def test_series_of_large_chunks(n, tail, hk):
+    """Leaf tiles hashed by blocks of one wavefront: part of a tile's wavefronts, all,
+    several tiles, with and without a short last chunk."""
+    C, rng = 4096, np.random.default_rng(n)
+    v = [rng.integers(0, 256, n * C + tail, dtype=np.uint8)]
+    for frac in (0.0, 0.02, 0.7, 0.01):
+        w = v[-1].copy()
+        for c in np.nonzero(rng.random(n) < frac)[0]:
+            w[c * C + 17] ^= 5
+        w[-1] ^= 1 if frac else 0
+        v.append(w)
+    same_as_oracle(v, C, hk)
