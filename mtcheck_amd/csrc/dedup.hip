@@ -1104,7 +1104,7 @@ __device__ __forceinline__ void for_pending(const DenseArgs& a, const Where& w, 
   const uint64_t groups = ((uint64_t)*a.total + 63) / 64;
   const uint64_t wave = ((uint64_t)w.blk * kThreads + threadIdx.x) >> 6;
   const uint64_t waves = ((uint64_t)w.nblk * kThreads) >> 6;
-  uint32_t G = 4;  // at least: a round fills a wavefront's lanes
+  uint32_t G = 16;  // at least: fewer gain a small list nothing and cost a large batch
   while (G < 64 && G * waves < groups) G *= 2;
   for (uint64_t g0 = wave * G; g0 < groups; g0 += waves * G) {
     const uint32_t cnt = lane < G && g0 + lane < groups ? a.pcnt[g0 + lane] : 0u;
@@ -3353,8 +3353,13 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
       ra.push_back(RegionArgs{h->first_roots.p, &h->ctl_d->F, M.g, h->region_off.p, h->compat,
                               PtableArgs{h->src_hist.p, M.nbins, h->baseline_id, h->ptable.p, h->ctl_d}, sa, SortArgs{}, sc,
                               M.Gs, M.passes ? M.Gs : 0u});
-      ib.push_back(M.Gs + grid_for(M.n, 2 * kScanTile, 512));
-      sb.push_back((M.passes ? M.Gs : 0u) + grid_for(M.n, kScanTile, 512));
+      // Blocks for the regions: a baseline has up to one per chunk, a later checkpoint
+      // rarely one per eight chunks (its blocks loop if it has more; empty blocks cost
+      // a large batch: 256 buffers, 23 GiB, 115 and 106 us for the two launches with a
+      // baseline's blocks throughout, 109 and 73 us so).
+      const uint32_t per = M.baseline ? kScanTile : 8 * kScanTile;
+      ib.push_back(M.Gs + grid_for(M.n, 2 * per, 512));
+      sb.push_back((M.passes ? M.Gs : 0u) + grid_for(M.n, per, 512));
       max_passes = std::max(max_passes, M.passes);
       sorted[i] = h->sort_val[M.passes % 2].p;
     }
