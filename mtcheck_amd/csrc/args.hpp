@@ -149,7 +149,7 @@ struct DenseArgs {
   uint8_t* tile_busy;   // per stage-0 tile: holds a leaf that is not a fixed duplicate
   const Digest* dense_dg;  // the listed chunks' digests, in dense order (a baseline: leaf_dg)
   int leaf_labels;         // the leaf kernel labelled the chunks (otherwise they count as pending)
-  uint32_t* pend;          // k_insert lists the chunks k_fixmin and k_resolve visit, each group of
+  uint32_t* pend;          // k_insert lists the chunks k_fixmin visits, each group of
                            // 64 dense entries at the front of its own 64 words ...
   uint8_t* pcnt;           // ... and counts them per group (ceil(n / 64) bytes)
   __device__ DenseArgs global() const {

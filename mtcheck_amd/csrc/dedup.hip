@@ -998,7 +998,7 @@ __device__ __forceinline__ uint64_t chunk_tile(const Geo& g, uint32_t R0, uint64
 
 // Table inserts (src/tree_approach.cpp:320-349; include/reference_impl.hpp:51): the
 // packed value (cur << 32 | leaf) with atomicMin leaves the lowest leaf of a new
-// digest in the table, and leaves an earlier checkpoint's entry as it is (k_resolve
+// digest in the table, and leaves an earlier checkpoint's entry as it is (sweep A
 // then labels the leaf a shifted duplicate).  Each probe reads the slot's sector
 // before any claim: a digest already in the table costs loads only, which matters
 // for digests that many changed chunks share (a copied zero chunk), where claim-
@@ -1043,9 +1043,9 @@ __device__ __forceinline__ void ph_insert(const Launch<DenseArgs>& L, const Wher
       // only the stage-0 tiles flagged here.
       if (a.R0) a.tile_busy[chunk_tile(a.g, a.R0, c)] = 1;
     }
-    // Decided here, so k_resolve skips them: a follower's leaf is above its head's,
+    // Decided here, so sweep A need not: a follower's leaf is above its head's,
     // so it never holds the minimum, and an entry of an earlier checkpoint keeps
-    // its value.  A zero digest is left to k_resolve: after a reset it may belong
+    // its value.  A zero digest is left to sweep A: after a reset it may belong
     // to a fixed leaf, whose label stays.  When the leaf kernel labelled nothing,
     // every listed chunk is a changed one (pending) until labelled here.
     const bool nz = (d.lo | d.hi) != 0;
@@ -1065,7 +1065,7 @@ __device__ __forceinline__ void ph_insert(const Launch<DenseArgs>& L, const Wher
     }
     if (nl >= 0) a.labels[c] = (uint8_t)nl;
     // Only entries marked for a min or still pending (a zero digest, a failed
-    // probe, or a leaf kernel's label kept) need k_fixmin and k_resolve.  A wave
+    // probe, or a leaf kernel's label kept) need k_fixmin or sweep A.  A wave
     // lists them at the front of its own 64 words and counts them per group, so
     // no counter is shared between wavefronts (one returning atomic add per
     // wavefront on a single counter made k_insert 1.96 ms instead of 1.11 ms at 20%
@@ -1073,7 +1073,10 @@ __device__ __forceinline__ void ph_insert(const Launch<DenseArgs>& L, const Wher
     const bool later = v && (nl < 0 || nl == L_PENDING || nl == L_MIN_PENDING || nl == L_MIN_FIXED);
     const uint64_t pm = __ballot(later);
     if (lane == 0) a.pcnt[wbase >> 6] = (uint8_t)__popcll(pm);
-    if (later) a.pend[wbase + __popcll(pm & ((1ull << lane) - 1))] = c;
+    if (later) {
+      a.pend[wbase + __popcll(pm & ((1ull << lane) - 1))] = c;
+      if (a.R0) a.tile_first[chunk_tile(a.g, a.R0, c)] = 1;  // sweep A decides it there
+    }
     claims += claimed;
   }
   const uint32_t wc = wave_sum(claims);
@@ -1084,7 +1087,7 @@ __global__ __launch_bounds__(kThreads) void k_insert(Launch<DenseArgs> L) {
   ph_insert(L, where(L), nullptr);
 }
 
-// The chunks k_insert left for k_fixmin and k_resolve.  A wavefront takes G groups of
+// The chunks k_insert left undecided, for k_fixmin.  A wavefront takes G groups of
 // 64 entries of the dense list at a time (one count per lane), ranks their entries with
 // a wave scan and gives each lane one entry per round: lane e of a round finds its
 // group by bisection over the exclusive prefix, so every lane has work whether the
@@ -1093,10 +1096,9 @@ __global__ __launch_bounds__(kThreads) void k_insert(Launch<DenseArgs> L) {
 // The grid is sized for 64 groups a wavefront of a baseline's full list.  A later list
 // is shorter, and each round is a chain of loads from anywhere, so G is the least that
 // lets the grid take the list at once: at 1 GiB in 64-byte chunks and 20% change
-// k_fixmin 17.6 us and k_resolve 9.7 us (30.0 and 14.4 with 64 groups always), at
-// 64 MiB in 128-byte chunks and 3% 5.2 and 3.5 (6.8 and 3.9).  Eight groups always and
-// eight times the blocks: 14.2 and 9.1 us there, but 48 and 23 us instead of 33 and 15
-// for a 4 GiB baseline, most of whose groups are empty.
+// k_fixmin 17.6 us (30.0 with 64 groups always), at 64 MiB in 128-byte chunks and 3%
+// 5.2 (6.8).  Eight groups always and eight times the blocks: 14.2 us there, but 48 us
+// instead of 33 for a 4 GiB baseline, most of whose groups are empty.
 constexpr uint32_t kPendPerBlock = (kThreads / 64) * 64 * 64;  // dense entries per block
 template <class F>
 __device__ __forceinline__ void for_pending(const DenseArgs& a, const Where& w, F&& f) {
@@ -1132,7 +1134,7 @@ __device__ __forceinline__ void for_pending(const DenseArgs& a, const Where& w, 
 // matched an entry of this checkpoint (digests that several changed chunks share).
 // The first match below the entry's holder sees the holder's value and relabels it
 // a shifted duplicate (a claimer is labelled first by k_insert); later, lower
-// matches do the same to the match they displace, whose own label k_resolve then
+// matches do the same to the match they displace, whose own label sweep A then
 // decides from the final value either way.  Fixed leaves keep their label.
 //
 // Atomics on one address run one after the other (about 13 ns each), and after a
@@ -1182,25 +1184,6 @@ __device__ __forceinline__ void ph_fixmin(const Launch<DenseArgs>& L, const Wher
 
 __global__ __launch_bounds__(kThreads) void k_fixmin(Launch<DenseArgs> L) {
   ph_fixmin(L, where(L), nullptr);
-}
-
-// Once every insert has landed: a pending leaf is FIRST when its digest's entry is
-// (cur, itself), SHIFT otherwise (include/reference_impl.hpp:52-69).
-__device__ __forceinline__ void ph_resolve(const Launch<DenseArgs>& L, const Where& w, uint8_t* lds) {
-  (void)lds;
-  const DenseArgs a = L.args[w.m].global();
-  for_pending(a, w, [&](bool valid, uint32_t c) {
-    if (!valid || a.labels[c] != L_PENDING) return;  // not pending: a fixed leaf right after a reset
-    const uint32_t s = a.leaf_slot[c];
-    uint8_t l = L_SHIFT;
-    if (s <= a.mask + 1) l = (a.tab[s].val == (((uint64_t)a.cur << 32) | (uint32_t)(a.n - 1 + c))) ? L_FIRST : L_SHIFT;
-    a.labels[c] = l;
-    if (a.R0 && l == L_FIRST) a.tile_first[chunk_tile(a.g, a.R0, c)] = 1;
-  });
-}
-
-__global__ __launch_bounds__(kThreads) void k_resolve(Launch<DenseArgs> L) {
-  ph_resolve(L, where(L), nullptr);
 }
 
 // Standalone chunk hashing (mtc_hash_chunks), by blocks of one wavefront and 64 chunks
@@ -1327,6 +1310,20 @@ struct SweepA {
 };
 
 // One tile of sweep A (the whole wavefront).
+// Once every insert and min has landed: a pending leaf is FIRST when its digest's entry
+// is (cur, itself), SHIFT otherwise (include/reference_impl.hpp:52-69).  The sweep that
+// reads the leaves' labels first decides it: pending leaves are few, their tiles are
+// flagged by k_insert, and a pass of its own was a launch of 3 to 10 us.
+__device__ __forceinline__ uint8_t leaf_label(const SweepArgs& a, uint64_t c) {
+  uint8_t l = a.labels[c];
+  if (l == L_PENDING) {
+    const uint32_t s = a.leaf_slot[c];
+    l = (s <= a.mask + 1 && a.tab[s].val == (((uint64_t)a.cur << 32) | (uint32_t)(a.g.n - 1 + c))) ? L_FIRST : L_SHIFT;
+    a.labels[c] = l;
+  }
+  return l;
+}
+
 template <int HK>
 __device__ __forceinline__ void sweep_a_tile(const SweepArgs& a, uint64_t tile, uint32_t lane, Digest* rec_dg,
                                              uint32_t* rec_node) {
@@ -1342,7 +1339,7 @@ __device__ __forceinline__ void sweep_a_tile(const SweepArgs& a, uint64_t tile, 
     const uint64_t p = base + lp;
     if (a.stage0) {
       if (p >= a.g.m) continue;
-      l0[i] = a.labels[bottom_chunk(a.g, p)];
+      l0[i] = leaf_label(a, bottom_chunk(a.g, p));
     } else {
       l0[i] = a.in_lab[p];
     }
@@ -1364,7 +1361,7 @@ __device__ __forceinline__ void sweep_a_tile(const SweepArgs& a, uint64_t tile, 
       const uint64_t q = (base >> 1) + j;
       if (j >= T / 2 || q < a.g.half) continue;
       const uint64_t c = q - a.g.half;
-      lf[k] = a.labels[c];
+      lf[k] = leaf_label(a, c);
       if (lf[k] == L_FIRST) gf[k] = a.leaf_dg[c];
       any |= (lf[k] == L_FIRST);
     }
@@ -1822,7 +1819,7 @@ __global__ __launch_bounds__(64 * WPB, MTC_SWEEP_B_WAVES) void k_sweep_b(Launch<
 __device__ __forceinline__ void ph_single_leaf(const Launch<SweepArgs>& L, const Where& w) {
   if (threadIdx.x != 0) return;
   const SweepArgs a = L.args[w.m].global();
-  const uint8_t l = a.labels[0];
+  const uint8_t l = leaf_label(a, 0);
   const bool root = a.compat ? l == L_FIRST : is_region(l);
   if (root) a.staging[0] = (l == L_FIRST ? (kFirstTag << 32) : ((uint64_t)a.leaf_slot[0] << 32)) | 0u;
   a.cnt_f[0] = (root && l == L_FIRST) ? 1u : 0u;
@@ -3176,7 +3173,6 @@ static void build_tree_ops(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
     const LaunchRec rd = img.add(da, db), rp = img.add(da, pb);
     ops.add<DenseArgs>(22, rd, [](Launch<DenseArgs> L, uint32_t g, hipStream_t st) { k_insert<<<g, kThreads, 0, st>>>(L); });
     ops.add<DenseArgs>(24, rp, [](Launch<DenseArgs> L, uint32_t g, hipStream_t st) { k_fixmin<<<g, kThreads, 0, st>>>(L); });
-    ops.add<DenseArgs>(23, rp, [](Launch<DenseArgs> L, uint32_t g, hipStream_t st) { k_resolve<<<g, kThreads, 0, st>>>(L); });
   }
   // 4. sweeps: every stage of sweep A (and its inserts) before any stage of sweep B
   {

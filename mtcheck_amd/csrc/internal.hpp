@@ -180,7 +180,7 @@ struct mtc_dedup {
   mtc::DevBuf<uint32_t> dense;        // the same, concatenated
   mtc::DevBuf<mtc::Digest> list_dg;   // tree handles: their digests beside the list entries
   mtc::DevBuf<mtc::Digest> dense_dg;  // and concatenated
-  mtc::DevBuf<uint32_t> pend;         // listed chunks left for k_fixmin / k_resolve
+  mtc::DevBuf<uint32_t> pend;         // listed chunks left for k_fixmin
   mtc::DevBuf<uint8_t> pcnt;          // their number per group of 64 dense entries
   mtc::DevBuf<uint32_t> blk_cnt, blk_off;
   uint64_t blk_zero = 0;             // leading entries of blk_cnt known to be zero (k_compact clears them)

@@ -329,3 +329,23 @@ def test_series_of_large_chunks(n, tail, hk):
         w[-1] ^= 1 if frac else 0
         v.append(w)
     same_as_oracle(v, C, hk)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 257, 300, 777, 5000])
+def test_pending_leaves_decided_by_the_sweep(n):
+    """Leaves whose label is open until every insert has landed (chunks that share
+    digests, zero chunks after a second baseline), on one and on two tree depths."""
+    C, rng = 32, np.random.default_rng(n)
+    bank = rng.integers(0, 256, (3, C), dtype=np.uint8)
+    bank[0] = 0
+    d, orc = M.TreeDeduplicator(C), O.OracleDedup(C, M.MURMUR3)
+    host = bank[rng.integers(0, 3, n)].copy()
+    for k in range(5):
+        if k:
+            at = rng.random(n) < (0.6 if k < 4 else 0.05)
+            host[at] = np.concatenate([bank, rng.integers(0, 256, (2, C), dtype=np.uint8)])[rng.integers(0, 5, int(at.sum()))]
+        flat = host.reshape(-1).copy()
+        g = d.checkpoint(torch.from_numpy(flat).to("cuda:0"), make_baseline=k in (0, 2))
+        e = orc.checkpoint(flat, make_baseline=k in (0, 2))
+        assert g == e, (k, first_mismatch(g, e))
+    d.close()
