@@ -509,7 +509,7 @@ def host_path_runs(series, C: int, hk: int, warmup: int, steps: int, diff_max: i
             d.set_tuning(*tune)
         for k in range(warmup):
             d.checkpoint_device(vs.get(k), make_baseline=(k == 0))
-        if mode == "overlapped":
+        if mode == "overlapped" and d.stats().diff_size <= cap:  # (not a baseline's diff, after one warm-up step)
             d.copy_last_diff_async(pinned[0])
             d.wait_copies()
         torch.cuda.synchronize()
