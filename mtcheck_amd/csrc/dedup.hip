@@ -1314,13 +1314,13 @@ struct SweepA {
 // is (cur, itself), SHIFT otherwise (include/reference_impl.hpp:52-69).  The sweep that
 // reads the leaves' labels first decides it: pending leaves are few, their tiles are
 // flagged by k_insert, and a pass of its own was a launch of 3 to 10 us.
-__device__ __forceinline__ uint8_t leaf_label(const SweepArgs& a, uint64_t c) {
-  uint8_t l = a.labels[c];
-  if (l == L_PENDING) {
-    const uint32_t s = a.leaf_slot[c];
-    l = (s <= a.mask + 1 && a.tab[s].val == (((uint64_t)a.cur << 32) | (uint32_t)(a.g.n - 1 + c))) ? L_FIRST : L_SHIFT;
-    a.labels[c] = l;
-  }
+// (After all of a tile's label loads: decided one by one as they were read, the loads
+// waited for each other, and sweep A lost at 20% change what the pass had cost.)
+__device__ __forceinline__ uint8_t decide_leaf(const SweepArgs& a, uint64_t c) {
+  const uint32_t s = a.leaf_slot[c];
+  const uint64_t me = ((uint64_t)a.cur << 32) | (uint32_t)(a.g.n - 1 + c);
+  const uint8_t l = (s <= a.mask + 1 && a.tab[s].val == me) ? L_FIRST : L_SHIFT;
+  a.labels[c] = l;
   return l;
 }
 
@@ -1339,11 +1339,10 @@ __device__ __forceinline__ void sweep_a_tile(const SweepArgs& a, uint64_t tile, 
     const uint64_t p = base + lp;
     if (a.stage0) {
       if (p >= a.g.m) continue;
-      l0[i] = leaf_label(a, bottom_chunk(a.g, p));
+      l0[i] = a.labels[bottom_chunk(a.g, p)];
     } else {
       l0[i] = a.in_lab[p];
     }
-    any |= (l0[i] == L_FIRST);
   }
   // Digests of positions 4 lane + i, loaded where a pair of first occurrences is
   // hashed (holding all four per lane cost wavefront slots in registers).
@@ -1355,17 +1354,26 @@ __device__ __forceinline__ void sweep_a_tile(const SweepArgs& a, uint64_t tile, 
   uint8_t lf[2] = {L_NONE, L_NONE};
   Digest gf[2];
   if (a.stage0) {
+    auto upper = [&](int k) -> uint64_t { return (base >> 1) + 2 * lane + k - a.g.half; };  // its chunk
 #pragma unroll
     for (int k = 0; k < 2; k++) {
       const uint32_t j = 2 * lane + k;
       const uint64_t q = (base >> 1) + j;
       if (j >= T / 2 || q < a.g.half) continue;
-      const uint64_t c = q - a.g.half;
-      lf[k] = leaf_label(a, c);
-      if (lf[k] == L_FIRST) gf[k] = a.leaf_dg[c];
+      lf[k] = a.labels[upper(k)];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (l0[i] == L_PENDING) l0[i] = decide_leaf(a, bottom_chunk(a.g, base + 4 * lane + i));
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      if (lf[k] == L_PENDING) lf[k] = decide_leaf(a, upper(k));
+      if (lf[k] == L_FIRST) gf[k] = a.leaf_dg[upper(k)];
       any |= (lf[k] == L_FIRST);
     }
   }
+#pragma unroll
+  for (int i = 0; i < 4; i++) any |= (l0[i] == L_FIRST);
   if (!__ballot(any)) {
     if (lane == 0) a.out_lab[tile] = L_NONE;
     return;
@@ -1819,7 +1827,8 @@ __global__ __launch_bounds__(64 * WPB, MTC_SWEEP_B_WAVES) void k_sweep_b(Launch<
 __device__ __forceinline__ void ph_single_leaf(const Launch<SweepArgs>& L, const Where& w) {
   if (threadIdx.x != 0) return;
   const SweepArgs a = L.args[w.m].global();
-  const uint8_t l = leaf_label(a, 0);
+  uint8_t l = a.labels[0];
+  if (l == L_PENDING) l = decide_leaf(a, 0);
   const bool root = a.compat ? l == L_FIRST : is_region(l);
   if (root) a.staging[0] = (l == L_FIRST ? (kFirstTag << 32) : ((uint64_t)a.leaf_slot[0] << 32)) | 0u;
   a.cnt_f[0] = (root && l == L_FIRST) ? 1u : 0u;
