@@ -318,10 +318,12 @@ __device__ __forceinline__ void st_relaxed(uint64_t* p, uint64_t v) {
 // with two stores.  Random stores cost by their number (45-55 G/s, claims 21 G/s): eight
 // checkpoints of 4 GiB (128-byte chunks, 2%), k_insert 3360 -> 2760 us and sweep A
 // 3260 -> 2770 us with one fewer per new entry.
+// The store's data registers must stay as they are for two wait states.  The compiler
+// sees to that for stores of its own; here the s_nop does, whatever follows.
 __device__ __forceinline__ void st_pair(uint64_t* p, uint64_t a, uint64_t b) {
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   const u32x4 x = {(uint32_t)a, (uint32_t)(a >> 32), (uint32_t)b, (uint32_t)(b >> 32)};
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(x) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(x) : "memory");
 }
 __device__ __forceinline__ uint64_t cas_relaxed(uint64_t* p, uint64_t expect, uint64_t desired) {
   __hip_atomic_compare_exchange_strong(p, &expect, desired, __ATOMIC_RELAXED, __ATOMIC_RELAXED,

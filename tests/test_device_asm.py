@@ -1,0 +1,32 @@
+"""What the compiler cannot know about instructions written as text (gfx950 assembly of
+this repository's own code).  CPU only."""
+import re
+import subprocess
+
+from mtcheck_amd import build as B
+
+SRC = """
+#include "device.hpp"
+using namespace mtc;
+__global__ void k(Slot* tab, uint64_t mask, const Digest* d, uint32_t* err, uint32_t* out) {
+  bool claimed;
+  out[threadIdx.x] = table_insert(tab, mask, d[threadIdx.x], threadIdx.x, false, err, &claimed, true);
+}
+"""
+
+
+def test_pair_store_waits_before_its_data_is_overwritten(tmp_path):
+    """A vector store of more than 8 bytes needs two wait states before an instruction
+    overwrites its data registers.  The compiler keeps them after its own stores only."""
+    src = tmp_path / "k.hip"
+    src.write_text(SRC)
+    out = tmp_path / "k.s"
+    subprocess.run([B.HIPCC, *B.CFLAGS, "-I", B.CSRC, "--offload-device-only", "-S", str(src), "-o", str(out)], check=True,
+                   capture_output=True)
+    code = [s.split(";")[0].strip() for s in out.read_text().splitlines()]
+    code = [s for s in code if s and not s.startswith((".", "#")) and not s.endswith(":")]
+    at = [i for i, s in enumerate(code) if re.match(r"global_store_dwordx[34] .*\bsc1\b", s)]
+    assert at
+    for i in at:
+        m = re.match(r"s_nop (\d+)", code[i + 1])
+        assert m and int(m.group(1)) >= 1, code[i:i + 2]
