@@ -2578,9 +2578,9 @@ void hash_chunks(const uint8_t* data, uint64_t len, uint32_t C, int hk, Digest* 
 // runtime's copy kernel (which loops), 4.7 to 5.5 TB/s with looping blocks.
 __global__ __launch_bounds__(kThreads) void k_copy(const uint8_t* src, uint8_t* dst, uint64_t size) {
   const uint32_t head = (uint32_t)min<uint64_t>((16 - ((uint32_t)(uintptr_t)dst & 15)) & 15, size & ~3ull);
-  const uint64_t units = (size - head) / 16, u = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
+  const uint64_t blk = wide_block(), units = (size - head) / 16, u = blk * kThreads + threadIdx.x;
   if (u < units) st_stream16(dst + head + 16 * u, ld_stream16_a4(src + head + 16 * u));
-  if (blockIdx.x == 0) {  // before the first aligned unit, and after the last
+  if (blk == 0) {  // before the first aligned unit, and after the last
     if (threadIdx.x < head) dst[threadIdx.x] = src[threadIdx.x];
     const uint64_t t = head + 16 * units + threadIdx.x;
     if (t < size) dst[t] = src[t];
@@ -2589,7 +2589,7 @@ __global__ __launch_bounds__(kThreads) void k_copy(const uint8_t* src, uint8_t* 
 
 void copy_device(const uint8_t* src, uint8_t* dst, uint64_t size, hipStream_t st) {
   if (!size) return;
-  k_copy<<<(uint32_t)(size / 16 / kThreads + 1), kThreads, 0, st>>>(src, dst, size);
+  k_copy<<<wide_grid(size / 16 / kThreads + 1), kThreads, 0, st>>>(src, dst, size);
   MTC_HIP(hipGetLastError());
 }
 
@@ -3143,10 +3143,11 @@ static void add_leaf_scan(std::vector<Member>& ms, Ops& ops, ArenaImage& img) {
 // than an eighth, and blocks without a tile cost too (256 MiB at 2% store 330
 // of 16384 tiles: k_basic_diff 6.2 us with 2048 blocks, 6.7 us as 1024 looping ones
 // before), so it gets a block for every sixteenth tile, at least its share of 1024
-// and at most 8192, and they loop if they have to.
+// and at most 8192, and they loop if they have to.  A batch's baselines share 2^23
+// blocks (a launch holds fewer than 2^32 threads).
 static uint32_t gather_blocks(const Member& M, size_t members) {
   const uint64_t tiles = AsmShape(M.h->chunk_size).tiles(M.n);
-  const uint64_t most = M.baseline ? 1u << 20 : std::min<uint64_t>(std::max<uint64_t>({tiles / 16, 1024 / members, 1}), 8192);
+  const uint64_t most = M.baseline ? std::min<uint64_t>(1u << 20, std::max<uint64_t>((1u << 23) / members, 1)) : std::min<uint64_t>(std::max<uint64_t>({tiles / 16, 1024 / members, 1}), 8192);
   return 1 + (uint32_t)std::min<uint64_t>(tiles, most);
 }
 

@@ -30,6 +30,17 @@ struct Status {
   std::string msg;
 };
 
+// A grid for kernels without a loop whose size follows a buffer's bytes: the runtime
+// refuses a dimension of 2^32 threads or more (64 GiB at 16 bytes a thread), so the
+// blocks wrap into y from 2^31 threads on (blocks of up to 256).  The kernel's block
+// number is wide_block(); the last row may hold a few numbers past the last.
+inline dim3 wide_grid(uint64_t blocks) {
+  constexpr uint64_t kRow = 1ull << 23;
+  const uint64_t rows = std::max<uint64_t>(1, (blocks + kRow - 1) / kRow);
+  return dim3((uint32_t)std::max<uint64_t>(1, (blocks + rows - 1) / rows), (uint32_t)rows);
+}
+__device__ __forceinline__ uint64_t wide_block() { return (uint64_t)blockIdx.y * gridDim.x + blockIdx.x; }
+
 // Device allocation owned by the library, grown on demand.
 template <class T>
 struct DevBuf {

@@ -360,7 +360,7 @@ __global__ void k_r_cover_age(uint64_t* cover, uint64_t n) {
 constexpr uint32_t kCopyUnits = 4;
 __global__ __launch_bounds__(kRThreads) void k_r_copy(Chain c, uint64_t datalen, uint32_t ulog, uint8_t* out) {
   if (*c.err) return;
-  const uint64_t units = datalen / 16, u0 = (uint64_t)blockIdx.x * (kCopyUnits * kRThreads) + threadIdx.x;
+  const uint64_t blk = wide_block(), units = datalen / 16, u0 = blk * (kCopyUnits * kRThreads) + threadIdx.x;
   uint64_t e[kCopyUnits];
 #pragma unroll
   for (uint32_t i = 0; i < kCopyUnits; i++) {
@@ -380,7 +380,7 @@ __global__ __launch_bounds__(kRThreads) void k_r_copy(Chain c, uint64_t datalen,
     const uint64_t u = u0 + i * kRThreads;
     if (u < units && e[i]) st_stream16(out + 16 * u, v[i]);
   }
-  if (blockIdx.x == 0 && threadIdx.x < (datalen & 15)) {  // the short last chunk's last bytes
+  if (blk == 0 && threadIdx.x < (datalen & 15)) {  // the short last chunk's last bytes
     const uint64_t o = 16 * units + threadIdx.x, ce = c.cover[o / c.C];
     if (ce) out[o] = reinterpret_cast<const uint8_t*>(ce & kAddrMask)[o % c.C];
     else c.fail(ERR_CORRUPT);
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(kRThreads) void k_r_copy(Chain c, uint64_t datalen,
 // are neighbours in the diff too, byte by byte elsewhere.
 __global__ __launch_bounds__(kRThreads) void k_r_copy_any(Chain c, uint64_t datalen, uint8_t* out) {
   if (*c.err) return;
-  const uint64_t o = 16 * ((uint64_t)blockIdx.x * kRThreads + threadIdx.x);
+  const uint64_t o = 16 * (wide_block() * kRThreads + threadIdx.x);
   if (o >= datalen) return;
   const uint64_t k = o / c.C;
   const uint32_t w = (uint32_t)(o - k * c.C);
@@ -578,10 +578,10 @@ static void launch_restart(const Chain& c, const uint64_t* meta_src, const uint6
   }
   const uint32_t C = c.C;
   if (C >= 16 && (C & (C - 1)) == 0 && (uintptr_t)out % 16 == 0 && t.words)
-    k_r_copy<<<(uint32_t)std::max<uint64_t>(1, (datalen / 16 + kCopyUnits * kRThreads - 1) / (kCopyUnits * kRThreads)), kRThreads,
-               0, st>>>(c, datalen, (uint32_t)__builtin_ctz(C) - 4, out);
+    k_r_copy<<<wide_grid((datalen / 16 + kCopyUnits * kRThreads - 1) / (kCopyUnits * kRThreads)), kRThreads, 0, st>>>(
+        c, datalen, (uint32_t)__builtin_ctz(C) - 4, out);
   else
-    k_r_copy_any<<<(uint32_t)((datalen + 16 * kRThreads - 1) / (16 * kRThreads)), kRThreads, 0, st>>>(c, datalen, out);
+    k_r_copy_any<<<wide_grid((datalen + 16 * kRThreads - 1) / (16 * kRThreads)), kRThreads, 0, st>>>(c, datalen, out);
   MTC_HIP(hipGetLastError());
 }
 

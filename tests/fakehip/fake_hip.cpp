@@ -49,13 +49,14 @@ struct Graph {
 struct State {
   std::mutex mu;
   uint8_t* heap = nullptr;
-  uint64_t heap_size = 1ull << 40;  // reserved, not committed
+  uint64_t heap_size = 8ull << 40;  // reserved, not committed
   uint64_t brk = 0;
   std::map<uintptr_t, Alloc> allocs;
   std::map<const void*, std::string> names;  // host stub -> device name
   std::map<const void*, std::pair<void*, uint64_t>> vars;  // host shadow -> (fake device address, size)
   std::vector<std::string> violations;
   std::vector<std::string> launches;  // kernel names in launch order
+  std::vector<dim3> grids;            // and their grids
   std::vector<int> leaf_all_labels;   // per leaf member launched: its all_labels flag
   std::vector<int> label_resets;      // per k_assemble member launched: reset_labels is set
   std::vector<int> leaf_hash_later;   // per leaf member launched: it stores no digest
@@ -387,6 +388,11 @@ void check(const void* fn, dim3 grid, dim3 block, void** args) {
   auto it = st.names.find(fn);
   const std::string name = it == st.names.end() ? std::string("<unregistered kernel>") : it->second;
   st.launches.push_back(name);
+  st.grids.push_back(grid);
+  // The runtime refuses a dimension of 2^32 threads or more.
+  const uint64_t tx = (uint64_t)grid.x * block.x, ty = (uint64_t)grid.y * block.y, tz = (uint64_t)grid.z * block.z;
+  if ((tx | ty | tz) >> 32 || grid.y > 65535 || grid.z > 65535) violation(name + ": launch larger than the runtime takes");
+  const uint64_t blocks = (uint64_t)grid.x * grid.y * grid.z;
   if (grid.x == 0 || grid.y == 0 || grid.z == 0 || block.x == 0) violation(name + ": empty launch");
   if (block.x * block.y * block.z > 1024) violation(name + ": block too large");
   if (name.find("6Launch") != std::string::npos) {
@@ -419,6 +425,23 @@ void check(const void* fn, dim3 grid, dim3 block, void** args) {
     std::memcpy(&p, args[0], 8);
     std::memcpy(&count, args[1], 8);
     need(name, "p", p, 8 * count);
+  } else if (name.find("k_copy") != std::string::npos) {  // 16 bytes a thread, no loop
+    const uint8_t *src, *dst;
+    uint64_t size;
+    std::memcpy(&src, args[0], 8);
+    std::memcpy(&dst, args[1], 8);
+    std::memcpy(&size, args[2], 8);
+    need(name, "src", src, size);
+    need(name, "dst", dst, size);
+    if (blocks * block.x * 16 < size) violation(name + ": threads do not cover the bytes");
+  } else if (name.find("k_r_copy") != std::string::npos) {  // (chain, datalen, ..., out): the same, 64 bytes a thread for one
+    const bool any = name.find("k_r_copy_any") != std::string::npos;
+    uint64_t datalen;
+    const uint8_t* out;
+    std::memcpy(&datalen, args[1], 8);
+    std::memcpy(&out, args[any ? 2 : 3], 8);
+    need(name, "out", out, datalen);
+    if (blocks * block.x * (any ? 16 : 64) < (any ? datalen : datalen & ~15ull)) violation(name + ": threads do not cover the bytes");
   }
 }
 
@@ -459,10 +482,17 @@ const char* fakehip_launch_name(int i) {
   std::lock_guard<std::mutex> g(S().mu);
   return (i >= 0 && i < (int)S().launches.size()) ? S().launches[i].c_str() : "";
 }
+uint64_t fakehip_launch_blocks(int i) {
+  std::lock_guard<std::mutex> g(S().mu);
+  if (i < 0 || i >= (int)S().grids.size()) return 0;
+  const dim3 d = S().grids[i];
+  return (uint64_t)d.x * d.y * d.z;
+}
 void fakehip_reset() {
   std::lock_guard<std::mutex> g(S().mu);
   S().violations.clear();
   S().launches.clear();
+  S().grids.clear();
   S().leaf_all_labels.clear();
   S().label_resets.clear();
   S().leaf_hash_later.clear();

@@ -1,0 +1,64 @@
+"""Launches at the limits of sizes, on the CPU: the library's host code through the
+stand-in HIP runtime (tests/fakehip), which reports a launch that the runtime would
+refuse (a dimension of 2^32 threads or more) or that leaves bytes uncovered.  Device
+memory is reserved and never touched, so sizes beyond a card's are fine.  CPU only.
+"""
+import ctypes
+
+import pytest
+
+from tests.test_host_launches import (BASIC, OK, TREE, Header, checkpoint, create, dev_alloc, fake, launches,  # noqa: F401
+                                      violations)
+
+GIB = 1 << 30
+
+
+@pytest.mark.parametrize("size", [1, 4097, GIB, 64 * GIB - 1, 64 * GIB, 72 * GIB + 5])
+@pytest.mark.parametrize("offset", [0, 4])
+def test_device_copy_of_any_size(fake, size, offset):
+    L = fake
+    L.fakehip_reset()
+    src, dst = dev_alloc(L, size), dev_alloc(L, size + offset)
+    getattr(L, "_ZN3mtc11copy_deviceEPKhPhmP12ihipStream_t")(src, ctypes.c_void_p(dst.value + offset), ctypes.c_uint64(size), None)
+    assert any("k_copy" in n for n in launches(L))
+    assert violations(L) == []
+    for p in (src, dst):
+        L.hipFree(p)
+
+
+@pytest.mark.parametrize("C,datalen", [(1000, 63 * GIB), (1000, 72 * GIB + 5), (1 << 20, 72 * GIB), (1 << 20, 256 * GIB + 7)])
+@pytest.mark.parametrize("offset", [0, 4])
+def test_restart_of_any_size(fake, C, datalen, offset):
+    """A header without regions is a chain as far as the host sees it."""
+    L = fake
+    L.fakehip_reset()
+    diff = Header(0, 0, datalen, C, 0, 0, 0)
+    out = dev_alloc(L, datalen + offset)
+    ptrs = (ctypes.c_void_p * 1)(ctypes.addressof(diff))
+    sizes = (ctypes.c_uint64 * 1)(32)
+    assert L.mtc_restart(ptrs, sizes, 1, 0, 0, ctypes.c_void_p(out.value + offset), ctypes.c_uint64(datalen), 0, None) == OK
+    assert any("k_r_copy" in n for n in launches(L))
+    assert violations(L) == []
+    L.hipFree(out)
+
+
+def test_batch_of_large_baselines(fake):
+    """Sixteen baselines of 2^20 one-chunk tiles each."""
+    L = fake
+    L.fakehip_reset()
+    b = ctypes.c_void_p()
+    assert L.mtc_batch_create(ctypes.byref(b), 0, 0) == OK
+    B, C = 16, 8193
+    size = C << 20
+    hs = [create(L, C, BASIC) for _ in range(B)]
+    H = (ctypes.c_void_p * B)(*[h.value for h in hs])
+    datas = [dev_alloc(L, size) for _ in range(B)]
+    D = (ctypes.c_void_p * B)(*[d.value for d in datas])
+    N = (ctypes.c_uint64 * B)(*[size] * B)
+    assert L.mtc_checkpoint_batch(b, H, D, N, (ctypes.c_int * B)(*[1] * B), B, 1, None, None, None) == OK
+    assert violations(L) == []
+    for h in hs:
+        L.mtc_destroy(h)
+    for d in datas:
+        L.hipFree(d)
+    L.mtc_batch_destroy(b)
