@@ -2214,7 +2214,7 @@ struct AsmShape {
   uint32_t K, pieces;
   __host__ __device__ explicit AsmShape(uint32_t C) : K(256), pieces(1) {
     while (K > 1 && (uint64_t)K * C > kAsmTile) K >>= 1;
-    if (C > kAsmTile) pieces = (C + kAsmTile - 1) / kAsmTile;
+    if (C > kAsmTile) pieces = C / kAsmTile + (C % kAsmTile != 0);  // C may be near 2^32
   }
   __host__ __device__ uint64_t tiles(uint64_t chunks) const { return pieces > 1 ? chunks * pieces : (chunks + K - 1) / K; }
 };

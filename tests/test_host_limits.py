@@ -62,3 +62,21 @@ def test_batch_of_large_baselines(fake):
     for d in datas:
         L.hipFree(d)
     L.mtc_batch_destroy(b)
+
+
+@pytest.mark.parametrize("C", [16384, 16385, 0xFFFFC000, 0xFFFFC001, 0xFFFFF001, 0xFFFFFFFF])
+@pytest.mark.parametrize("approach", [TREE, BASIC])
+def test_gather_tiles_of_the_largest_chunks(fake, C, approach):
+    """A chunk larger than a gather tile (16 KiB) is sliced, up to the largest chunk
+    size: a baseline of one chunk has a block for every slice and one for the header."""
+    L = fake
+    L.fakehip_reset()
+    L.fakehip_launch_blocks.restype = ctypes.c_uint64
+    h = create(L, C, approach)
+    data = dev_alloc(L, 1000)
+    rc, _ = checkpoint(L, h, data, 1000, baseline=True)
+    assert rc == OK, L.mtc_last_error(h)
+    blocks = [L.fakehip_launch_blocks(i) for i, n in enumerate(launches(L)) if "assemble" in n or "basic_diff" in n]
+    assert blocks == [1 + -(-C // 16384)]
+    assert violations(L) == []
+    L.mtc_destroy(h)
