@@ -387,6 +387,10 @@ __device__ __forceinline__ Digest staged_hash(const uint8_t* data, uint64_t firs
 //   MD5      100 B 4474 -> 1324   333 B 2552 -> 1208   1000 B 3199 -> 1076   5000 B 1362 -> 1154
 // The leaf kernel of 200 MB in 1000-byte chunks: 144 -> 80.
 constexpr uint32_t kAnySeg = 128, kAnyCols = kAnySeg / 16 + 1, kAnyPacked = 112;
+// Passes over a chunk: counted, because an offset would wrap before it reached a C
+// within a pass of 2^32.
+constexpr uint32_t any_passes(uint32_t C) { return C / kAnySeg + (C % kAnySeg != 0); }
+static_assert(any_passes(1) == 1 && any_passes(128) == 1 && any_passes(129) == 2 && any_passes(~0u) == 1u << 25);
 
 // Bytes sh .. sh + 15 of the 32 bytes {a, b} (0 <= sh < 16).
 __device__ __forceinline__ uint4 cut16(const uint4& a, const uint4& b, uint32_t sh) {
@@ -445,8 +449,9 @@ __device__ __forceinline__ Digest any_digest(const uint8_t* data, uint64_t len, 
     }
   };
   load(0);
+  uint32_t at = 0;
 #pragma unroll 1
-  for (uint32_t at = 0; at < C; at += kAnySeg) {
+  for (uint32_t pass = any_passes(C); pass; pass--, at += kAnySeg) {
     // The LDS accesses of one wavefront execute in order.
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
