@@ -66,6 +66,39 @@ static void use_device(int dev) {
   MTC_HIP(hipSetDevice(dev));
 }
 
+// A pair of timing events of the handle for one copy, given back at its end.
+struct CopyEvents {
+  mtc_dedup* h;
+  hipEvent_t a = nullptr, b = nullptr;
+  explicit CopyEvents(mtc_dedup* handle) : h(handle) {
+    {
+      std::lock_guard<std::mutex> g(h->copy_mu);
+      if (!h->copy_ev.empty()) {
+        a = h->copy_ev.back().first;
+        b = h->copy_ev.back().second;
+        h->copy_ev.pop_back();
+        return;
+      }
+    }
+    MTC_HIP(hipEventCreate(&a));
+    const hipError_t e = hipEventCreate(&b);
+    if (e != hipSuccess) {
+      (void)hipEventDestroy(a);
+      throw HipError{e, "hipEventCreate"};
+    }
+  }
+  ~CopyEvents() {
+    try {
+      std::lock_guard<std::mutex> g(h->copy_mu);
+      h->copy_ev.emplace_back(a, b);
+    } catch (...) {  // no memory to keep them
+      (void)hipEventDestroy(a);
+      (void)hipEventDestroy(b);
+    }
+  }
+  CopyEvents(const CopyEvents&) = delete;
+};
+
 extern "C" {
 
 int mtc_create(mtc_dedup** out, uint32_t chunk_size, int approach, int hash_kind, int device) {
@@ -116,8 +149,10 @@ int mtc_destroy(mtc_dedup* h) {
     for (hipEvent_t e : h->copy_done)
       if (e) (void)hipEventDestroy(e);
   }
-  for (hipEvent_t e : h->copy_ev)
-    if (e) (void)hipEventDestroy(e);
+  for (auto& e : h->copy_ev) {
+    (void)hipEventDestroy(e.first);
+    (void)hipEventDestroy(e.second);
+  }
   if (h->ctl_d) (void)hipFree(h->ctl_d);
   if (h->ctl_h) (void)hipHostFree(h->ctl_h);
   delete h;  // device buffers are released by their destructors
@@ -153,9 +188,8 @@ int mtc_copy_diff(mtc_dedup* h, void* host_dst, uint64_t capacity, void* stream)
     if (capacity < h->last_diff_size) throw Status{MTC_ERR_BUFFER_TOO_SMALL, "host buffer smaller than the diff"};
     MTC_HIP(hipSetDevice(h->device));
     hipStream_t st = static_cast<hipStream_t>(stream);
-    for (hipEvent_t& e : h->copy_ev)
-      if (!e) MTC_HIP(hipEventCreate(&e));
-    MTC_HIP(hipEventRecord(h->copy_ev[0], st));
+    CopyEvents ev(h);
+    MTC_HIP(hipEventRecord(ev.a, st));
     // Device memory of this GPU: the library's own copy kernel (word-aligned); other
     // memory: the runtime's (unified addressing decides the direction).
     hipPointerAttribute_t attr;
@@ -164,11 +198,9 @@ int mtc_copy_diff(mtc_dedup* h, void* host_dst, uint64_t capacity, void* stream)
     (void)hipGetLastError();  // a plain host pointer is no error
     if (here) mtc::copy_device(h->diff_ptr(), static_cast<uint8_t*>(host_dst), h->last_diff_size, st);
     else MTC_HIP(hipMemcpyAsync(host_dst, h->diff_ptr(), h->last_diff_size, hipMemcpyDefault, st));
-    MTC_HIP(hipEventRecord(h->copy_ev[1], st));
-    // (the stream, not the event: another thread may record the event again)
-    MTC_HIP(hipStreamSynchronize(st));
-    (void)hipEventElapsedTime(&h->last_ms[3], h->copy_ev[0], h->copy_ev[1]);
-    (void)hipGetLastError();
+    MTC_HIP(hipEventRecord(ev.b, st));
+    MTC_HIP(hipEventSynchronize(ev.b));
+    (void)hipEventElapsedTime(&h->last_ms[3], ev.a, ev.b);
   });
 }
 

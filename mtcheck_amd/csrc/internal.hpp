@@ -5,8 +5,9 @@
 
 #include <algorithm>
 #include <atomic>
-
+#include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/mtcheck.h"
@@ -220,7 +221,10 @@ struct mtc_dedup {
   hipStream_t copy_st = nullptr;      // asynchronous diff copies
   hipEvent_t copy_done[2] = {nullptr, nullptr};  // after the last copy out of each arena
   bool copy_pending[2] = {false, false};
-  hipEvent_t copy_ev[2] = {nullptr, nullptr};    // around a synchronous copy (its timer)
+  // Around a synchronous copy (its timer): kept pairs that no copy is using.  Several
+  // threads may copy one diff at once, each between a pair of its own.
+  std::mutex copy_mu;
+  std::vector<std::pair<hipEvent_t, hipEvent_t>> copy_ev;
   const uint8_t* diff_ptr() const { return diff_cur ? diff_alt.p : diff.p; }
   mtc::DevBuf<mtc::Digest> dbg_tree;  // debug: full tree, as the serial reference leaves it
   mtc::DevBuf<uint8_t> dbg_labels;    // debug: all node labels

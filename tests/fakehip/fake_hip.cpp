@@ -18,10 +18,14 @@
 #include <cstring>
 #include <sys/mman.h>
 
+#include <chrono>
+#include <condition_variable>
 #include <cstdio>
 #include <map>
 #include <mutex>
+#include <set>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../mtcheck_amd/csrc/args.hpp"
@@ -68,6 +72,13 @@ struct State {
   hipStream_t capturing = nullptr;
   std::vector<Node> captured;
   uint64_t bytes_alive = 0;
+  uint64_t diff_size = 0;  // what a diff kernel reports (no kernel runs)
+  std::set<hipEvent_t> timing;                       // events that take the time
+  std::map<hipEvent_t, std::thread::id> recorded;    // by whom, until the time is read
+  // Waits for the stream or an event last until this many threads wait (a time limit
+  // ends them all the same).
+  int hold = 0, holding = 0;
+  std::condition_variable held;
 };
 
 State& S() {
@@ -359,6 +370,7 @@ void check_launch(const std::string& name, const uint8_t* arg0, uint32_t grid) {
       need(w, "ctl", a.ctl, kCtl);
       need(w, "ctr", a.ctr, 8);
       need_host(w, "out", a.out, kCtl);
+      if (S().diff_size) a.out->diff_size = S().diff_size;
     });
   } else if (has("8DiffArgs")) {
     check_members<DiffArgs>(name, L, grid, [](const std::string& w, const DiffArgs& a, uint32_t) {
@@ -374,6 +386,7 @@ void check_launch(const std::string& name, const uint8_t* arg0, uint32_t grid) {
       need(w, "ctr", a.ctr, 8);
       need(w, "changed", a.changed, 4);
       need_host(w, "out", a.out, kCtl);
+      if (S().diff_size) a.out->diff_size = S().diff_size;
       need(w, "dense", a.dense, 4ull * a.n);
       maybe(w, "reset_labels", a.reset_labels, a.n);
       S().label_resets.push_back(a.reset_labels ? 1 : 0);
@@ -482,6 +495,15 @@ const char* fakehip_launch_name(int i) {
   std::lock_guard<std::mutex> g(S().mu);
   return (i >= 0 && i < (int)S().launches.size()) ? S().launches[i].c_str() : "";
 }
+void fakehip_set_diff_size(uint64_t size) {
+  std::lock_guard<std::mutex> g(S().mu);
+  S().diff_size = size;
+}
+void fakehip_hold(int threads) {
+  std::lock_guard<std::mutex> g(S().mu);
+  S().hold = threads;
+  S().holding = 0;
+}
 uint64_t fakehip_launch_blocks(int i) {
   std::lock_guard<std::mutex> g(S().mu);
   if (i < 0 || i >= (int)S().grids.size()) return 0;
@@ -493,6 +515,8 @@ void fakehip_reset() {
   S().violations.clear();
   S().launches.clear();
   S().grids.clear();
+  S().diff_size = 0;
+  S().hold = S().holding = 0;
   S().leaf_all_labels.clear();
   S().label_resets.clear();
   S().leaf_hash_later.clear();
@@ -675,20 +699,50 @@ hipError_t hipStreamDestroy(hipStream_t s) {
   delete reinterpret_cast<uint64_t*>(s);
   return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+static hipError_t wait_held() {
+  std::unique_lock<std::mutex> g(S().mu);
+  if (S().hold) {
+    S().holding++;
+    S().held.notify_all();
+    S().held.wait_for(g, std::chrono::seconds(5), [] { return S().holding >= S().hold; });
+  }
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) { return wait_held(); }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned int) { return hipSuccess; }
-hipError_t hipEventCreate(hipEvent_t* e) {
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned int) {
   *e = reinterpret_cast<hipEvent_t>(new uint64_t(0));
   return hipSuccess;
 }
-hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned int) { return hipEventCreate(e); }
+hipError_t hipEventCreate(hipEvent_t* e) {
+  (void)hipEventCreateWithFlags(e, 0);
+  std::lock_guard<std::mutex> g(S().mu);
+  S().timing.insert(*e);
+  return hipSuccess;
+}
 hipError_t hipEventDestroy(hipEvent_t e) {
+  {
+    std::lock_guard<std::mutex> g(S().mu);
+    S().timing.erase(e);
+    S().recorded.erase(e);
+  }
   delete reinterpret_cast<uint64_t*>(e);
   return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+  std::lock_guard<std::mutex> g(S().mu);
+  if (!S().timing.count(e)) return hipSuccess;
+  auto it = S().recorded.find(e);
+  if (it != S().recorded.end() && it->second != std::this_thread::get_id())
+    violation("an event recorded by two threads before either has read its time");
+  S().recorded[e] = std::this_thread::get_id();
+  return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t) { return wait_held(); }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) {
+  std::lock_guard<std::mutex> g(S().mu);
+  S().recorded.erase(a);
+  S().recorded.erase(b);
   *ms = 0.0f;
   return hipSuccess;
 }

@@ -4,6 +4,7 @@ refuse (a dimension of 2^32 threads or more) or that leaves bytes uncovered.  De
 memory is reserved and never touched, so sizes beyond a card's are fine.  CPU only.
 """
 import ctypes
+import threading
 
 import pytest
 
@@ -79,4 +80,28 @@ def test_gather_tiles_of_the_largest_chunks(fake, C, approach):
     blocks = [L.fakehip_launch_blocks(i) for i, n in enumerate(launches(L)) if "assemble" in n or "basic_diff" in n]
     assert blocks == [1 + -(-C // 16384)]
     assert violations(L) == []
+    L.mtc_destroy(h)
+
+
+def test_copies_of_one_handle_by_two_threads(fake):
+    """Each copy takes its time between events of its own."""
+    L = fake
+    L.fakehip_reset()
+    h = create(L, 128)
+    data = dev_alloc(L, 1 << 20)
+    L.fakehip_set_diff_size(ctypes.c_uint64(5000))
+    assert checkpoint(L, h, data, 1 << 20, baseline=True)[0] == OK
+    dst = [dev_alloc(L, 5000) for _ in range(2)]
+    for _ in range(2):  # the second time with what the first one left in the handle
+        L.fakehip_hold(2)
+        rcs = []
+        ts = [threading.Thread(target=lambda p=p: rcs.append(L.mtc_copy_diff(h, p, ctypes.c_uint64(5000), None))) for p in dst]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        L.fakehip_hold(0)
+        assert rcs == [OK, OK]
+        assert violations(L) == []
+    L.fakehip_reset()
     L.mtc_destroy(h)
