@@ -191,11 +191,18 @@ int mtc_copy_diff(mtc_dedup* h, void* host_dst, uint64_t capacity, void* stream)
     CopyEvents ev(h);
     MTC_HIP(hipEventRecord(ev.a, st));
     // Device memory of this GPU: the library's own copy kernel (word-aligned); other
-    // memory: the runtime's (unified addressing decides the direction).
+    // memory: the runtime's (unified addressing decides the direction), which also
+    // refuses a destination that is shorter than the caller says.
     hipPointerAttribute_t attr;
-    const bool here = hipPointerGetAttributes(&attr, host_dst) == hipSuccess && attr.type == hipMemoryTypeDevice &&
-                      attr.device == h->device && (uintptr_t)host_dst % 4 == 0;
-    (void)hipGetLastError();  // a plain host pointer is no error
+    hipDeviceptr_t base = nullptr;
+    size_t span = 0;
+    hipError_t e = hipPointerGetAttributes(&attr, host_dst);
+    bool here = e == hipSuccess && attr.type == hipMemoryTypeDevice && attr.device == h->device && (uintptr_t)host_dst % 4 == 0;
+    if (here) {
+      e = hipMemGetAddressRange(&base, &span, host_dst);
+      here = e == hipSuccess && h->last_diff_size <= (uintptr_t)base + span - (uintptr_t)host_dst;
+    }
+    if (e != hipSuccess) (void)hipGetLastError();  // a plain host pointer is no error
     if (here) mtc::copy_device(h->diff_ptr(), static_cast<uint8_t*>(host_dst), h->last_diff_size, st);
     else MTC_HIP(hipMemcpyAsync(host_dst, h->diff_ptr(), h->last_diff_size, hipMemcpyDefault, st));
     MTC_HIP(hipEventRecord(ev.b, st));

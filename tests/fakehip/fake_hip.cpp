@@ -636,8 +636,14 @@ hipError_t hipHostFree(void* p) {
 static hipError_t copy(void* dst, const void* src, size_t n) {
   {
     std::lock_guard<std::mutex> g(S().mu);
-    if (in_heap(dst) && !find(dst, n)) violation("copy writes past a device allocation");
-    if (in_heap(src) && !find(src, n)) violation("copy reads past a device allocation");
+    if (in_heap(dst) && !find(dst, n)) {
+      violation("copy writes past a device allocation");
+      return hipErrorInvalidValue;  // the runtime refuses it
+    }
+    if (in_heap(src) && !find(src, n)) {
+      violation("copy reads past a device allocation");
+      return hipErrorInvalidValue;
+    }
   }
   if (n) std::memmove(dst, src, n);
   return hipSuccess;
@@ -665,6 +671,16 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t* attr, const void*) {
   std::memset(attr, 0, sizeof(*attr));
   attr->type = hipMemoryTypeDevice;
   attr->device = 0;
+  return hipSuccess;
+}
+
+hipError_t hipMemGetAddressRange(hipDeviceptr_t* base, size_t* size, hipDeviceptr_t p) {
+  std::lock_guard<std::mutex> g(S().mu);
+  uintptr_t start = 0;
+  const Alloc* a = find(p, 1, &start);
+  if (!a || !a->alive) return hipErrorInvalidValue;
+  if (base) *base = reinterpret_cast<hipDeviceptr_t>(start);
+  if (size) *size = a->size;
   return hipSuccess;
 }
 

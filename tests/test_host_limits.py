@@ -105,3 +105,22 @@ def test_copies_of_one_handle_by_two_threads(fake):
         assert violations(L) == []
     L.fakehip_reset()
     L.mtc_destroy(h)
+
+
+@pytest.mark.parametrize("room", [5000, 4999, 64])
+def test_device_copy_stays_in_the_destination(fake, room):
+    """The runtime refuses a copy past the end of the destination's allocation.  A
+    capacity larger than the allocation still ends in that refusal, not in a kernel."""
+    L = fake
+    L.fakehip_reset()
+    h = create(L, 128)
+    data = dev_alloc(L, 1 << 20)
+    L.fakehip_set_diff_size(ctypes.c_uint64(5000))
+    assert checkpoint(L, h, data, 1 << 20, baseline=True)[0] == OK
+    p = dev_alloc(L, room + 16)
+    L.fakehip_reset()
+    rc = L.mtc_copy_diff(h, ctypes.c_void_p(p.value + 16), ctypes.c_uint64(1 << 20), None)
+    copied = any("k_copy" in n for n in launches(L))
+    assert (rc, copied) == ((OK, True) if room >= 5000 else (6, False))
+    L.fakehip_reset()
+    L.mtc_destroy(h)
