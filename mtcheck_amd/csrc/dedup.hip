@@ -1324,7 +1324,7 @@ struct SweepA {
 __device__ __forceinline__ uint8_t decide_leaf(const SweepArgs& a, uint64_t c) {
   const uint32_t s = a.leaf_slot[c];
   const uint64_t me = ((uint64_t)a.cur << 32) | (uint32_t)(a.g.n - 1 + c);
-  const uint8_t l = (s <= a.mask + 1 && a.tab[s].val == me) ? L_FIRST : L_SHIFT;
+  const uint8_t l = (s <= a.mask + 1 && ld_relaxed(&a.tab[s].val) == me) ? L_FIRST : L_SHIFT;
   a.labels[c] = l;
   return l;
 }

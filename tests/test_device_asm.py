@@ -15,6 +15,31 @@ __global__ void k(Slot* tab, uint64_t mask, const Digest* d, uint32_t* err, uint
 """
 
 
+def assembly(tmp_path, source):
+    src, out = tmp_path / "k.hip", tmp_path / "k.s"
+    src.write_text(source)
+    subprocess.run([B.HIPCC, *B.CFLAGS, "-I", B.CSRC, "--offload-device-only", "-S", str(src), "-o", str(out)], check=True,
+                   capture_output=True)
+    return out.read_text()
+
+
+DECIDE = """
+#include "dedup.hip"
+namespace mtc {
+__global__ void k_decide(SweepArgs a, uint8_t* out) { out[threadIdx.x] = decide_leaf(a, threadIdx.x); }
+}
+"""
+
+
+def test_sweep_a_reads_table_values_at_agent_scope(tmp_path):
+    """Sweep A inserts, so it reads a slot's value past the caches of its own die (sc1)
+    where it decides a pending leaf too."""
+    text = assembly(tmp_path, DECIDE)
+    body = re.search(r"^_ZN3mtc8k_decide\w*:.*?s_endpgm", text, re.M | re.S).group(0)
+    loads = re.findall(r"global_load_dwordx2 .*", body)
+    assert len(loads) == 1 and "sc1" in loads[0], loads
+
+
 def test_pair_store_waits_before_its_data_is_overwritten(tmp_path):
     """A vector store of more than 8 bytes needs two wait states before an instruction
     overwrites its data registers.  The compiler keeps them after its own stores only."""
