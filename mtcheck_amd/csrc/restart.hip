@@ -238,36 +238,46 @@ struct Regions {
   }
 };
 
-// Chunks of the first-occurrence regions of the pass's oldest diff, which hold nearly
-// the whole buffer when it is the baseline: plain stores, nothing else writes the
-// cover meanwhile (atomic max runs at a third of their rate).
-__global__ __launch_bounds__(kRThreads) void k_r_cover_base(Chain c, uint32_t p) {
-  if (*c.err) return;
-  Regions d(c, p);
-  const uint64_t data = c.data()[p];
-  for (uint64_t j = (uint64_t)blockIdx.x * kRThreads + threadIdx.x; j < d.total; j += (uint64_t)gridDim.x * kRThreads)
-    c.cover[d.chunk(c, (uint32_t)j)] = (1ull << kAddrBits) | (data + j * c.C);
-}
-
-// The other diffs of a pass (positions lo .. hi - 1; lo's regions are covered
-// already), in one launch: nblk blocks for the first-occurrence chunks, the rest for
-// the shifted entries.  Each leaf of a shifted entry's `node` takes the data slot of
-// the matching leaf of `prev` inside the source diff's region
-// (src/tree_approach.cpp:887-925, 1058-1118); a wavefront shares the leaves of its
-// larger entries.
+// Covers first-occurrence chunks (diffs flo .. hi - 1 of the pass that starts at lo; nblk
+// blocks) and the leaves of shifted entries (diffs slo .. hi - 1; the other blocks).  Each
+// leaf of a shifted entry's `node` takes the data slot of the matching leaf of `prev`
+// inside the source diff's region (src/tree_approach.cpp:887-925, 1058-1118); a wavefront
+// shares the leaves of its larger entries.
+// PLAIN: one diff (hi - 1), by plain stores over what the earlier ones left: the pass's
+// oldest, which holds nearly the whole buffer when it is the baseline, and any diff that
+// stores kCoverPlain chunks.  The others share a launch, in which the newest entry of a
+// chunk stands by atomic max: it needs no order, but runs at a third of a plain store's
+// rate.  A chain of three whole rewrites, 1 GiB in 48-byte chunks (22 million): 760 us
+// with the last two by atomics, 510 so; 256 MiB in 64-byte chunks (2^22) 212 and 177, in
+// 96-byte chunks no difference.  (Many shifted entries are no reason for a launch of
+// their own: their lookups take the time, 2-3% more of it with fewer in flight.)
 constexpr uint32_t kShiftOwn = 4;  // most leaves a lane covers by itself
-__global__ __launch_bounds__(kRThreads) void k_r_cover_rest(Chain c, uint32_t lo, uint32_t hi, uint32_t nblk) {
+constexpr uint64_t kCoverPlain = 1u << 22;
+template <bool PLAIN>
+__global__ __launch_bounds__(kRThreads) void k_r_cover(Chain c, uint32_t lo, uint32_t flo, uint32_t slo, uint32_t hi,
+                                                       uint32_t nblk) {
   if (*c.err) return;
+  auto put = [&](uint32_t chunk, uint64_t v) {
+    if (PLAIN) c.cover[chunk] = v;
+    else atomicMax((unsigned long long*)&c.cover[chunk], (unsigned long long)v);
+  };
   if (blockIdx.x < nblk) {
+    if (PLAIN) {
+      const uint32_t p = hi - 1;
+      Regions d(c, p);
+      const uint64_t top = (uint64_t)(p - lo + 1) << kAddrBits, data = c.data()[p];
+      for (uint64_t j = (uint64_t)blockIdx.x * kRThreads + threadIdx.x; j < d.total; j += (uint64_t)nblk * kRThreads)
+        put(d.chunk(c, (uint32_t)j), top | (data + j * c.C));
+      return;
+    }
     const uint64_t* base = c.chunk_base();
     const uint64_t end = base[hi];
-    for (uint64_t j = base[lo + 1] + (uint64_t)blockIdx.x * kRThreads + threadIdx.x; j < end; j += (uint64_t)nblk * kRThreads) {
-      const uint32_t p = owner(base, lo + 1, hi, j);
+    for (uint64_t j = base[flo] + (uint64_t)blockIdx.x * kRThreads + threadIdx.x; j < end; j += (uint64_t)nblk * kRThreads) {
+      const uint32_t p = owner(base, flo, hi, j);
       const uint64_t slot = j - base[p];
       Regions d(c, p);
       if (slot >= d.total) continue;
-      atomicMax((unsigned long long*)&c.cover[d.chunk(c, (uint32_t)slot)],
-                (unsigned long long)(((uint64_t)(p - lo + 1) << kAddrBits) | (c.data()[p] + slot * c.C)));
+      put(d.chunk(c, (uint32_t)slot), ((uint64_t)(p - lo + 1) << kAddrBits) | (c.data()[p] + slot * c.C));
     }
     return;
   }
@@ -276,12 +286,12 @@ __global__ __launch_bounds__(kRThreads) void k_r_cover_rest(Chain c, uint32_t lo
   const uint64_t nodes = 2ull * c.g.n - 1;
   const uint32_t lane = lane_id();
   const uint64_t stride = (uint64_t)(gridDim.x - nblk) * kRThreads;
-  for (uint64_t w0 = base[lo] + (uint64_t)(blockIdx.x - nblk) * kRThreads + (threadIdx.x & ~63u); w0 < end; w0 += stride) {
+  for (uint64_t w0 = base[slo] + (uint64_t)(blockIdx.x - nblk) * kRThreads + (threadIdx.x & ~63u); w0 < end; w0 += stride) {
     const uint64_t i = w0 + lane;
     uint32_t node = 0, prev = 0, root = 0, rbase = 0, spos = 0, cnt = 0, p = 0;
     bool ok = i < end;
     if (ok) {
-      p = owner(base, lo, hi, i);
+      p = owner(base, slo, hi, i);
       const uint32_t e = (uint32_t)(i - base[p]);
       const uint8_t* sh = reinterpret_cast<const uint8_t*>(c.shift()[p]) + 8ull * e;
       node = ld32(sh);
@@ -331,7 +341,7 @@ __global__ __launch_bounds__(kRThreads) void k_r_cover_rest(Chain c, uint32_t lo
           c.fail(ERR_CORRUPT);
           break;
         }
-        atomicMax((unsigned long long*)&c.cover[run_at(nr, ns, nc, j)], (unsigned long long)(top | (data + slot * c.C)));
+        put(run_at(nr, ns, nc, j), top | (data + slot * c.C));
       }
     };
     if (cnt && cnt <= kShiftOwn) cover_leaves(node, prev, root, rbase, spos, p, 0, 1, cnt);
@@ -570,10 +580,25 @@ static void launch_restart(const Chain& c, const uint64_t* meta_src, const uint6
   for (uint64_t lo = 0; lo < L; lo += kCoverPos) {
     const uint32_t hi = (uint32_t)std::min<uint64_t>(L, lo + kCoverPos);
     if (lo) k_r_cover_age<<<rgrid(n), kRThreads, 0, st>>>(c.cover, n);
-    k_r_cover_base<<<rgrid(cbase[lo + 1] - cbase[lo], 4096), kRThreads, 0, st>>>(c, (uint32_t)lo);
-    const uint64_t first = cbase[hi] - cbase[lo + 1], shifted = sbase[hi] - sbase[lo];
-    const uint32_t fblk = first ? rgrid(first) : 0, sblk = shifted ? rgrid(shifted) : 0;
-    if (fblk + sblk) k_r_cover_rest<<<fblk + sblk, kRThreads, 0, st>>>(c, (uint32_t)lo, hi, fblk);
+    auto blocks = [](uint64_t items) { return items ? rgrid(items) : 0u; };
+    uint32_t flo = (uint32_t)lo, slo = flo;  // the first diffs not covered yet
+    auto plain = [&](uint32_t p, uint32_t sblk) {
+      const uint32_t fblk = rgrid(cbase[p + 1] - cbase[p], 4096);
+      k_r_cover<true><<<fblk + sblk, kRThreads, 0, st>>>(c, (uint32_t)lo, p, p, p + 1, fblk);
+    };
+    auto together = [&](uint32_t end) {  // all before end
+      const uint32_t fblk = blocks(cbase[end] - cbase[flo]), sblk = blocks(sbase[end] - sbase[slo]);
+      if (fblk + sblk) k_r_cover<false><<<fblk + sblk, kRThreads, 0, st>>>(c, (uint32_t)lo, flo, slo, end, fblk);
+      flo = slo = end;
+    };
+    plain(flo++, 0);  // its shifted entries come with the next launch
+    for (uint32_t p = flo; p < hi; p++)
+      if (cbase[p + 1] - cbase[p] >= kCoverPlain) {
+        together(p);
+        plain(p, blocks(sbase[p + 1] - sbase[p]));
+        flo = slo = p + 1;
+      }
+    together(hi);
     MTC_HIP(hipGetLastError());
   }
   const uint32_t C = c.C;
