@@ -3,6 +3,8 @@ this repository's own code).  CPU only."""
 import re
 import subprocess
 
+import pytest
+
 from mtcheck_amd import build as B
 
 SRC = """
@@ -15,15 +17,7 @@ __global__ void k(Slot* tab, uint64_t mask, const Digest* d, uint32_t* err, uint
 """
 
 
-def assembly(tmp_path, source):
-    src, out = tmp_path / "k.hip", tmp_path / "k.s"
-    src.write_text(source)
-    subprocess.run([B.HIPCC, *B.CFLAGS, "-I", B.CSRC, "--offload-device-only", "-S", str(src), "-o", str(out)], check=True,
-                   capture_output=True)
-    return out.read_text()
-
-
-DECIDE = """
+WHOLE = """
 #include "dedup.hip"
 namespace mtc {
 __global__ void k_decide(SweepArgs a, uint8_t* out) { out[threadIdx.x] = decide_leaf(a, threadIdx.x); }
@@ -31,12 +25,24 @@ __global__ void k_decide(SweepArgs a, uint8_t* out) { out[threadIdx.x] = decide_
 """
 
 
-def test_sweep_a_reads_table_values_at_agent_scope(tmp_path):
+@pytest.fixture(scope="module")
+def whole(tmp_path_factory):
+    """The assembly of dedup.hip, and of decide_leaf in a kernel of its own."""
+    d = tmp_path_factory.mktemp("asm")
+    (d / "k.hip").write_text(WHOLE)
+    subprocess.run([B.HIPCC, *B.CFLAGS, "-I", B.CSRC, "--offload-device-only", "-S", str(d / "k.hip"), "-o", str(d / "k.s")],
+                   check=True, capture_output=True)
+    return (d / "k.s").read_text()
+
+
+def kernel(text, name):
+    return re.search(rf"^{name}\w*:.*?s_endpgm", text, re.M | re.S).group(0)
+
+
+def test_sweep_a_reads_table_values_at_agent_scope(whole):
     """Sweep A inserts, so it reads a slot's value past the caches of its own die (sc1)
     where it decides a pending leaf too."""
-    text = assembly(tmp_path, DECIDE)
-    body = re.search(r"^_ZN3mtc8k_decide\w*:.*?s_endpgm", text, re.M | re.S).group(0)
-    loads = re.findall(r"global_load_dwordx2 .*", body)
+    loads = re.findall(r"global_load_dwordx2 .*", kernel(whole, "_ZN3mtc8k_decide"))
     assert len(loads) == 1 and "sc1" in loads[0], loads
 
 
@@ -55,3 +61,12 @@ def test_pair_store_waits_before_its_data_is_overwritten(tmp_path):
     for i in at:
         m = re.match(r"s_nop (\d+)", code[i + 1])
         assert m and int(m.group(1)) >= 1, code[i:i + 2]
+
+
+def test_md5_by_bytes_issues_a_blocks_loads_together(whole):
+    """The four 16-byte loads of a 64-byte block, with nothing between them: the other wavefronts
+    of a compute unit push a line out of its cache before a late one of them reads it."""
+    lines = [s.strip() for s in kernel(whole, "_ZN3mtc13k_hash_chunksILi1ELin1EE").splitlines()]
+    lines = [s for s in lines if s and not s.startswith(";")]
+    at = [i for i, s in enumerate(lines) if s.startswith("global_load_dwordx4")]
+    assert len(at) == 4 and at[3] - at[0] == 3, lines[at[0]:at[-1] + 1]
