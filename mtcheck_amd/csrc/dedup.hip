@@ -2539,18 +2539,47 @@ static uint64_t next_pow2(uint64_t x) {
 }
 
 // The kernel that hashes chunks of C bytes: one for the size (16-byte aligned data), 0
-// for any other, or -1: byte by byte, which is still the better way for chunks under 20
-// bytes, for Murmur3 chunks under 50 with at most four beyond whole 16-byte blocks (their reads hit the
-// cache, and little is left of the wide columns' gain) and for MD5 of few chunks (each
-// thread's chain of steps decides).  Microseconds staged / byte by byte:
-//   Murmur3, 4 GiB:  20 B 2346 / 1855   33 B 1469 / 1296   48 B 1146 / 1037
-//                    28 B 1672 / 2477   40 B 1264 / 1792   50 B 1140 / 1395
-//   64 MiB, 7 B:     Murmur3 102 / 74   MD5 189 / 135
-//   MD5, 64 MiB:     1500 B (44.7 thousand chunks) 48 / 41   5000 B (13.4 thousand) 115 / 84
-//                    1000 B (67.1 thousand) 45 / 47          333 B 42 / 49
-static int leaf_cb(int hk, uint32_t C, uint64_t n, const void* data) {
+// (staged) for any other, or -1 (byte by byte, which the compiler turns into wide loads)
+// where that is the faster one.  Staging pays where a lane's lines leave the cache before
+// the lane is through with them (many chunks) or straddle words (odd addresses); it costs
+// registers, LDS and, with few wavefronts, the latency of its passes.  leaf: the leaf
+// kernel, whose blocks hold four wavefronts, and not mtc_hash_chunks.  Microseconds staged
+// / byte by byte, each call on other bytes than the last (dword: every chunk starts at one):
+//   Chunks under 20 bytes, and Murmur3's under 50 with at most 4 beyond whole 16-byte
+//   blocks: 4 GiB, Murmur3, 20 B 2346 / 1855, 33 B 1469 / 1296, 48 B 1146 / 1037 (28 B
+//   1672 / 2477); 64 MiB, 7 B, Murmur3 102 / 74, MD5 189 / 135.
+//   A leaf's under 26 (MD5: 25): 24 B, 64 MiB, Murmur3 48 / 41, MD5 93 / 89.
+//   Murmur3, leaves, dword: very few (256 KiB in 2500-byte chunks 45 / 32); whole 64-byte
+//   blocks below 32 MiB (320 B, 16 MiB 9.7 / 8.7, 64 MiB 22 / 34); 64 B at any size (256
+//   MiB 88 / 74); rows a multiple of 8 KiB apart, which meet in one channel (8 KiB, 16
+//   MiB 133 / 110, 1 GiB 272 / 531; hashed alone, 16 MiB 131 / 117, 256 MiB even), and of
+//   4 KiB (4 KiB, 16 MiB 72 / 66).
+//   MD5: under 65536 chunks, whose lines the cache holds (64 MiB: 1500 B 48 / 41, 333 B 42
+//   / 49); 64 B at any address (leaves, 1 GiB 691 / 429); dword, whole 64-byte blocks below
+//   1 KiB (leaves, 1 GiB: 192 B 395 / 281, 384 B 307 / 252, 512 B 328 / 315; hashed alone
+//   192 B 309 / 278, 384 B 256 / 275), from there on up to 131072 chunks (leaves, 1 KiB:
+//   65536 chunks 33 / 25, 262144 93 / 94), leaves 8 KiB apart always; dword, up to 8 bytes
+//   beyond whole blocks, below 262144 chunks (leaves, 200 B, 16 MiB 15 / 11, 64 MiB 39 /
+//   49), leaves under 128 B always (72 B, 64 MiB 48 / 40).
+static int leaf_cb(int hk, uint32_t C, uint64_t n, const void* data, bool leaf) {
   if ((uintptr_t)data % 16 == 0 && C >= 16 && C <= 4096 && (C & (C - 1)) == 0) return (int)C;
-  return C < 20 || (hk == HASH_MD5 ? n < 65536 : C < 50 && C % 16 <= 4) ? -1 : 0;
+  const bool dword = (uintptr_t)data % 4 == 0 && C % 4 == 0, blocks = dword && C % 64 == 0, rows8k = dword && C % 8192 == 0;
+  const uint64_t len = n * C, MiB = 1u << 20;
+  bool bytes = C < 20;
+  if (hk == HASH_MD5) {
+    bytes |= n < 65536 || C == 64 || (leaf && C < 25);
+    bytes |= blocks && (C < 1024 || n < 131072 || (leaf && rows8k));
+    bytes |= dword && C % 64 != 0 && C % 64 <= 8 && ((n < 262144 && C < 4096) || (leaf && C < 128));
+  } else {
+    bytes |= C < 50 && C % 16 <= 4;
+    if (leaf) {
+      bytes |= C < 26 || C == 64 || (dword && len < MiB / 2);
+      bytes |= (blocks && len < 32 * MiB) || ((rows8k || (dword && C == 4096)) && n < 131072);
+    } else {
+      bytes |= rows8k && n < 131072 && len < 128 * MiB;
+    }
+  }
+  return bytes ? -1 : 0;
 }
 
 template <int HK, int CB>
@@ -2561,7 +2590,7 @@ static void launch_hash_cb(const uint8_t* data, uint64_t len, uint32_t n, uint32
 
 template <int HK>
 static void launch_hash_chunks(const uint8_t* data, uint64_t len, uint32_t n, uint32_t C, Digest* out, hipStream_t st) {
-  switch (leaf_cb(HK, C, n, data)) {
+  switch (leaf_cb(HK, C, n, data, false)) {
     case -1: launch_hash_cb<HK, -1>(data, len, n, C, out, st); break;
     case 16: launch_hash_cb<HK, 16>(data, len, n, C, out, st); break;
     case 32: launch_hash_cb<HK, 32>(data, len, n, C, out, st); break;
@@ -3081,7 +3110,7 @@ static void prepare_member(Member& M, hipStream_t st) {
   M.n = h->n;
   M.cur = h->current_id;
   M.g = make_geo(M.n);
-  M.cb = leaf_cb(h->hash_kind, h->chunk_size, M.n, M.data);
+  M.cb = leaf_cb(h->hash_kind, h->chunk_size, M.n, M.data, true);
   // With asynchronous copies, checkpoints alternate diff arenas; this step waits
   // (on the device) for the copy still reading the arena it is about to write.
   // The pending flag is cleared once the step has completed.

@@ -1,5 +1,9 @@
 """Sizes beyond one row of a launch's blocks (2^31 threads)."""
+import numpy as np
 import pytest
+
+from oracle import oracle as O
+from tests.helpers import first_mismatch
 
 torch = pytest.importorskip("torch")
 import mtcheck_amd as M  # noqa: E402
@@ -25,3 +29,34 @@ def test_copy_and_restart_beyond_one_row_of_blocks():
     M.restart_into(out, [kept], 0)
     for i in range(0, n, 1 << 30):
         assert torch.equal(out[i:i + (1 << 30)], data[i:i + (1 << 30)]), i
+
+
+def series(versions, C, hk=0, offset=0, load_factor=0.125):
+    n = len(versions[0])
+    buf = torch.zeros(n + 16, dtype=torch.uint8, device="cuda:0")
+    d, orc = M.TreeDeduplicator(C, hash_kind=hk), O.OracleDedup(C, hk)
+    d.set_tuning(1, load_factor, 8)
+    for k, host in enumerate(versions):
+        print(f"C={C} hash {hk} n={n} offset {offset} load factor {load_factor} checkpoint {k}", flush=True)
+        buf[offset:offset + n] = torch.from_numpy(host)
+        g = d.checkpoint(buf[offset:offset + n], make_baseline=(k == 0))
+        e = orc.checkpoint(host, make_baseline=(k == 0), threads=8)
+        assert g == e, (k, first_mismatch(g, e))
+    d.close()
+
+
+@pytest.mark.parametrize("C,hk,n,offset", [
+    (100, 0, 5_000, 0), (100, 0, 5_300, 0), (25, 0, 5_000, 1), (64, 0, 9_000, 4), (320, 0, 300, 0), (320, 0, 106_000, 0),
+    (4096, 0, 300, 4), (8192, 0, 150, 0), (8192, 0, 150, 3), (24, 1, 70_000, 0), (64, 1, 66_000, 1), (72, 1, 70_000, 0),
+    (200, 1, 66_000, 0), (200, 1, 66_000, 2), (128, 1, 66_000, 1), (128, 1, 66_000, 4)])
+def test_series_by_bytes_and_staged(C, hk, n, offset):
+    """Chunk sizes, numbers and addresses on both sides of the rules that choose the leaf kernel."""
+    rng = np.random.default_rng(C + n + offset)
+    v = [rng.integers(0, 256, n * C - C // 3, dtype=np.uint8)]
+    for _ in range(2):
+        w = v[-1].copy()
+        for first in rng.integers(0, n, 9):
+            w[first * C:(first + 2) * C] = rng.integers(0, 256, w[first * C:(first + 2) * C].size, dtype=np.uint8)
+        w[-1] ^= 1
+        v.append(w)
+    series(v, C, hk, offset)

@@ -153,3 +153,42 @@ def test_large_diffs_of_a_chain_are_covered_by_plain_stores(fake, chunks, plain,
     assert cover == plain
     assert violations(L) == []
     L.hipFree(out)
+
+
+@pytest.mark.parametrize("hk,C,n,offset,alone,leaf", [
+    # what one of the kernels for a chunk size takes, whatever its number
+    (0, 128, 5, 0, 128, 128), (1, 4096, 9, 16, 4096, 4096),
+    # Murmur3: 0 is the staged kernel, -1 the one by bytes
+    (0, 19, 90_000, 0, -1, -1), (0, 20, 90_000, 0, -1, -1), (0, 25, 700_000, 1, 0, -1), (0, 26, 90_000, 0, 0, 0),
+    (0, 50, 90_000, 0, 0, 0), (0, 64, 1 << 22, 4, 0, -1), (0, 64, 1 << 22, 1, 0, -1),
+    (0, 1000, 200_000, 0, 0, 0), (0, 100, 5_000, 0, 0, -1), (0, 100, 5_243, 0, 0, 0), (0, 99, 5_000, 0, 0, 0),
+    (0, 320, 100_000, 0, 0, -1), (0, 320, 110_000, 0, 0, 0), (0, 320, 100_000, 1, 0, 0),
+    (0, 4096, 100_000, 4, 0, -1), (0, 4096, 1 << 17, 4, 0, 0), (0, 8192, 16_383, 0, -1, -1), (0, 8192, 16_384, 0, 0, -1),
+    (0, 8192, 1 << 17, 0, 0, 0), (0, 8192, 1_000, 3, 0, 0),
+    # MD5
+    (1, 1000, 65_535, 0, -1, -1), (1, 1000, 65_536, 0, 0, 0), (1, 24, 1 << 20, 0, 0, -1), (1, 25, 1 << 20, 0, 0, 0),
+    (1, 64, 1 << 20, 1, -1, -1), (1, 128, 1 << 20, 4, -1, -1), (1, 128, 1 << 20, 1, 0, 0), (1, 960, 1 << 20, 0, -1, -1),
+    (1, 1024, 131_071, 4, -1, -1), (1, 1024, 131_072, 4, 0, 0), (1, 8192, 1 << 18, 0, 0, -1),
+    (1, 72, 1 << 20, 0, 0, -1), (1, 200, 262_143, 0, -1, -1), (1, 200, 262_144, 0, 0, 0), (1, 200, 100_000, 2, 0, 0),
+    (1, 204, 100_000, 0, 0, 0), (1, 5000, 100_000, 0, 0, 0),
+])
+def test_kernel_of_a_chunk_size(fake, hk, C, n, offset, alone, leaf):
+    """Which kernel hashes chunks: where staging them was measured to be the slower way, alone or
+    in a checkpoint, they go by bytes."""
+    L = fake
+    L.fakehip_reset()
+    size = n * C
+    data, out = dev_alloc(L, size + 16), dev_alloc(L, 16 * n)
+    p = ctypes.c_void_p(data.value + offset)
+    assert L.mtc_hash_chunks(p, ctypes.c_uint64(size), C, hk, out, None) == OK
+    tag = lambda cb: f"ILi{hk}ELi{'n' if cb < 0 else ''}{abs(cb)}E"  # noqa: E731
+    assert [k for k in launches(L) if "k_hash_chunks" + tag(alone) in k], launches(L)
+    h = create(L, C, TREE, hk)
+    L.fakehip_reset()
+    assert checkpoint(L, h, p, size, baseline=True)[0] == OK
+    names = [k for k in launches(L) if "k_leaf" in k]
+    assert len(names) == 1 and tag(leaf) in names[0], names
+    assert violations(L) == []
+    L.mtc_destroy(h)
+    L.hipFree(data)
+    L.hipFree(out)
