@@ -2880,16 +2880,17 @@ static void rehash_to(mtc_dedup* h, uint64_t cap, hipStream_t st) {
 // The table is reset at a baseline (filled by the step's first launch).  Probing
 // always ends while one slot stays empty, so a checkpoint may start only if the
 // table holds all its possible inserts (the reference rehashes to size +
-// num_nodes, src/tree_approach.cpp:1622-1623).  Returns false when the worst case
-// (2n-1 new entries) fits and the table is at most 80% full: the step runs in one
-// piece.  Otherwise the step pauses after the leaf kernel, when an exact bound is
-// known (twice the chunks to insert: every new internal node has two new leaves
-// below it), and grow_exact rehashes only if that bound does not fit.
-// The next checkpoint runs in one piece in a table of `cap` slots: its worst case
-// (2n - 1 new entries) fits and the table is at most 80% full.
+// num_nodes, src/tree_approach.cpp:1622-1623).  The step runs in one piece when the
+// worst case (2n - 1 new entries) leaves a sixteenth of the slots empty and the table
+// is at most 80% full.  Otherwise the step pauses after the leaf kernel, when an exact
+// bound is known (twice the chunks to insert: every new internal node has two new
+// leaves below it), and grow_exact rehashes only if that bound does not fit.
+// A probe's length goes with the square of 1 / (empty share): with a sixteenth left
+// it is about 130 slots.  Up to the last slot, three whole rewrites of a buffer of 2^21
+// chunks filled its 2^24 slots but four, and the third took 31 seconds.
 static bool table_fits_step(const mtc_dedup* h, uint64_t cap) {
   const uint64_t nodes = 2ull * h->n - 1;
-  return h->table_size + nodes < cap && h->table_size <= cap / 10 * 8;
+  return h->table_size + nodes <= cap / 16 * 15 && h->table_size <= cap / 10 * 8;
 }
 
 // Slots of a baseline's digest table (without the overflow slot): a power of two

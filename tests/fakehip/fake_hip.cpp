@@ -73,6 +73,7 @@ struct State {
   std::vector<Node> captured;
   uint64_t bytes_alive = 0;
   uint64_t diff_size = 0;  // what a diff kernel reports (no kernel runs)
+  uint64_t claims = 0;     // and the table entries its step created
   std::set<hipEvent_t> timing;                       // events that take the time
   std::map<hipEvent_t, std::thread::id> recorded;    // by whom, until the time is read
   // Waits for the stream or an event last until this many threads wait (a time limit
@@ -387,6 +388,7 @@ void check_launch(const std::string& name, const uint8_t* arg0, uint32_t grid) {
       need(w, "changed", a.changed, 4);
       need_host(w, "out", a.out, kCtl);
       if (S().diff_size) a.out->diff_size = S().diff_size;
+      a.out->claims = S().claims;
       need(w, "dense", a.dense, 4ull * a.n);
       maybe(w, "reset_labels", a.reset_labels, a.n);
       S().label_resets.push_back(a.reset_labels ? 1 : 0);
@@ -499,6 +501,10 @@ void fakehip_set_diff_size(uint64_t size) {
   std::lock_guard<std::mutex> g(S().mu);
   S().diff_size = size;
 }
+void fakehip_set_claims(uint64_t claims) {
+  std::lock_guard<std::mutex> g(S().mu);
+  S().claims = claims;
+}
 void fakehip_hold(int threads) {
   std::lock_guard<std::mutex> g(S().mu);
   S().hold = threads;
@@ -515,7 +521,7 @@ void fakehip_reset() {
   S().violations.clear();
   S().launches.clear();
   S().grids.clear();
-  S().diff_size = 0;
+  S().diff_size = S().claims = 0;
   S().hold = S().holding = 0;
   S().leaf_all_labels.clear();
   S().label_resets.clear();

@@ -60,3 +60,12 @@ def test_series_by_bytes_and_staged(C, hk, n, offset):
         w[-1] ^= 1
         v.append(w)
     series(v, C, hk, offset)
+
+
+@pytest.mark.parametrize("load_factor", [0.125, 0.5, 0.7])
+@pytest.mark.parametrize("n", [1 << 12, 1 << 16])
+def test_whole_rewrites_grow_the_table(n, load_factor):
+    """Every chunk new in every version: each adds 2n - 1 entries to the table, which grows
+    before it is nearly full (a baseline's table too, at load factors of a half and more)."""
+    rng = np.random.default_rng(n)
+    series([rng.integers(0, 256, n * 16, dtype=np.uint8) for _ in range(6)], 16, load_factor=load_factor)

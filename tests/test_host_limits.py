@@ -192,3 +192,39 @@ def test_kernel_of_a_chunk_size(fake, hk, C, n, offset, alone, leaf):
     L.mtc_destroy(h)
     L.hipFree(data)
     L.hipFree(out)
+
+
+@pytest.mark.parametrize("entries,one_piece", [(0, True), (21 / 32, True), (22 / 32, True), (23 / 32, False), (3 / 4, False), (7 / 8, False)])
+def test_a_step_that_could_fill_the_table_waits_for_its_bound(fake, entries, one_piece):
+    """n = 2^12 chunks have 2^15 slots; a step may add 2^13 - 1 entries.  It runs in one piece
+    only while that leaves a sixteenth of the slots empty (probes grow with the square of
+    the empty share's inverse); else it pauses for the exact bound."""
+    L = fake
+    L.fakehip_reset()
+    n, C = 1 << 12, 128
+    h = create(L, C)
+    data = dev_alloc(L, n * C)
+    L.fakehip_set_claims(ctypes.c_uint64(int(entries * 8 * n)))
+    assert checkpoint(L, h, data, n * C, baseline=True)[0] == OK
+    L.fakehip_reset()
+    assert checkpoint(L, h, data, n * C)[0] == OK
+    assert any("k_leaf1_direct" in k for k in launches(L)) == one_piece
+    assert violations(L) == []
+    L.mtc_destroy(h)
+    L.hipFree(data)
+
+
+def test_a_table_of_half_the_usual_load_takes_a_baseline(fake):
+    """At load factor 0.5 a baseline's 2n - 1 entries could fill the 2n slots: it pauses, and
+    the table grows first."""
+    L = fake
+    L.fakehip_reset()
+    n, C = 1 << 12, 128
+    h = create(L, C)
+    assert L.mtc_set_tuning(h, 1, ctypes.c_float(0.5), 8) == OK
+    data = dev_alloc(L, n * C)
+    for k in range(3):
+        assert checkpoint(L, h, data, n * C, baseline=(k != 1))[0] == OK, L.mtc_last_error(h)
+    assert violations(L) == []
+    L.mtc_destroy(h)
+    L.hipFree(data)
