@@ -238,38 +238,39 @@ struct Regions {
   }
 };
 
-// Covers first-occurrence chunks (diffs flo .. hi - 1 of the pass that starts at lo; nblk
-// blocks) and the leaves of shifted entries (diffs slo .. hi - 1; the other blocks).  Each
-// leaf of a shifted entry's `node` takes the data slot of the matching leaf of `prev`
-// inside the source diff's region (src/tree_approach.cpp:887-925, 1058-1118); a wavefront
-// shares the leaves of its larger entries.
-// PLAIN: one diff (hi - 1), by plain stores over what the earlier ones left: the pass's
-// oldest, which holds nearly the whole buffer when it is the baseline, and any diff that
-// stores kCoverPlain chunks.  The others share a launch, in which the newest entry of a
-// chunk stands by atomic max: it needs no order, but runs at a third of a plain store's
-// rate.  A chain of three whole rewrites, 1 GiB in 48-byte chunks (22 million): 760 us
-// with the last two by atomics, 510 so; 256 MiB in 64-byte chunks (2^22) 212 and 177, in
-// 96-byte chunks no difference.  (Many shifted entries are no reason for a launch of
-// their own: their lookups take the time, 2-3% more of it with fewer in flight.)
-constexpr uint32_t kShiftOwn = 4;  // most leaves a lane covers by itself
+// Diffs are covered in one of two ways.  Most share a launch, in which the newest entry of
+// a chunk stands by atomic max: that needs no order.  Plain stores run at three times an
+// atomic's rate, but need a launch of their own, after the earlier diffs' and before the
+// later ones'.  So are covered the first-occurrence chunks of the pass's oldest diff, which
+// holds nearly the whole buffer when it is the baseline, and any diff's if it stores
+// kCoverPlain chunks; its shifted entries too if there are as many.  1 GiB in 48-byte chunks
+// (22 million), all but the oldest diff by atomics / so: a chain of three whole rewrites 750
+// / 510 us, of half constant buffers (a shifted entry a chunk) 1040 / 880; 256 MiB in
+// 64-byte chunks (2^22) rewritten 212 / 177, in 96-byte chunks no difference.  (Where one of
+// many shifted entries spans half the buffer, which one wavefront walks, less runs beside
+// it: 21.1 / 21.6 ms.)
 constexpr uint64_t kCoverPlain = 1u << 22;
-template <bool PLAIN>
-__global__ __launch_bounds__(kRThreads) void k_r_cover(Chain c, uint32_t lo, uint32_t flo, uint32_t slo, uint32_t hi,
-                                                       uint32_t nblk) {
+
+// First-occurrence chunks of diff p of the pass that starts at lo, by plain stores.
+__global__ __launch_bounds__(kRThreads) void k_r_cover_base(Chain c, uint32_t lo, uint32_t p) {
   if (*c.err) return;
-  auto put = [&](uint32_t chunk, uint64_t v) {
-    if (PLAIN) c.cover[chunk] = v;
-    else atomicMax((unsigned long long*)&c.cover[chunk], (unsigned long long)v);
-  };
-  if (blockIdx.x < nblk) {
-    if (PLAIN) {
-      const uint32_t p = hi - 1;
-      Regions d(c, p);
-      const uint64_t top = (uint64_t)(p - lo + 1) << kAddrBits, data = c.data()[p];
-      for (uint64_t j = (uint64_t)blockIdx.x * kRThreads + threadIdx.x; j < d.total; j += (uint64_t)nblk * kRThreads)
-        put(d.chunk(c, (uint32_t)j), top | (data + j * c.C));
-      return;
-    }
+  Regions d(c, p);
+  const uint64_t top = (uint64_t)(p - lo + 1) << kAddrBits, data = c.data()[p];
+  for (uint64_t j = (uint64_t)blockIdx.x * kRThreads + threadIdx.x; j < d.total; j += (uint64_t)gridDim.x * kRThreads)
+    c.cover[d.chunk(c, (uint32_t)j)] = top | (data + j * c.C);
+}
+
+// First-occurrence chunks of diffs flo .. hi - 1 (nblk blocks) and shifted entries of diffs
+// slo .. hi - 1 (the other blocks) of the pass that starts at lo.  Each leaf of a shifted
+// entry's `node` takes the data slot of the matching leaf of `prev` inside the source diff's
+// region (src/tree_approach.cpp:887-925, 1058-1118); a wavefront shares the leaves of its
+// larger entries.  PLAIN: one diff's shifted entries, by plain stores.
+constexpr uint32_t kShiftOwn = 4;  // most leaves a lane covers by itself
+template <bool PLAIN>
+__global__ __launch_bounds__(kRThreads) void k_r_cover_rest(Chain c, uint32_t lo, uint32_t flo, uint32_t slo, uint32_t hi,
+                                                            uint32_t nblk) {
+  if (*c.err) return;
+  if (!PLAIN && blockIdx.x < nblk) {
     const uint64_t* base = c.chunk_base();
     const uint64_t end = base[hi];
     for (uint64_t j = base[flo] + (uint64_t)blockIdx.x * kRThreads + threadIdx.x; j < end; j += (uint64_t)nblk * kRThreads) {
@@ -277,7 +278,8 @@ __global__ __launch_bounds__(kRThreads) void k_r_cover(Chain c, uint32_t lo, uin
       const uint64_t slot = j - base[p];
       Regions d(c, p);
       if (slot >= d.total) continue;
-      put(d.chunk(c, (uint32_t)slot), ((uint64_t)(p - lo + 1) << kAddrBits) | (c.data()[p] + slot * c.C));
+      atomicMax((unsigned long long*)&c.cover[d.chunk(c, (uint32_t)slot)],
+                (unsigned long long)(((uint64_t)(p - lo + 1) << kAddrBits) | (c.data()[p] + slot * c.C)));
     }
     return;
   }
@@ -341,7 +343,10 @@ __global__ __launch_bounds__(kRThreads) void k_r_cover(Chain c, uint32_t lo, uin
           c.fail(ERR_CORRUPT);
           break;
         }
-        put(run_at(nr, ns, nc, j), top | (data + slot * c.C));
+        uint64_t* at = &c.cover[run_at(nr, ns, nc, j)];
+        const uint64_t v = top | (data + slot * c.C);
+        if (PLAIN) *at = v;
+        else atomicMax((unsigned long long*)at, (unsigned long long)v);
       }
     };
     if (cnt && cnt <= kShiftOwn) cover_leaves(node, prev, root, rbase, spos, p, 0, 1, cnt);
@@ -581,23 +586,20 @@ static void launch_restart(const Chain& c, const uint64_t* meta_src, const uint6
     const uint32_t hi = (uint32_t)std::min<uint64_t>(L, lo + kCoverPos);
     if (lo) k_r_cover_age<<<rgrid(n), kRThreads, 0, st>>>(c.cover, n);
     auto blocks = [](uint64_t items) { return items ? rgrid(items) : 0u; };
-    uint32_t flo = (uint32_t)lo, slo = flo;  // the first diffs not covered yet
-    auto plain = [&](uint32_t p, uint32_t sblk) {
-      const uint32_t fblk = rgrid(cbase[p + 1] - cbase[p], 4096);
-      k_r_cover<true><<<fblk + sblk, kRThreads, 0, st>>>(c, (uint32_t)lo, p, p, p + 1, fblk);
-    };
-    auto together = [&](uint32_t end) {  // all before end
+    uint32_t flo = (uint32_t)lo, slo = flo;  // the first diffs whose chunks, and whose shifted entries, are not covered yet
+    auto together = [&](uint32_t end) {      // all before end
       const uint32_t fblk = blocks(cbase[end] - cbase[flo]), sblk = blocks(sbase[end] - sbase[slo]);
-      if (fblk + sblk) k_r_cover<false><<<fblk + sblk, kRThreads, 0, st>>>(c, (uint32_t)lo, flo, slo, end, fblk);
+      if (fblk + sblk) k_r_cover_rest<false><<<fblk + sblk, kRThreads, 0, st>>>(c, (uint32_t)lo, flo, slo, end, fblk);
       flo = slo = end;
     };
-    plain(flo++, 0);  // its shifted entries come with the next launch
-    for (uint32_t p = flo; p < hi; p++)
-      if (cbase[p + 1] - cbase[p] >= kCoverPlain) {
-        together(p);
-        plain(p, blocks(sbase[p + 1] - sbase[p]));
-        flo = slo = p + 1;
-      }
+    for (uint32_t p = flo; p < hi; p++) {
+      const uint64_t first = cbase[p + 1] - cbase[p], shifted = sbase[p + 1] - sbase[p];
+      const bool f = p == lo || first >= kCoverPlain, s = shifted >= kCoverPlain;
+      if (!f && !s) continue;
+      together(p);
+      if (f) k_r_cover_base<<<rgrid(first, 4096), kRThreads, 0, st>>>(c, (uint32_t)lo, flo++);
+      if (s) k_r_cover_rest<true><<<rgrid(shifted), kRThreads, 0, st>>>(c, (uint32_t)lo, p, slo++, p + 1, 0);
+    }
     together(hi);
     MTC_HIP(hipGetLastError());
   }

@@ -8,11 +8,10 @@ import mtcheck_amd as M  # noqa: E402
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("C,n", [(16, (1 << 22) - 1), (8, 1 << 22), (12, (1 << 22) + 777)])
+@pytest.mark.parametrize("C,n", [(16, (1 << 22) - 1), (8, 1 << 22), (12, (1 << 22) + 777), (8, 1 << 23)])
 def test_large_diffs_between_small_ones(C, n):
-    """Diffs below and from 2^22 chunks on, the oldest among them, with and without shifted
-    entries: every later one replaces what the earlier ones covered, in any order of the
-    two kinds."""
+    """Diffs below and from 2^22 chunks or shifted entries on, the oldest among them: every later
+    one replaces what the earlier ones covered, in any order of the two kinds."""
     g = torch.Generator(device="cuda")
     g.manual_seed(n + C)
     rand = lambda k: torch.randint(0, 256, (k, C), dtype=torch.uint8, device="cuda", generator=g)  # noqa: E731

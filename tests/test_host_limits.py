@@ -126,31 +126,34 @@ def test_device_copy_stays_in_the_destination(fake, room):
     L.mtc_destroy(h)
 
 
-@pytest.mark.parametrize("chunks,plain", [
-    ([5], [1]),
-    ([5, 5, 5], [1, 0]),                       # the oldest diff, then all others together
-    ([1 << 22, 5, 5], [1, 0]),
-    ([0, 1 << 22, 5, 1 << 22], [1, 1, 0, 1]),
-    ([5, 5, 1 << 22, (1 << 22) - 1], [1, 0, 1, 0]),
-    ([5, 1 << 22], [1, 1]),
+# What covers a chain's diffs, launch by launch: chunks (C) or shifted entries (S) of one diff by
+# plain stores, or all that is left of several by atomics (A).
+@pytest.mark.parametrize("chunks,shifted,order", [
+    ([5], [0], "C"),
+    ([5, 5, 5], [0, 0, 0], "CA"),                       # the oldest diff's chunks, then all others together
+    ([5, 5, 5], [3, 3, 3], "CA"),
+    ([5], [3], "CA"),
+    ([1 << 22, 5, 5], [0, 0, 3], "CA"),
+    ([0, 1 << 22, 5, 1 << 22], [0, 0, 0, 0], "CCAC"),   # in the chain's order
+    ([0, 1 << 22, 5, 1 << 22], [3, 3, 3, 3], "CACACA"),
+    ([5, 5, 1 << 22, (1 << 22) - 1], [0, 0, 0, 0], "CACA"),
+    ([5], [1 << 22], "CS"),
+    ([0], [(1 << 22) - 1], "CA"),
+    ([5, 5, 5], [1 << 22, 0, 5], "CSA"),
+    ([5, 5, 5], [5, 1 << 22, 5], "CASA"),
+    ([0, 1 << 22, 1], [0, 1 << 22, 1], "CCSA"),
+    ([0, 0, 0], [0, (1 << 22) - 1, 1 << 22], "CAS"),
 ])
-@pytest.mark.parametrize("shifted", [0, 3])
-def test_large_diffs_of_a_chain_are_covered_by_plain_stores(fake, chunks, plain, shifted):
-    """A restart covers a diff of 2^22 chunks in a launch of its own, which needs no atomics;
-    the others share launches, in the chain's order, the first of them with the shifted
-    entries of the oldest."""
+def test_large_diffs_of_a_chain_are_covered_by_plain_stores(fake, chunks, shifted, order):
     L = fake
     L.fakehip_reset()
     n = 1 << 23
-    bufs = [ctypes.create_string_buffer(bytes(Header(0, k, n, 1, 0, 0, shifted)), 32 + 8 * shifted + c) for k, c in enumerate(chunks)]
+    bufs = [ctypes.create_string_buffer(bytes(Header(0, k, n, 1, 0, 0, s)), 32 + 8 * s + f) for k, (f, s) in enumerate(zip(chunks, shifted))]
     ptrs = (ctypes.c_void_p * len(bufs))(*[ctypes.addressof(b) for b in bufs])
     sizes = (ctypes.c_uint64 * len(bufs))(*[len(b) for b in bufs])
     out = dev_alloc(L, n)
     assert L.mtc_restart(ptrs, sizes, len(bufs), len(bufs) - 1, 0, out, ctypes.c_uint64(n), 0, None) == OK
-    cover = [int("Lb1" in k) for k in launches(L) if "k_r_cover" in k]
-    if shifted and (len(chunks) == 1 or plain[1]):
-        plain = [1, 0] + plain[1:]
-    assert cover == plain
+    assert "".join("C" if "base" in k else "S" if "Lb1" in k else "A" for k in launches(L) if "k_r_cover" in k) == order
     assert violations(L) == []
     L.hipFree(out)
 
