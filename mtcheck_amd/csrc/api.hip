@@ -206,7 +206,9 @@ int mtc_copy_diff(mtc_dedup* h, void* host_dst, uint64_t capacity, void* stream)
     if (here) mtc::copy_device(h->diff_ptr(), static_cast<uint8_t*>(host_dst), h->last_diff_size, st);
     else MTC_HIP(hipMemcpyAsync(host_dst, h->diff_ptr(), h->last_diff_size, hipMemcpyDefault, st));
     MTC_HIP(hipEventRecord(ev.b, st));
-    MTC_HIP(hipEventSynchronize(ev.b));
+    // (The wait for the event itself is slower: ten checkpoints of 256 MiB and their copies
+    // 1240-1300 us, 1225 us so.)
+    MTC_HIP(hipStreamSynchronize(st));
     (void)hipEventElapsedTime(&h->last_ms[3], ev.a, ev.b);
   });
 }
