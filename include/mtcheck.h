@@ -136,7 +136,8 @@ int mtc_get_stats(const mtc_dedup* h, mtc_stats* out);
 /* TreeDeduplicator::restart(View, vector<HostMirror>&, logname, chkpt_id),
  * src/tree_approach.cpp:1786-1797 (-> restart_chkpt :712-1128), and the raw-pointer
  * overload :1809-1817.  diffs[i] is the diff of checkpoint i (entries below the
- * chain's ref_id may be NULL); diffs_on_device selects device or host pointers.
+ * chain's ref_id may be NULL); diffs_on_device selects device or host pointers (device
+ * diffs lie below 2^47, as every address of a process does unless it asks for higher ones).
  * The restored buffer (header.datalen bytes) is written to device pointer dev_out. */
 int mtc_restart(const void* const* diffs, const uint64_t* sizes, uint32_t count, uint32_t chkpt_id,
                 int diffs_on_device, void* dev_out, uint64_t out_len, int device, void* stream);

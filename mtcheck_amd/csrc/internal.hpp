@@ -195,7 +195,7 @@ struct mtc_dedup {
   mtc::DevBuf<uint32_t> pend;         // listed chunks left for k_fixmin
   mtc::DevBuf<uint8_t> pcnt;          // their number per group of 64 dense entries
   mtc::DevBuf<uint32_t> blk_cnt, blk_off;
-  uint64_t blk_zero = 0;             // leading entries of blk_cnt known to be zero (k_compact clears them)
+  uint64_t blk_zero = 0;             // leading entries of blk_cnt known to be zero (their last reader clears them)
   const void* blk_zero_p = nullptr;  // ... in this allocation
   mtc::DevBuf<uint8_t> tile_flags;    // per stage-0 tile: has-first, then busy
   mtc::DevBuf<mtc::Slot> table;
