@@ -69,3 +69,39 @@ def test_whole_rewrites_grow_the_table(n, load_factor):
     before it is nearly full (a baseline's table too, at load factors of a half and more)."""
     rng = np.random.default_rng(n)
     series([rng.integers(0, 256, n * 16, dtype=np.uint8) for _ in range(6)], 16, load_factor=load_factor)
+
+
+@pytest.mark.parametrize("C", [2, 5, 6, 15, 17, 33, 4097, 5001, 8191, 20_001])
+def test_chunks_gathered_and_restored_by_words(C):
+    """Diffs and outputs that start at any byte of a word: single chunks, runs, and words of up to
+    four chunks."""
+    n = max(9, 60_000 // C)
+    rng = np.random.default_rng(C)
+    v = [rng.integers(0, 256, n * C - C // 2, dtype=np.uint8)]
+    for _ in range(2):
+        w = v[-1].copy()
+        for first in rng.integers(0, n, n // 6):
+            w[first * C:(first + int(rng.integers(1, 4))) * C] ^= 255
+        v.append(w)
+    hk, size = (M.MD5 if C < 16 else M.MURMUR3), len(v[0])
+    for offset in (0, 3):
+        for approach in (M.TREE, M.BASIC):
+            buf = torch.zeros(size + 16, dtype=torch.uint8, device="cuda:0")
+            d = M.TreeDeduplicator(C, approach, hash_kind=hk)
+            orc = O.OracleDedup(C, hk) if approach == M.TREE else O.OracleBasic(C, hk)
+            chain = []
+            for k, host in enumerate(v):
+                print(f"C={C} offset {offset} approach {approach} checkpoint {k}", flush=True)
+                buf[offset:offset + size] = torch.from_numpy(host)
+                g, e = d.checkpoint(buf[offset:offset + size], make_baseline=(k == 0)), orc.checkpoint(host, make_baseline=(k == 0))
+                assert g == e, (k, first_mismatch(g, e))
+                chain.append(torch.frombuffer(bytearray(g), dtype=torch.uint8).to("cuda:0"))
+            d.close()
+            if approach == M.BASIC:
+                continue
+            for at in (0, 1, 2, 3, 4):
+                out = torch.full((size + 32,), 0xA5, dtype=torch.uint8, device="cuda:0")
+                M.restart_into(out[at:at + size], chain, 2)
+                got = out.cpu().numpy()
+                assert np.array_equal(got[at:at + size], v[2])
+                assert (got[:at] == 0xA5).all() and (got[at + size:] == 0xA5).all()
