@@ -449,14 +449,15 @@ void check(const void* fn, dim3 grid, dim3 block, void** args) {
     need(name, "src", src, size);
     need(name, "dst", dst, size);
     if (blocks * block.x * 16 < size) violation(name + ": threads do not cover the bytes");
-  } else if (name.find("k_r_copy") != std::string::npos) {  // (chain, datalen, ..., out): the same, 64 bytes a thread for one
+  } else if (name.find("k_r_copy") != std::string::npos) {  // (chain, datalen, ..., out): the same, 4, 16 or 64 bytes a thread
     const bool any = name.find("k_r_copy_any") != std::string::npos;
     uint64_t datalen;
     const uint8_t* out;
     std::memcpy(&datalen, args[1], 8);
     std::memcpy(&out, args[any ? 2 : 3], 8);
     need(name, "out", out, datalen);
-    if (blocks * block.x * (any ? 16 : 64) < (any ? datalen : datalen & ~15ull)) violation(name + ": threads do not cover the bytes");
+    const uint64_t per = !any ? 64 : name.find("anyILj4E") != std::string::npos ? 4 : 16;
+    if (blocks * block.x * per < (any ? datalen + ((uintptr_t)out & 3) : datalen & ~15ull)) violation(name + ": threads do not cover the bytes");
   }
 }
 

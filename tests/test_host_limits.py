@@ -231,3 +231,21 @@ def test_a_table_of_half_the_usual_load_takes_a_baseline(fake):
     assert violations(L) == []
     L.mtc_destroy(h)
     L.hipFree(data)
+
+
+@pytest.mark.parametrize("C,datalen", [(15, 1), (15, 29 * GIB + 3), (4, 8 * GIB - 4), (16, 30 * GIB + 3), (17, 16)])
+@pytest.mark.parametrize("offset", [0, 1, 2, 3])
+def test_restart_copies_whole_words(fake, C, datalen, offset):
+    """Chunks under 16 bytes by threads of a word each, larger ones by threads of four, from the word
+    on that the output starts in."""
+    L = fake
+    L.fakehip_reset()
+    diff = Header(0, 0, datalen, C, 0, 0, 0)
+    out = dev_alloc(L, datalen + offset)
+    ptrs = (ctypes.c_void_p * 1)(ctypes.addressof(diff))
+    sizes = (ctypes.c_uint64 * 1)(32)
+    assert L.mtc_restart(ptrs, sizes, 1, 0, 0, ctypes.c_void_p(out.value + offset), ctypes.c_uint64(datalen), 0, None) == OK
+    copies = [n for n in launches(L) if "k_r_copy" in n]
+    assert len(copies) == 1 and (C == 16 and offset == 0 or f"k_r_copy_anyILj{4 if C < 16 else 16}E" in copies[0]), copies
+    assert violations(L) == []
+    L.hipFree(out)
