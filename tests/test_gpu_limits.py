@@ -1,4 +1,4 @@
-"""Sizes beyond one row of a launch's blocks (2^31 threads)."""
+"""Sizes, table loads, chunk sizes and addresses at the limits of the kernels and their rules."""
 import numpy as np
 import pytest
 
